@@ -912,6 +912,8 @@ __global__ void __launch_bounds__(256)
 
 // Kernels of the FFT passes are instantiated on LOGN: n = 2^LOGN known at
 // compile time (LOGN > 0) or taken from the plan (LOGN = 0).
+template <typename T, int LOGN>
+constexpr int kFftMaxThreads = LOGN > 0 ? 1024 : kGenMaxThreads<T>;
 template <int LOGN>
 __device__ __forceinline__ int fft_len(const FftPlan &pl) {
   if constexpr (LOGN > 0)
@@ -1049,7 +1051,7 @@ __device__ __forceinline__ void d_fft_z_r2c(const int *__restrict__ act, const T
   }
 }
 template <typename T, int E, int LOGN>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_z_r2c(const int *__restrict__ act, const T *__restrict__ R, cx<T> *__restrict__ C, FftPlan pl,
                 const cx<T> *__restrict__ twg, int nx, int ny, int P,
                 FastDiv dXB, FastDiv dP) {
@@ -1072,7 +1074,7 @@ struct A_fft_z_r2c {
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
 template <typename T, int E, int LOGN>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_z_r2c_multi(const A_fft_z_r2c<T, E, LOGN> *__restrict__ a) {
   const A_fft_z_r2c<T, E, LOGN> &A = a[blockIdx.z];
   d_fft_z_r2c<T, E, LOGN, const FftPlan &>(A.act, A.R, A.C, A.pl, A.twg, A.nx, A.ny, A.P, A.dXB, A.dP);
@@ -1142,7 +1144,7 @@ __device__ __forceinline__ void d_fft_z_c2r(const int *__restrict__ act, const c
   }
 }
 template <typename T, int E, int LOGN>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_z_c2r(const int *__restrict__ act, const cx<T> *__restrict__ C, T *__restrict__ R, FftPlan pl,
                 const cx<T> *__restrict__ twg, int nx, int ny, int P,
                 FastDiv dP) {
@@ -1164,7 +1166,7 @@ struct A_fft_z_c2r {
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
 template <typename T, int E, int LOGN>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_z_c2r_multi(const A_fft_z_c2r<T, E, LOGN> *__restrict__ a) {
   const A_fft_z_c2r<T, E, LOGN> &A = a[blockIdx.z];
   d_fft_z_c2r<T, E, LOGN, const FftPlan &>(A.act, A.C, A.R, A.pl, A.twg, A.nx, A.ny, A.P, A.dP);
@@ -1217,7 +1219,7 @@ __device__ __forceinline__ void d_fft_y(const int *__restrict__ act, cx<T> *__re
   }
 }
 template <typename T, int E, int LOGN>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_y(const int *__restrict__ act, cx<T> *__restrict__ C, FftPlan pl, const cx<T> *__restrict__ twg,
             int nx, int nh, int B, int inverse, FastDiv dB) {
   d_fft_y<T, E, LOGN>(act, C, pl, twg, nx, nh, B, inverse, dB);
@@ -1238,7 +1240,7 @@ struct A_fft_y {
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
 template <typename T, int E, int LOGN>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_y_multi(const A_fft_y<T, E, LOGN> *__restrict__ a) {
   const A_fft_y<T, E, LOGN> &A = a[blockIdx.z];
   d_fft_y<T, E, LOGN, const FftPlan &>(A.act, A.C, A.pl, A.twg, A.nx, A.nh, A.B, A.inverse, A.dB);
@@ -1329,7 +1331,7 @@ __device__ __forceinline__ void d_fft_x_project(const int *__restrict__ act, cx<
   }
 }
 template <typename T, int E, int LOGN>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_x_project(const int *__restrict__ act, cx<T> *__restrict__ C, FftPlan pl,
                     const cx<T> *__restrict__ twg, ProjConst pc, int Q,
                     FastDiv dQ) {
@@ -1349,7 +1351,7 @@ struct A_fft_x_project {
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
 template <typename T, int E, int LOGN>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_x_project_multi(const A_fft_x_project<T, E, LOGN> *__restrict__ a) {
   const A_fft_x_project<T, E, LOGN> &A = a[blockIdx.z];
   d_fft_x_project<T, E, LOGN, const FftPlan &, const ProjConst &>(A.act, A.C, A.pl, A.twg, A.pc, A.Q, A.dQ);
@@ -1800,64 +1802,28 @@ __global__ void k_friction(const int *__restrict__ act, int n3, const double *__
 // ---------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------
-// Calls f(std::integral_constant<int, E>) for the register tile E of a plan.
-template <typename F>
-static bool with_E(int E, F f) {
-  switch (E) {
-    case 6: f(std::integral_constant<int, 6>{}); return true;
-    case 8: f(std::integral_constant<int, 8>{}); return true;
-    case 10: f(std::integral_constant<int, 10>{}); return true;
-    case 12: f(std::integral_constant<int, 12>{}); return true;
-    case 16: f(std::integral_constant<int, 16>{}); return true;
-    case 20: f(std::integral_constant<int, 20>{}); return true;
-    case 24: f(std::integral_constant<int, 24>{}); return true;
-    case 30: f(std::integral_constant<int, 30>{}); return true;
-  }
-  return false;
-}
-
 static int largest_divisor_le(int n, int t);
 
-// Register tile E and compile-time length of an FFT plan's kernels: n = 2^LOGN
-// for n in {128, 256, 512} with E = 8 or 16, provided the plan's radices are
-// those of the compile-time rule (p2_radix); otherwise LOGN = 0 (run-time
-// plan).
-static bool p2_plan_matches(const FftPlan &pl, int logn) {
-  int ls = 0, s = 0;
-  while (ls < logn) {
-    int rem = logn - ls;
-    int r = (rem >= 4 && pl.E >= 16) ? 16 : (rem >= 3 && pl.E >= 8) ? 8
-            : (rem >= 2)                ? 4
-                                        : 2;
-    if (s >= pl.nst || pl.rad[s] != r) return false;
-    ++s;
-    ls += (r == 16 ? 4 : r == 8 ? 3 : r == 4 ? 2 : 1);
-  }
-  return s == pl.nst;
-}
-
+// Register tile E and compile-time length of an FFT plan's kernels: n =
+// 2^LOGN with E = 8 or 16 for the compile-time plans, E = LOGN = 0 for the
+// run-time plan.
 template <typename F>
 static bool with_EL(const FftPlan &pl, F f) {
   using L0 = std::integral_constant<int, 0>;
-  int logn = 0;
-  if (pl.n == 128) logn = 7;
-  if (pl.n == 256) logn = 8;
-  if (pl.n == 512) logn = 9;
-  if (logn && (pl.E == 8 || pl.E == 16) && p2_plan_matches(pl, logn)) {
-    auto go = [&](auto e) {
-      switch (logn) {
-        case 7: f(e, std::integral_constant<int, 7>{}); break;
-        case 8: f(e, std::integral_constant<int, 8>{}); break;
-        default: f(e, std::integral_constant<int, 9>{}); break;
-      }
-    };
-    if (pl.E == 8)
-      go(std::integral_constant<int, 8>{});
-    else
-      go(std::integral_constant<int, 16>{});
+  if (pl.E == 0) {
+    f(L0{}, L0{});
     return true;
   }
-  return with_E(pl.E, [&](auto e) { f(e, L0{}); });
+  auto go = [&](auto e) {
+    switch (p2_log(pl.n)) {
+      case 7: f(e, std::integral_constant<int, 7>{}); return true;
+      case 8: f(e, std::integral_constant<int, 8>{}); return true;
+      case 9: f(e, std::integral_constant<int, 9>{}); return true;
+    }
+    return false;
+  };
+  return pl.E == 8 ? go(std::integral_constant<int, 8>{})
+                   : go(std::integral_constant<int, 16>{});
 }
 
 template <typename F>
@@ -1999,6 +1965,12 @@ int FcmImpl::init(const fs_fcm_params &pp, int maxnp, int prec) {
   tune.spread_zrun = 8;
   tune.spread_mfma = 1;
   tune.fft_xlines = (prec == FS_FP32) ? 4 : 2;
+  // run-time plans: about 3,072 (FP32) or 2,048 (FP64) complex values a
+  // workgroup, as the lines of 256 points have, so that short lines do not
+  // leave it with one wavefront
+  if (plx.E == 0)
+    tune.fft_xlines =
+        std::max(1, std::min(16, (prec == FS_FP32 ? 1024 : 680) / p.nx));
   FS_TRY(set_geometry());
   for (int i = 0; i < 8; ++i) FS_HIP(hipEventCreate(&ev[i]));
   for (int i = 0; i < 11; ++i) FS_HIP(hipEventCreate(&kev[i]));
@@ -2110,18 +2082,19 @@ int FcmImpl::set_geometry() {
   const size_t cs = 2 * tsz, lds_max = 160 * 1024;
   zP = 0;
   for (int xb = std::min(16, p.nx); xb >= 2; --xb)
-    if (xb % 2 == 0 && p.nx % xb == 0 && p.nz / plz.E * (xb / 2) <= 1024 &&
+    if (xb % 2 == 0 && p.nx % xb == 0 && fft_threads(plz, xb / 2) <= fft_max_threads(plz, tsz) &&
         cs * (p.nz + (size_t)(xb / 2) * fft_padded_len(p.nz)) <= lds_max) {
       zP = xb / 2;
       break;
     }
   yB = largest_divisor_le(p.nx, tune.fft_batch);
-  while (yB > 1 && p.ny / ply.E * yB > 1024) yB = largest_divisor_le(p.nx, yB - 1);
+  while (yB > 1 && fft_threads(ply, yB) > fft_max_threads(ply, tsz)) yB = largest_divisor_le(p.nx, yB - 1);
   xQ = largest_divisor_le(p.ny, tune.fft_xlines);
-  while (xQ > 1 && (p.nx / plx.E * 3 * xQ > 1024 ||
+  while (xQ > 1 && (fft_threads(plx, 3 * xQ) > fft_max_threads(plx, tsz) ||
                     cs * (p.nx + 3 * (size_t)xQ * fft_padded_len(p.nx)) > lds_max))
     xQ = largest_divisor_le(p.ny, xQ - 1);
-  FS_CHECK(zP >= 1 && p.ny / ply.E * yB <= 1024 && p.nx / plx.E * 3 * xQ <= 1024,
+  FS_CHECK(zP >= 1 && fft_threads(ply, yB) <= fft_max_threads(ply, tsz) &&
+               fft_threads(plx, 3 * xQ) <= fft_max_threads(plx, tsz),
            FS_ERR_ARG, "no FFT workgroup shape fits %dx%dx%d", p.nx, p.ny, p.nz);
   return FS_OK;
 }
@@ -2282,7 +2255,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   bool ok = with_EL(plz, [&](auto e, auto l) {
     constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
     hipLaunchKernelGGL((k_fft_z_r2c<T, EE, LL>), dim3(p.ny * (p.nx / (2 * zP)), 3),
-                       dim3(p.nz / EE * zP),
+                       dim3(fft_threads(plz, zP)),
                        csz * (p.nz + (size_t)zP * fft_padded_len(p.nz)), st, act,
                        R.as<T>(), C.as<cx<T>>(), plz, twz.as<cx<T>>(), p.nx,
                        p.ny, zP, make_div(2 * zP), make_div(zP));
@@ -2291,7 +2264,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   ok &= with_EL(ply, [&](auto e, auto l) {
     constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
     hipLaunchKernelGGL((k_fft_y<T, EE, LL>), dim3(nh * (p.nx / yB), 3),
-                       dim3(p.ny / EE * yB), csz * (p.ny + (size_t)yB * fft_rowpad_len(p.ny)), st, act,
+                       dim3(fft_threads(ply, yB)), csz * (p.ny + (size_t)yB * fft_rowpad_len(p.ny)), st, act,
                        C.as<cx<T>>(), ply, twy.as<cx<T>>(), p.nx, nh, yB, 0,
                        make_div(yB));
   });
@@ -2303,7 +2276,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   ok = with_EL(plx, [&](auto e, auto l) {
     constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
     hipLaunchKernelGGL((k_fft_x_project<T, EE, LL>), dim3(nh * (p.ny / xQ)),
-                       dim3(p.nx / EE * 3 * xQ),
+                       dim3(fft_threads(plx, 3 * xQ)),
                        csz * (p.nx + 3 * (size_t)xQ * fft_padded_len(p.nx)), st, act,
                        C.as<cx<T>>(),
                        plx, twx.as<cx<T>>(), pc, xQ, make_div(xQ));
@@ -2315,7 +2288,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   ok = with_EL(ply, [&](auto e, auto l) {
     constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
     hipLaunchKernelGGL((k_fft_y<T, EE, LL>), dim3(nh * (p.nx / yB), 3),
-                       dim3(p.ny / EE * yB), csz * (p.ny + (size_t)yB * fft_rowpad_len(p.ny)), st, act,
+                       dim3(fft_threads(ply, yB)), csz * (p.ny + (size_t)yB * fft_rowpad_len(p.ny)), st, act,
                        C.as<cx<T>>(), ply, twy.as<cx<T>>(), p.nx, nh, yB, 1,
                        make_div(yB));
   });
@@ -2323,7 +2296,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   ok &= with_EL(plz, [&](auto e, auto l) {
     constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
     hipLaunchKernelGGL((k_fft_z_c2r<T, EE, LL>), dim3(p.ny * (p.nx / (2 * zP)), 3),
-                       dim3(p.nz / EE * zP),
+                       dim3(fft_threads(plz, zP)),
                        csz * (p.nz + (size_t)zP * fft_padded_len(p.nz)), st, act,
                        C.as<cx<T>>(), R.as<T>(), plz, twz.as<cx<T>>(), p.nx,
                        p.ny, zP, make_div(zP));
@@ -2532,7 +2505,7 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
     if (!host)
       hipLaunchKernelGGL((k_fft_z_r2c_multi<T, EE, LL>),
                          dim3(p.ny * (p.nx / (2 * f0.zP)), 3, S),
-                         dim3(p.nz / EE * f0.zP),
+                         dim3(fft_threads(f0.plz, f0.zP)),
                          csz * (p.nz + (size_t)f0.zP * fft_padded_len(p.nz)), st,
                          (const A_fft_z_r2c<T, EE, LL> *)t);
   });
@@ -2546,7 +2519,7 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
       });
       if (!host)
         hipLaunchKernelGGL((k_fft_y_multi<T, EE, LL>),
-                           dim3(nh * (p.nx / f0.yB), 3, S), dim3(p.ny / EE * f0.yB),
+                           dim3(nh * (p.nx / f0.yB), 3, S), dim3(fft_threads(f0.ply, f0.yB)),
                            csz * (p.ny + (size_t)f0.yB * fft_rowpad_len(p.ny)), st,
                            (const A_fft_y<T, EE, LL> *)t);
     });
@@ -2562,7 +2535,7 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
         if (!host)
           hipLaunchKernelGGL((k_fft_x_project_multi<T, EE, LL>),
                              dim3(nh * (p.ny / f0.xQ), 1, S),
-                             dim3(p.nx / EE * 3 * f0.xQ),
+                             dim3(fft_threads(f0.plx, 3 * f0.xQ)),
                              csz * (p.nx + 3 * (size_t)f0.xQ * fft_padded_len(p.nx)),
                              st, (const A_fft_x_project<T, EE, LL> *)t);
       });
@@ -2578,7 +2551,7 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
     if (!host)
       hipLaunchKernelGGL((k_fft_z_c2r_multi<T, EE, LL>),
                          dim3(p.ny * (p.nx / (2 * f0.zP)), 3, S),
-                         dim3(p.nz / EE * f0.zP),
+                         dim3(fft_threads(f0.plz, f0.zP)),
                          csz * (p.nz + (size_t)f0.zP * fft_padded_len(p.nz)), st,
                          (const A_fft_z_c2r<T, EE, LL> *)t);
   });

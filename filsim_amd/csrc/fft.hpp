@@ -1,4 +1,4 @@
-// fft.hpp -- mixed-radix (2,3,4,5,8) Stockham FFT staged in LDS.
+// fft.hpp -- mixed-radix Stockham FFT staged in LDS.
 //
 // Replaces FFTW 2.1.5 rfftwnd (FCMfunctions.cpp:16-19, 360-406). A workgroup
 // transforms `ncols` sequences of length n held in LDS; element (m, col) lives
@@ -6,12 +6,13 @@
 // sequence: butterfly j reads inputs j + r*n/R, twiddles them by
 // W_{ns R}^{r (j mod ns)} and writes outputs (j/ns)*ns*R + (j mod ns) + r*ns
 // (decimation in time, autosorting: the result is in natural order).
-// Stages run in place: every thread holds E = lcm(radices) complex values
-// (E/R butterflies) in registers across the barrier that separates the
-// reads from the writes, so one LDS buffer holds the data and the workgroup
-// has exactly n*ncols/E threads. Transforms are unnormalised; sign -1
+// Stages run in place: every thread holds its butterflies' values in
+// registers across the barrier that separates the reads from the writes, so
+// one LDS buffer holds the data. Transforms are unnormalised; sign -1
 // forward, +1 inverse.
 #pragma once
+
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -37,56 +38,126 @@ inline FastDiv make_div(int d) {
 struct FftPlan {
   int n;
   int nst;
-  int E;  // elements per thread (multiple of every radix)
+  // elements per thread of the compile-time plans (lengths 2^LOGN below);
+  // 0: run-time plan
+  int E;
   int rad[kMaxStages];
   FastDiv dn;               // by n
   FastDiv dnb[kMaxStages];  // by n / rad[s]
   FastDiv dns[kMaxStages];  // by the stage's span ns (product of earlier radices)
 };
 
-inline int gcd_i(int a, int b) { return b == 0 ? a : gcd_i(b, a % b); }
-inline int lcm_i(int a, int b) { return a / gcd_i(a, b) * b; }
+// Elements per thread the run-time plan's workgroups are sized for: a stage
+// of radix R gives every thread ceil(kGenE / R) butterflies (some idle when R
+// does not divide kGenE). Threads used to hold whole multiples of
+// lcm(radices) elements instead: 24 for a 192-point line (radices 8, 8, 3),
+// 64 threads per 12 KB (FP32) of LDS, a third of the wavefronts this gives.
+// Measured at 192^3, FP64, per pass: z 199 -> 97 us, y 180 / 126 -> 92 / 70,
+// x + projection 225 -> 109, z inverse 153 -> 87 (FP32 92, 69 / 64, 107, 77 ->
+// 53, 49 / 44, 73, 57).
+constexpr int kGenE = 8;
+// Register-heavy FP64 radices: 512 threads leave 256 VGPRs each.
+template <typename T>
+constexpr int kGenMaxThreads = sizeof(T) == 8 ? 512 : 1024;
 
-// Radices for n = 2^a 3^b 5^c: largest power-of-two radices first (up to
-// max_radix: 16, 8, 4, 2), reduced until lcm(radices) <= 30 (the largest
-// register tile instantiated). Radix 16 halves the LDS passes of a
-// 256-point transform (two stages instead of three) but also halves the
-// threads of a workgroup; it pays only where the workgroup stays wide.
-inline bool make_plan(int n, FftPlan *p, int max_radix = 16) {
-  int a = 0, b = 0, c = 0, m = n;
-  while (m % 2 == 0) m /= 2, ++a;
-  while (m % 3 == 0) m /= 3, ++b;
-  while (m % 5 == 0) m /= 5, ++c;
-  if (m != 1 || n < 2) return false;
-  for (int maxr2 = max_radix; maxr2 >= 2; maxr2 /= 2) {
-    p->n = n;
-    p->nst = 0;
-    int r2 = a;
-    while (r2 > 0 && p->nst < kMaxStages) {
-      int r = (r2 >= 4 && maxr2 >= 16) ? 16
-              : (r2 >= 3 && maxr2 >= 8) ? 8
-              : (r2 >= 2 && maxr2 >= 4) ? 4
-                                        : 2;
-      p->rad[p->nst++] = r;
-      r2 -= (r == 16 ? 4 : r == 8 ? 3 : r == 4 ? 2 : 1);
-    }
-    for (int i = 0; i < b && p->nst < kMaxStages; ++i) p->rad[p->nst++] = 3;
-    for (int i = 0; i < c && p->nst < kMaxStages; ++i) p->rad[p->nst++] = 5;
-    int L = 1;
-    for (int s = 0; s < p->nst; ++s) L = lcm_i(L, p->rad[s]);
-    p->E = (L < 6) ? 8 : L;  // n >= 8 with only 2s always has an 8
-    if (p->E <= 30) {
-      p->dn = make_div(n);
-      int ns = 1;
-      for (int s = 0; s < p->nst; ++s) {
-        p->dnb[s] = make_div(n / p->rad[s]);
-        p->dns[s] = make_div(ns);
-        ns *= p->rad[s];
-      }
-      return true;
-    }
+// Threads of a workgroup that transforms ncols sequences of n.
+inline int fft_threads(const FftPlan &p, int ncols) {
+  if (p.E > 0) return p.n / p.E * ncols;
+  return ((p.n * ncols + kGenE - 1) / kGenE + 63) / 64 * 64;
+}
+inline int fft_max_threads(const FftPlan &p, int tsz) {
+  return p.E > 0 || tsz == 4 ? 1024 : 512;
+}
+
+// log2(n) for the lengths with compile-time plans, else 0.
+inline int p2_log(int n) {
+  return n == 128 ? 7 : n == 256 ? 8 : n == 512 ? 9 : 0;
+}
+
+// Radices of a run-time plan, largest first: as few stages as possible (each
+// is a round trip through LDS and a barrier), and among those the smallest
+// largest radix (the registers of a butterfly).
+inline bool gen_radices(int n, int maxr, int left, int *rad, int *nst,
+                        int depth = 0) {
+  static const int set[] = {16, 12, 10, 9, 8, 6, 5, 4, 3, 2};
+  if (n == 1) {
+    *nst = depth;
+    return true;
   }
+  if (left == 0) return false;
+  for (int r : set)
+    if (r <= maxr && n % r == 0) {
+      rad[depth] = r;
+      if (gen_radices(n / r, r, left - 1, rad, nst, depth + 1)) return true;
+    }
   return false;
+}
+
+// Plan of n = 2^a 3^b 5^c. Lengths 128, 256 and 512 take the compile-time
+// plan: radix max_radix (16 or 8), then what is left. Radix 16 halves the LDS
+// passes of a 256-point transform (two stages instead of three) but also
+// halves the threads of a workgroup; it pays only where the workgroup stays
+// wide.
+inline bool make_plan(int n, FftPlan *p, int max_radix = 16) {
+  int a = 0, m = n;
+  while (m % 2 == 0) m /= 2, ++a;
+  while (m % 3 == 0) m /= 3;
+  while (m % 5 == 0) m /= 5;
+  if (m != 1 || n < 2) return false;
+  p->n = n;
+  p->nst = 0;
+  p->E = 0;
+  if (p2_log(n)) {
+    p->E = max_radix >= 16 ? 16 : 8;
+    while (a > 0) {
+      const int l = a >= 4 && p->E == 16 ? 4 : a >= 3 ? 3 : a >= 2 ? 2 : 1;
+      p->rad[p->nst++] = 1 << l;
+      a -= l;
+    }
+  } else {
+    bool ok = false;
+    for (int st = 1; st <= kMaxStages && !ok; ++st)
+      for (int maxr = 2; maxr <= 16 && !ok; ++maxr)
+        ok = gen_radices(n, maxr, st, p->rad, &p->nst);
+    if (!ok) return false;
+  }
+  p->dn = make_div(n);
+  int ns = 1;
+  for (int s = 0; s < p->nst; ++s) {
+    p->dnb[s] = make_div(n / p->rad[s]);
+    p->dns[s] = make_div(ns);
+    ns *= p->rad[s];
+  }
+  return true;
+}
+
+// cos and sin of 2 pi k / n at compile time (Taylor series on the first
+// octant, reduced exactly in integers).
+constexpr double ct_series(double x, bool cosine) {
+  double term = cosine ? 1.0 : x, sum = term;
+  for (int i = cosine ? 1 : 2; i < 24; i += 2) {
+    term = -term * x * x / (double)(i * (i + 1));
+    sum += term;
+  }
+  return sum;
+}
+constexpr double ct_cos(int k, int n) {
+  k = ((k % n) + n) % n;
+  if (2 * k > n) k = n - k;                        // cos is even
+  if (4 * k > n) return -ct_cos(n - 2 * k, 2 * n); // cos(pi - x) = -cos x
+  constexpr double pi = 3.14159265358979323846264338327950288;
+  if (8 * k > n) return ct_series(pi / 2 - 2 * pi * k / n, false);
+  return ct_series(2 * pi * k / n, true);
+}
+constexpr double ct_sin(int k, int n) { return ct_cos(4 * k - n, 4 * n); }
+
+// f(integral_constant I) for I = A .. B - 1
+template <int A, int B, typename F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (A < B) {
+    f(std::integral_constant<int, A>{});
+    static_for<A + 1, B>(f);
+  }
 }
 
 template <typename T>
@@ -212,13 +283,50 @@ __device__ __forceinline__ void dft5(cx<T> *v, bool inv) {
 }
 
 template <typename T, int R>
+__device__ __forceinline__ void dftR(cx<T> *v, bool inv);
+
+// R1 R2 points: R1-point transforms over n1 of v[R2 n1 + n2], twiddles
+// W^(n2 k1), R2-point transforms over n2; natural order in and out.
+template <typename T, int R1, int R2>
+__device__ __forceinline__ void dft_comp(cx<T> *v, bool inv) {
+  constexpr int R = R1 * R2;
+  cx<T> y[R2][R1];
+#pragma unroll
+  for (int n2 = 0; n2 < R2; ++n2) {
+#pragma unroll
+    for (int n1 = 0; n1 < R1; ++n1) y[n2][n1] = v[R2 * n1 + n2];
+    dftR<T, R1>(y[n2], inv);
+  }
+  static_for<1, R2>([&](auto n2) {
+    static_for<1, R1>([&](auto k1) {
+      constexpr int m = n2() * k1();
+      constexpr double c = ct_cos(m, R), s = ct_sin(m, R);
+      y[n2()][k1()] = cmul(y[n2()][k1()], cx<T>{(T)c, inv ? (T)s : (T)-s});
+    });
+  });
+#pragma unroll
+  for (int k1 = 0; k1 < R1; ++k1) {
+    cx<T> u[R2];
+#pragma unroll
+    for (int n2 = 0; n2 < R2; ++n2) u[n2] = y[n2][k1];
+    dftR<T, R2>(u, inv);
+#pragma unroll
+    for (int k2 = 0; k2 < R2; ++k2) v[k1 + R1 * k2] = u[k2];
+  }
+}
+
+template <typename T, int R>
 __device__ __forceinline__ void dftR(cx<T> *v, bool inv) {
-  if (R == 2) dft2(v);
-  if (R == 3) dft3(v, inv);
-  if (R == 4) dft4(v, inv);
-  if (R == 5) dft5(v, inv);
-  if (R == 8) dft8(v, inv);
-  if (R == 16) dft16(v, inv);
+  if constexpr (R == 2) dft2(v);
+  if constexpr (R == 3) dft3(v, inv);
+  if constexpr (R == 4) dft4(v, inv);
+  if constexpr (R == 5) dft5(v, inv);
+  if constexpr (R == 6) dft_comp<T, 3, 2>(v, inv);
+  if constexpr (R == 8) dft8(v, inv);
+  if constexpr (R == 9) dft_comp<T, 3, 3>(v, inv);
+  if constexpr (R == 10) dft_comp<T, 5, 2>(v, inv);
+  if constexpr (R == 12) dft_comp<T, 4, 3>(v, inv);
+  if constexpr (R == 16) dft16(v, inv);
 }
 
 // Padded LDS layout for contiguous sequences: element i of a sequence sits at
@@ -268,86 +376,89 @@ __device__ __forceinline__ int lds_idx(int i, int col, int sm, int sc) {
   return PAD ? col * sc + fft_pad(i) : fft_rowpad(i) * sm + col * sc;
 }
 
-// One in-place stage; blockDim.x * (E/R) == (n/R) * ncols exactly.
-template <typename T, int R, int E, bool PAD, bool INV>
+// One in-place stage of the run-time plan; blockDim.x * kGenE >= n * ncols.
+template <typename T, int R, bool PAD, bool INV>
 __device__ __forceinline__ void fft_stage(cx<T> *buf, int n, int ns, int ncols,
                                           int sm, int sc, const cx<T> *tw,
                                           FastDiv dnb, FastDiv dns,
                                           FastDiv dcols) {
-  constexpr bool inv = INV;
-  constexpr int NB = E / R;
-  const int nb = n / R;
-  const int twstep = n / (ns * R);
-  cx<T> v[E];
-  int jj[NB], cc[NB];
+  constexpr int NB = (kGenE + R - 1) / R;
+  const int nb = dnb.d;
+  const int nbf = nb * ncols;
+  const int twstep = dns.q(nb);  // n / (ns R)
+  cx<T> v[NB * R];
+  int dst[NB];
 #pragma unroll
   for (int m = 0; m < NB; ++m) {
     const int t = threadIdx.x + m * blockDim.x;
-    int j, col;
-    if (sm == 1) {  // sequences contiguous: butterflies fastest
-      col = dnb.q(t);
-      j = t - col * nb;
-    } else {  // sequences interleaved: columns fastest
-      j = dcols.q(t);
-      col = t - j * ncols;
-    }
-    jj[m] = j;
-    cc[m] = col;
-    const int jq = dns.q(j);
-    const int k = j - jq * ns;
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      v[m * R + r] = buf[lds_idx<PAD>(j + r * nb, col, sm, sc)];
-    if (ns > 1) {
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        cx<T> w = tw[r * k * twstep];
-        if (inv) w.y = -w.y;
-        v[m * R + r] = cmul(v[m * R + r], w);
+    dst[m] = -1;
+    if (t < nbf) {
+      int j, col;
+      if constexpr (PAD) {  // sequences contiguous: butterflies fastest
+        col = dnb.q(t);
+        j = t - col * nb;
+      } else {  // sequences interleaved: columns fastest
+        j = dcols.q(t);
+        col = t - j * ncols;
       }
+      const int jq = dns.q(j);
+      const int k = j - jq * ns;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        v[m * R + r] = buf[lds_idx<PAD>(j + r * nb, col, sm, sc)];
+      if (ns > 1) {
+        const int kt = k * twstep;
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+          cx<T> w = tw[r * kt];
+          if constexpr (INV) w.y = -w.y;
+          v[m * R + r] = cmul(v[m * R + r], w);
+        }
+      }
+      dftR<T, R>(&v[m * R], INV);
+      // 16 bits each: element of output 0 and column
+      dst[m] = (jq * ns * R + k) | (col << 16);
     }
-    dftR<T, R>(&v[m * R], inv);
   }
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < NB; ++m) {
-    const int j = jj[m], col = cc[m];
-    const int jq = dns.q(j);
-    const int d = jq * ns * R + (j - jq * ns);
+    if (dst[m] >= 0) {
+      const int d = dst[m] & 0xffff, col = dst[m] >> 16;
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-      buf[lds_idx<PAD>(d + r * ns, col, sm, sc)] = v[m * R + r];
+      for (int r = 0; r < R; ++r)
+        buf[lds_idx<PAD>(d + r * ns, col, sm, sc)] = v[m * R + r];
+    }
   }
   __syncthreads();
 }
 
-// All stages of the plan, in place in buf. Needs blockDim.x = n*ncols/E.
+// All stages of the run-time plan, in place in buf (fft_threads threads).
 // PAD: contiguous padded sequences (sm = 1, sc = fft_padded_len(n)).
-template <typename T, int E, bool PAD, bool INV>
+template <typename T, bool PAD, bool INV>
 __device__ void lds_fft_plan(cx<T> *buf, const FftPlan &pl, int ncols, int sm,
                              int sc, const cx<T> *tw, FastDiv dcols) {
   int ns = 1;
   for (int s = 0; s < pl.nst; ++s) {
     const int R = pl.rad[s];
     const FastDiv a = pl.dnb[s], b = pl.dns[s];
-    if constexpr (E % 16 == 0)
-      if (R == 16)
-        fft_stage<T, 16, E, PAD, INV>(buf, pl.n, ns, ncols, sm, sc, tw, a, b, dcols);
-    if constexpr (E % 8 == 0)
-      if (R == 8)
-        fft_stage<T, 8, E, PAD, INV>(buf, pl.n, ns, ncols, sm, sc, tw, a, b, dcols);
-    if constexpr (E % 4 == 0)
-      if (R == 4)
-        fft_stage<T, 4, E, PAD, INV>(buf, pl.n, ns, ncols, sm, sc, tw, a, b, dcols);
-    if constexpr (E % 2 == 0)
-      if (R == 2)
-        fft_stage<T, 2, E, PAD, INV>(buf, pl.n, ns, ncols, sm, sc, tw, a, b, dcols);
-    if constexpr (E % 3 == 0)
-      if (R == 3)
-        fft_stage<T, 3, E, PAD, INV>(buf, pl.n, ns, ncols, sm, sc, tw, a, b, dcols);
-    if constexpr (E % 5 == 0)
-      if (R == 5)
-        fft_stage<T, 5, E, PAD, INV>(buf, pl.n, ns, ncols, sm, sc, tw, a, b, dcols);
+    switch (R) {
+#define FS_STAGE(RR)                                                         \
+  case RR:                                                                   \
+    fft_stage<T, RR, PAD, INV>(buf, pl.n, ns, ncols, sm, sc, tw, a, b, dcols); \
+    break;
+      FS_STAGE(16)
+      FS_STAGE(12)
+      FS_STAGE(10)
+      FS_STAGE(9)
+      FS_STAGE(8)
+      FS_STAGE(6)
+      FS_STAGE(5)
+      FS_STAGE(4)
+      FS_STAGE(3)
+      FS_STAGE(2)
+#undef FS_STAGE
+    }
     ns *= R;
   }
 }
@@ -470,7 +581,7 @@ __device__ __forceinline__ void lds_fft(cx<T> *buf, const FftPlan &pl,
   if constexpr (LOGN > 0)
     p2_stages<T, E, PAD, INV, LOGN, 0>(buf, ncols, sm, tw, dcols);
   else
-    lds_fft_plan<T, E, PAD, INV>(buf, pl, ncols, sm, sc, tw, dcols);
+    lds_fft_plan<T, PAD, INV>(buf, pl, ncols, sm, sc, tw, dcols);
 }
 
 }  // namespace fs
