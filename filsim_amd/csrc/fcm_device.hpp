@@ -1,0 +1,114 @@
+// fcm_device.hpp -- device pieces the FCM kernels share: Gaussian constants,
+// segment records and tile lists, matrix-core steps.
+#pragma once
+
+#include "common.hpp"
+#include "fcm_impl.hpp"
+
+namespace fs {
+
+constexpr double kPi = 3.14159265358979323846264338327950288;
+constexpr int kCoef = 8;  // spread coefficients per segment (6 used)
+constexpr int kMaxBinsPerTile = 64;
+
+struct GaussConst {
+  double dx, anorm, anorm2, anormdip, anormdip2, sigmadipsq;
+  int ngd, ngdh, nx, ny, nz;
+  // FP32 weights: g = anorm 2^(-xx^2 e2), gD = anormdip 2^(-xx^2 ed2),
+  // e2 = log2(e) / anorm2, ed2 = log2(e) / anormdip2
+  double e2, ed2;
+  double nrsd;  // -1 / sigmadipsq
+};
+
+// What a tile needs of one segment: per axis the FP64 offset xx0 = (grid
+// coordinate of stencil point 0) * dx - y (point i lies at xx0 + i dx), its
+// id, stencil origin (10 bits per axis, x lowest) and spread coefficients
+// (force, half torque: GA_setup).
+template <typename T>
+struct alignas(16) SegRec {
+  double xx0[3];
+  int id, org;
+  T cf[6];
+};
+constexpr int kTileCap = 32;  // records in a tile's slab; the rest: pool
+inline size_t rec_bytes(int tsz) {
+  return tsz == 8 ? sizeof(SegRec<double>) : sizeof(SegRec<float>);
+}
+
+// Whether a stencil of ngd points starting at o overlaps the te points
+// starting at p0 on a periodic axis of n points (o, p0 in [0, n)).
+__device__ __forceinline__ bool stencil_meets(int o, int p0, int te, int ngd,
+                                             int n) {
+  int d = o - p0;
+  if (d < 0) d += n;
+  return d < te || d > n - ngd;
+}
+
+// Stages records [r0, r0 + n) of tile `tile` into s_rec: r0 = 0 copies the
+// whole slab (issued before the count is known; entries past the count are
+// never used), r0 >= kTileCap the tile's pool block. 256 threads.
+template <typename T>
+__device__ __forceinline__ void stage_tile_records(
+    const SegRec<T> *__restrict__ slab, const SegRec<T> *__restrict__ pool,
+    int tile, int ovf, int r0, int n, SegRec<T> *s_rec) {
+  constexpr int W = sizeof(SegRec<T>) / 16;
+  static_assert(kTileCap * W <= 256, "one 16-byte word per thread");
+  const int4 *src =
+      r0 == 0 ? reinterpret_cast<const int4 *>(slab + (size_t)tile * kTileCap)
+              : reinterpret_cast<const int4 *>(pool + ovf + r0 - kTileCap);
+  const int nw = (r0 == 0 ? kTileCap : n) * W;
+  if ((int)threadIdx.x < nw)
+    reinterpret_cast<int4 *>(s_rec)[threadIdx.x] = src[threadIdx.x];
+}
+
+// A tile's record count and this thread's 16-byte word of its slab, loaded
+// ahead of use: the persistent tile kernels fetch the next tile's while
+// they work on the current one.
+template <typename T>
+struct TilePrefetch {
+  static constexpr int W = sizeof(SegRec<T>) / 16;
+  int4 w;
+  int cnt;
+  __device__ __forceinline__ void load(const SegRec<T> *__restrict__ slab,
+                                       const int *__restrict__ tcnt, int tile) {
+    if ((int)threadIdx.x < kTileCap * W)
+      w = reinterpret_cast<const int4 *>(slab + (size_t)tile * kTileCap)[threadIdx.x];
+    cnt = tcnt[tile];
+  }
+  __device__ __forceinline__ void store(SegRec<T> *s_rec) const {
+    if ((int)threadIdx.x < kTileCap * W)
+      reinterpret_cast<int4 *>(s_rec)[threadIdx.x] = w;
+  }
+};
+
+// One 16x16x4 matrix-core step D += A B in the real type, and the row of
+// D held in accumulator element r of lane l (column l % 16): 4 (l / 16) + r
+// for FP32, 4 r + l / 16 for FP64 (the instructions' output layouts).
+template <typename T>
+struct Mfma;
+template <>
+struct Mfma<float> {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 step(float a, float b, v4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) {
+    return 4 * (lane >> 4) + r;
+  }
+};
+template <>
+struct Mfma<double> {
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 step(double a, double b, v4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) {
+    return 4 * r + (lane >> 4);
+  }
+};
+
+// Tiles of te points that a stencil of ngd points can meet along an axis.
+__host__ __device__ constexpr int stencil_tiles(int ngd, int te) {
+  return (ngd + te - 2) / te + 1;
+}
+}  // namespace fs

@@ -1,4 +1,4 @@
-// fft.hpp -- mixed-radix Stockham FFT staged in LDS.
+// fft.hpp -- mixed-radix Stockham FFT exchanged through LDS.
 //
 // Replaces FFTW 2.1.5 rfftwnd (FCMfunctions.cpp:16-19, 360-406). A workgroup
 // transforms `ncols` sequences of length n held in LDS; element (m, col) lives
@@ -71,7 +71,7 @@ inline int fft_max_threads(const FftPlan &p, int tsz) {
 
 // log2(n) for the lengths with compile-time plans, else 0.
 inline int p2_log(int n) {
-  return n == 128 ? 7 : n == 256 ? 8 : n == 512 ? 9 : 0;
+  return n == 64 ? 6 : n == 128 ? 7 : n == 256 ? 8 : n == 512 ? 9 : 0;
 }
 
 // Radices of a run-time plan, largest first: as few stages as possible (each
@@ -93,12 +93,11 @@ inline bool gen_radices(int n, int maxr, int left, int *rad, int *nst,
   return false;
 }
 
-// Plan of n = 2^a 3^b 5^c. Lengths 128, 256 and 512 take the compile-time
-// plan: radix max_radix (16 or 8), then what is left. Radix 16 halves the LDS
-// passes of a 256-point transform (two stages instead of three) but also
-// halves the threads of a workgroup; it pays only where the workgroup stays
-// wide.
-inline bool make_plan(int n, FftPlan *p, int max_radix = 16) {
+// Plan of n = 2^a 3^b 5^c. Lengths 64 to 512 that are powers of two
+// take the compile-time plan: radix 8, then what is left. (Radix 16, two stages instead of three at
+// 256 points, is within 3% of it in FP32 and 20% slower in FP64: a thread's 16
+// values leave half the wavefronts.)
+inline bool make_plan(int n, FftPlan *p) {
   int a = 0, m = n;
   while (m % 2 == 0) m /= 2, ++a;
   while (m % 3 == 0) m /= 3;
@@ -108,15 +107,16 @@ inline bool make_plan(int n, FftPlan *p, int max_radix = 16) {
   p->nst = 0;
   p->E = 0;
   if (p2_log(n)) {
-    p->E = max_radix >= 16 ? 16 : 8;
+    p->E = 8;
     while (a > 0) {
-      const int l = a >= 4 && p->E == 16 ? 4 : a >= 3 ? 3 : a >= 2 ? 2 : 1;
+      const int l = a >= 3 ? 3 : a >= 2 ? 2 : 1;
       p->rad[p->nst++] = 1 << l;
       a -= l;
     }
   } else {
     bool ok = false;
-    for (int st = 1; st <= kMaxStages && !ok; ++st)
+    // at least two stages: the first reads global memory, the last writes it
+    for (int st = 2; st <= kMaxStages && !ok; ++st)
       for (int maxr = 2; maxr <= 16 && !ok; ++maxr)
         ok = gen_radices(n, maxr, st, p->rad, &p->nst);
     if (!ok) return false;
@@ -358,6 +358,16 @@ __host__ __device__ __forceinline__ constexpr int fft_padded_len(int n) {
   return l;
 }
 
+// Threads and LDS (complex values) of an x pass workgroup of Q lines: the
+// compile-time plans' threads hold the three components, the run-time plan's
+// LDS does.
+inline int x_threads(const FftPlan &pl, int Q) {
+  return pl.E > 0 ? pl.n / pl.E * Q : fft_threads(pl, 3 * Q);
+}
+inline size_t x_lds_values(const FftPlan &pl, int Q) {
+  return pl.n + (size_t)(pl.E > 0 ? 1 : 3) * Q * fft_padded_len(pl.n);
+}
+
 // Element-major layout (element m of every sequence in one row of sm): row
 // m sits at row m + m / 8, so rows 8 apart (the lanes of a radix-8 stage's
 // writes) fall on different banks.
@@ -376,36 +386,57 @@ __device__ __forceinline__ int lds_idx(int i, int col, int sm, int sc) {
   return PAD ? col * sc + fft_pad(i) : fft_rowpad(i) * sm + col * sc;
 }
 
-// One in-place stage of the run-time plan; blockDim.x * kGenE >= n * ncols.
-template <typename T, int R, bool PAD, bool INV>
-__device__ __forceinline__ void fft_stage(cx<T> *buf, int n, int ns, int ncols,
-                                          int sm, int sc, const cx<T> *tw,
-                                          FastDiv dnb, FastDiv dns,
-                                          FastDiv dcols) {
+// Where a stage reads or writes: LdsIO is the LDS buffer (element i of
+// sequence col), any other functor global memory, value ld(i, col) and
+// st(i, col, value). A pass's first stage reads global memory into its
+// registers and its last stage writes it, instead of staging the lines in LDS
+// before and after: one LDS round trip and barrier pair less at either end
+// (192^3 FP64 y pass 92 / 70 -> 64 / 59 us; 256^3 FP64 189 / 167 -> 172 / 155).
+template <typename T, bool PAD>
+struct LdsIO {
+  cx<T> *buf;
+  int sm, sc;
+  __device__ __forceinline__ cx<T> operator()(int i, int col) const {
+    return buf[lds_idx<PAD>(i, col, sm, sc)];
+  }
+  __device__ __forceinline__ void operator()(int i, int col, cx<T> v) const {
+    buf[lds_idx<PAD>(i, col, sm, sc)] = v;
+  }
+};
+
+// One stage of the run-time plan; blockDim.x * kGenE >= n * ncols. SYNC: a
+// barrier between the reads and the writes (both of the same LDS buffer).
+template <typename T, int R, bool PAD, bool INV, bool SYNC, typename LD,
+          typename ST>
+__device__ __forceinline__ void fft_stage(int ns, int ncols, const cx<T> *tw,
+                                          FastDiv dnb, FastDiv dns, FastDiv dcols,
+                                          LD ld, ST st) {
   constexpr int NB = (kGenE + R - 1) / R;
   const int nb = dnb.d;
   const int nbf = nb * ncols;
   const int twstep = dns.q(nb);  // n / (ns R)
   cx<T> v[NB * R];
-  int dst[NB];
+  int jj[NB], cc[NB];
 #pragma unroll
   for (int m = 0; m < NB; ++m) {
     const int t = threadIdx.x + m * blockDim.x;
-    dst[m] = -1;
+    if constexpr (PAD) {  // butterflies fastest
+      cc[m] = dnb.q(t);
+      jj[m] = t - cc[m] * nb;
+    } else {  // columns fastest
+      jj[m] = dcols.q(t);
+      cc[m] = t - jj[m] * ncols;
+    }
     if (t < nbf) {
-      int j, col;
-      if constexpr (PAD) {  // sequences contiguous: butterflies fastest
-        col = dnb.q(t);
-        j = t - col * nb;
-      } else {  // sequences interleaved: columns fastest
-        j = dcols.q(t);
-        col = t - j * ncols;
-      }
-      const int jq = dns.q(j);
-      const int k = j - jq * ns;
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        v[m * R + r] = buf[lds_idx<PAD>(j + r * nb, col, sm, sc)];
+      for (int r = 0; r < R; ++r) v[m * R + r] = ld(jj[m] + r * nb, cc[m]);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < NB; ++m) {
+    const int t = threadIdx.x + m * blockDim.x;
+    if (t < nbf) {
+      const int j = jj[m], jq = dns.q(j), k = j - jq * ns;
       if (ns > 1) {
         const int kt = k * twstep;
 #pragma unroll
@@ -416,48 +447,63 @@ __device__ __forceinline__ void fft_stage(cx<T> *buf, int n, int ns, int ncols,
         }
       }
       dftR<T, R>(&v[m * R], INV);
-      // 16 bits each: element of output 0 and column
-      dst[m] = (jq * ns * R + k) | (col << 16);
+      jj[m] = jq * ns * R + k;  // element of output 0
     }
   }
-  __syncthreads();
+  if constexpr (SYNC) __syncthreads();
 #pragma unroll
   for (int m = 0; m < NB; ++m) {
-    if (dst[m] >= 0) {
-      const int d = dst[m] & 0xffff, col = dst[m] >> 16;
+    const int t = threadIdx.x + m * blockDim.x;
+    if (t < nbf) {
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        buf[lds_idx<PAD>(d + r * ns, col, sm, sc)] = v[m * R + r];
+      for (int r = 0; r < R; ++r) st(jj[m] + r * ns, cc[m], v[m * R + r]);
     }
   }
-  __syncthreads();
 }
 
-// All stages of the run-time plan, in place in buf (fft_threads threads).
-// PAD: contiguous padded sequences (sm = 1, sc = fft_padded_len(n)).
-template <typename T, bool PAD, bool INV>
-__device__ void lds_fft_plan(cx<T> *buf, const FftPlan &pl, int ncols, int sm,
-                             int sc, const cx<T> *tw, FastDiv dcols) {
+#define FS_RADICES(X) X(16) X(12) X(10) X(9) X(8) X(6) X(5) X(4) X(3) X(2)
+
+// All stages of the run-time plan (fft_threads threads), the first reading
+// from ld, the last writing to st, the others in place in LDS. Ends without a
+// barrier after the last writes.
+template <typename T, bool PAD, bool INV, typename LD, typename ST>
+__device__ void lds_fft_plan(LdsIO<T, PAD> io, const FftPlan &pl, int ncols,
+                             const cx<T> *tw, FastDiv dcols, LD ld, ST st) {
+  constexpr bool same = std::is_same<LD, LdsIO<T, PAD>>::value;
+  constexpr bool into = std::is_same<ST, LdsIO<T, PAD>>::value;
   int ns = 1;
   for (int s = 0; s < pl.nst; ++s) {
     const int R = pl.rad[s];
     const FastDiv a = pl.dnb[s], b = pl.dns[s];
-    switch (R) {
-#define FS_STAGE(RR)                                                         \
-  case RR:                                                                   \
-    fft_stage<T, RR, PAD, INV>(buf, pl.n, ns, ncols, sm, sc, tw, a, b, dcols); \
+    if (s == 0) {
+      switch (R) {
+#define FS_STAGE(RR)                                                           \
+  case RR:                                                                     \
+    fft_stage<T, RR, PAD, INV, same>(ns, ncols, tw, a, b, dcols, ld, io);      \
     break;
-      FS_STAGE(16)
-      FS_STAGE(12)
-      FS_STAGE(10)
-      FS_STAGE(9)
-      FS_STAGE(8)
-      FS_STAGE(6)
-      FS_STAGE(5)
-      FS_STAGE(4)
-      FS_STAGE(3)
-      FS_STAGE(2)
+        FS_RADICES(FS_STAGE)
 #undef FS_STAGE
+      }
+      __syncthreads();
+    } else if (s + 1 < pl.nst) {
+      switch (R) {
+#define FS_STAGE(RR)                                                           \
+  case RR:                                                                     \
+    fft_stage<T, RR, PAD, INV, true>(ns, ncols, tw, a, b, dcols, io, io);      \
+    break;
+        FS_RADICES(FS_STAGE)
+#undef FS_STAGE
+      }
+      __syncthreads();
+    } else {
+      switch (R) {
+#define FS_STAGE(RR)                                                           \
+  case RR:                                                                     \
+    fft_stage<T, RR, PAD, INV, into>(ns, ncols, tw, a, b, dcols, io, st);      \
+    break;
+        FS_RADICES(FS_STAGE)
+#undef FS_STAGE
+      }
     }
     ns *= R;
   }
@@ -479,9 +525,11 @@ constexpr int p2_radix() {
                                          : 2;
 }
 
-template <typename T, int E, bool PAD, bool INV, int LOGN, int LOGNS>
-__device__ __forceinline__ void p2_stage(cx<T> *buf, int ncols, int sm,
-                                         const cx<T> *tw, FastDiv dcols) {
+template <typename T, int E, bool PAD, bool INV, int LOGN, int LOGNS,
+          typename LD, typename ST>
+__device__ __forceinline__ void p2_stage(LdsIO<T, PAD> io, int ncols,
+                                         const cx<T> *tw, FastDiv dcols, LD ld,
+                                         ST st) {
   constexpr int R = p2_radix<LOGN, LOGNS, E>();
   constexpr int LOGR = ilog2_c(R);
   constexpr int NB = E / R;
@@ -490,7 +538,13 @@ __device__ __forceinline__ void p2_stage(cx<T> *buf, int ncols, int sm,
   constexpr int ns = 1 << LOGNS;
   constexpr int LOGTW = LOGN - LOGNS - LOGR;  // twiddle step n / (ns R)
   constexpr int PN = fft_padded_len(1 << LOGN);
+  constexpr bool from_lds =
+      LOGNS > 0 || std::is_same<LD, LdsIO<T, PAD>>::value;
+  constexpr bool to_lds =
+      LOGNS + LOGR < LOGN || std::is_same<ST, LdsIO<T, PAD>>::value;
   static_assert(E % R == 0, "register tile must hold whole butterflies");
+  cx<T> *buf = io.buf;
+  const int sm = io.sm;
   cx<T> v[E];
   int jj[NB], cc[NB];
 #pragma unroll
@@ -506,8 +560,10 @@ __device__ __forceinline__ void p2_stage(cx<T> *buf, int ncols, int sm,
     }
     jj[m] = j;
     cc[m] = col;
-    const int k = j & (ns - 1);
-    if constexpr (PAD) {
+    if constexpr (!from_lds) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[m * R + r] = ld(j + r * nb, col);
+    } else if constexpr (PAD) {
       const cx<T> *src = buf + col * PN;
       const int pj = fft_pad(j);
 #pragma unroll
@@ -524,6 +580,10 @@ __device__ __forceinline__ void p2_stage(cx<T> *buf, int ncols, int sm,
       for (int r = 0; r < R; ++r)
         v[m * R + r] = buf[fft_rowpad(j + r * nb) * sm + col];
     }
+  }
+#pragma unroll
+  for (int m = 0; m < NB; ++m) {
+    const int k = jj[m] & (ns - 1);
     if constexpr (LOGNS > 0) {
 #pragma unroll
       for (int r = 1; r < R; ++r) {
@@ -534,12 +594,15 @@ __device__ __forceinline__ void p2_stage(cx<T> *buf, int ncols, int sm,
     }
     dftR<T, R>(&v[m * R], INV);
   }
-  __syncthreads();
+  if constexpr (from_lds && to_lds) __syncthreads();
 #pragma unroll
   for (int m = 0; m < NB; ++m) {
     const int j = jj[m], col = cc[m];
     const int d = ((j >> LOGNS) << (LOGNS + LOGR)) + (j & (ns - 1));
-    if constexpr (PAD) {
+    if constexpr (!to_lds) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) st(d + r * ns, col, v[m * R + r]);
+    } else if constexpr (PAD) {
       cx<T> *dst = buf + col * PN;
       const int pd = fft_pad(d);
 #pragma unroll
@@ -557,31 +620,25 @@ __device__ __forceinline__ void p2_stage(cx<T> *buf, int ncols, int sm,
         buf[fft_rowpad(d + r * ns) * sm + col] = v[m * R + r];
     }
   }
-  __syncthreads();
-}
-
-template <typename T, int E, bool PAD, bool INV, int LOGN, int LOGNS>
-__device__ __forceinline__ void p2_stages(cx<T> *buf, int ncols, int sm,
-                                          const cx<T> *tw, FastDiv dcols) {
-  if constexpr (LOGNS < LOGN) {
-    p2_stage<T, E, PAD, INV, LOGN, LOGNS>(buf, ncols, sm, tw, dcols);
-    constexpr int LOGR = ilog2_c(p2_radix<LOGN, LOGNS, E>());
-    p2_stages<T, E, PAD, INV, LOGN, LOGNS + LOGR>(buf, ncols, sm, tw, dcols);
+  if constexpr (LOGNS + LOGR < LOGN) {
+    __syncthreads();
+    p2_stage<T, E, PAD, INV, LOGN, LOGNS + LOGR>(io, ncols, tw, dcols, ld, st);
   }
 }
 
 // The transform for kernels instantiated on LOGN: LOGN > 0 takes the
 // compile-time plan (n = 2^LOGN, PAD: sc = fft_padded_len(n)), LOGN = 0 the
-// run-time plan pl.
-template <typename T, int E, bool PAD, bool INV, int LOGN>
-__device__ __forceinline__ void lds_fft(cx<T> *buf, const FftPlan &pl,
-                                        int ncols, int sm, int sc,
-                                        const cx<T> *tw,
+// run-time plan pl. The first stage reads from ld, the last writes to st:
+// global memory, or io for LDS. No barrier after the last writes.
+template <typename T, int E, bool PAD, bool INV, int LOGN, typename LD,
+          typename ST>
+__device__ __forceinline__ void lds_fft(LdsIO<T, PAD> io, const FftPlan &pl,
+                                        int ncols, const cx<T> *tw, LD ld, ST st,
                                         FastDiv dcols = FastDiv{0, 0}) {
   if constexpr (LOGN > 0)
-    p2_stages<T, E, PAD, INV, LOGN, 0>(buf, ncols, sm, tw, dcols);
+    p2_stage<T, E, PAD, INV, LOGN, 0>(io, ncols, tw, dcols, ld, st);
   else
-    lds_fft_plan<T, PAD, INV>(buf, pl, ncols, sm, sc, tw, dcols);
+    lds_fft_plan<T, PAD, INV>(io, pl, ncols, tw, dcols, ld, st);
 }
 
 }  // namespace fs
