@@ -107,6 +107,71 @@ struct Mfma<double> {
   }
 };
 
+// Sums over the four 16-lane groups of four values at once: lane group q gets
+// the total of v_q, (0 + 2) + (1 + 3). v_permlane32_swap exchanges the upper
+// half of one register with the lower half of another, v_permlane16_swap the
+// odd with the even rows of 16: five exchanges less than four butterflies,
+// and none through LDS.
+template <typename T>
+__device__ __forceinline__ T lane_reduce4(T v0, T v1, T v2, T v3) {
+  constexpr int W = sizeof(T) / 4;
+  const auto swap = [](T &a, T &b, auto exchange) {
+    unsigned ua[W], ub[W];
+    __builtin_memcpy(ua, &a, sizeof(T));
+    __builtin_memcpy(ub, &b, sizeof(T));
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const auto r = exchange(ua[w], ub[w]);
+      ua[w] = r[0];
+      ub[w] = r[1];
+    }
+    __builtin_memcpy(&a, ua, sizeof(T));
+    __builtin_memcpy(&b, ub, sizeof(T));
+  };
+  const auto s32 = [](unsigned a, unsigned b) {
+    return __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  };
+  const auto s16 = [](unsigned a, unsigned b) {
+    return __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  };
+  swap(v0, v2, s32);
+  swap(v1, v3, s32);
+  T s = v0 + v2, t = v1 + v3;  // rows (v0, v0, v2, v2) and (v1, v1, v3, v3)
+  swap(s, t, s16);
+  return s + t;
+}
+
+// 2^t for t <= 0 in FP64: 2^(t - n) by its Taylor series on [-1/2, 1/2]
+// (degree 13: remainder 4e-18) scaled by 2^n. What underflows is 0, NaN stays
+// NaN. Half the instructions of exp(), whose range checks the weights do not
+// need.
+__device__ __forceinline__ double exp2_neg(double t) {
+  t = t < -1100.0 ? -1100.0 : t;
+  const double n = rint(t), f = (t - n) * 0.69314718055994530941723212145818;
+  double p = 1.0 / 6227020800.0;
+  p = fma(p, f, 1.0 / 479001600.0);
+  p = fma(p, f, 1.0 / 39916800.0);
+  p = fma(p, f, 1.0 / 3628800.0);
+  p = fma(p, f, 1.0 / 362880.0);
+  p = fma(p, f, 1.0 / 40320.0);
+  p = fma(p, f, 1.0 / 5040.0);
+  p = fma(p, f, 1.0 / 720.0);
+  p = fma(p, f, 1.0 / 120.0);
+  p = fma(p, f, 1.0 / 24.0);
+  p = fma(p, f, 1.0 / 6.0);
+  p = fma(p, f, 0.5);
+  p = fma(p, f, 1.0);
+  p = fma(p, f, 1.0);
+  return ldexp(p, (int)n);
+}
+
+// Orders a wavefront's own LDS writes before its reads of them.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Tiles of te points that a stencil of ngd points can meet along an axis.
 __host__ __device__ constexpr int stencil_tiles(int ngd, int te) {
   return (ngd + te - 2) / te + 1;

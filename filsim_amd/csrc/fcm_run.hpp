@@ -586,10 +586,12 @@ __global__ void __launch_bounds__(256)
 // Gaussian weights of one segment at a tile's axis points. Point a: x
 // (a < 8), y (8 <= a < 16), z (16 <= a < 32) of the tile starting at
 // (px0, py0, pz0). w[a] = g (monopole), w[32 + a] = gD (dipole), w[64 + a]
-// = the gradient factor -xx / sigma_dip^2, zero off the stencil; xx is
-// formed in FP64. FP64 uses the expressions of k_prepare_tab; FP32 rounds
-// the exponent, formed in FP64 in base 2, before the hardware exp2.
-constexpr int kTileW = 104;  // weights (96) + coefficients (8) per record
+// = its derivative h = gD (-xx / sigma_dip^2), zero off the stencil; xx is
+// formed in FP64, and so is the exponent (base 2); FP32 rounds it before the
+// hardware exp2.
+// weights (96) + coefficients (6) per record; odd, so that 16 rows read at one
+// point fall on different banks
+constexpr int kTileW = 105;
 template <typename T>
 __device__ __forceinline__ void tile_weights(const GaussConst &g,
                                              const SegRec<T> &r, int a, int px0,
@@ -599,67 +601,87 @@ __device__ __forceinline__ void tile_weights(const GaussConst &g,
   const int n = d == 0 ? g.nx : (d == 1 ? g.ny : g.nz);
   int i = p - ((r.org >> (10 * d)) & 1023);
   if (i < 0) i += n;
-  T ga = 0, gd = 0, gr = 0;
+  T ga = 0, gd = 0, h = 0;
   if (i < g.ngd) {
     const double x0 = d == 0 ? r.xx0[0] : (d == 1 ? r.xx0[1] : r.xx0[2]);
     const double xx = x0 + (double)i * g.dx;
+    const double x2 = xx * xx;
     if constexpr (sizeof(T) == 8) {
-      ga = g.anorm * exp(-xx * xx / g.anorm2);
-      gd = g.anormdip * exp(-xx * xx / g.anormdip2);
-      gr = -xx / g.sigmadipsq;
+      ga = g.anorm * exp2_neg(-x2 * g.e2);
+      gd = g.anormdip * exp2_neg(-x2 * g.ed2);
     } else {
-      const double x2 = xx * xx;
       ga = (float)g.anorm * __builtin_amdgcn_exp2f((float)(-x2 * g.e2));
       gd = (float)g.anormdip * __builtin_amdgcn_exp2f((float)(-x2 * g.ed2));
-      gr = (float)(xx * g.nrsd);
     }
+    h = gd * (T)(xx * g.nrsd);
   }
   w[a] = ga;
   w[32 + a] = gd;
-  w[64 + a] = gr;
+  w[64 + a] = h;
 }
 
 // Weights (and, with CF, coefficients) of records s_rec[c0 .. c0 + nc) into
-// s_w[0 .. KC); rows nc .. KC are zero. 256 threads.
-template <typename T, int KC, bool CF>
+// s_w[0 .. nc). 256 threads.
+template <typename T, bool CF>
 __device__ __forceinline__ void tile_chunk_weights(const GaussConst &g,
                                                    const SegRec<T> *s_rec,
                                                    int c0, int nc, int px0,
                                                    int py0, int pz0,
                                                    T (*s_w)[kTileW]) {
-#pragma unroll
-  for (int e = threadIdx.x; e < KC * 32; e += 256) {
+  for (int e = threadIdx.x; e < nc * 32; e += 256) {
     const int c = e >> 5, a = e & 31;
-    if (c < nc) {
-      tile_weights<T>(g, s_rec[c0 + c], a, px0, py0, pz0, s_w[c]);
-    } else {
-      s_w[c][a] = 0;
-      s_w[c][32 + a] = 0;
-      s_w[c][64 + a] = 0;
-    }
+    tile_weights<T>(g, s_rec[c0 + c], a, px0, py0, pz0, s_w[c]);
   }
   if constexpr (CF) {
-    for (int e = threadIdx.x; e < KC * 8; e += 256) {
-      const int c = e >> 3, k = e & 7;
-      s_w[c][96 + k] = (c < nc && k < 6) ? s_rec[c0 + c].cf[k] : (T)0;
+    for (int e = threadIdx.x; e < nc * 6; e += 256) {
+      const int c = e / 6, k = e - 6 * c;
+      s_w[c][96 + k] = s_rec[c0 + c].cf[k];
     }
   }
+}
+
+// A wavefront's candidates among rows s_w[0 .. nc): those with a stencil
+// point in x columns 2 wave and 2 wave + 1 of the tile (non-zero monopole or
+// dipole weight; the others add exact zeros there). Their rows go to wl[0 ..
+// count), then pad entries of the zero row KC.
+template <typename T, int KC>
+__device__ __forceinline__ int wave_candidates(const T (*s_w)[kTileW], int nc,
+                                               int wave, int lane, int pad,
+                                               int *wl) {
+  const T *w = s_w[lane < nc ? lane : KC];
+  const bool mine =
+      lane < nc && (w[2 * wave] != (T)0 || w[2 * wave + 1] != (T)0 ||
+                    w[32 + 2 * wave] != (T)0 || w[33 + 2 * wave] != (T)0);
+  const unsigned long long mm = __ballot(mine);
+  const int n = __popcll(mm);
+  if (mine) wl[__popcll(mm & ((1ull << lane) - 1ull))] = lane;
+  if (lane < pad) wl[n + lane] = KC;
+  wave_lds_fence();
+  return n;
 }
 
 // ---------------------------------------------------------------------
 // spread on the matrix cores: one workgroup per 8 x 8 x 16 tile,
 // four wavefronts of 16 (x, y) points each. Per component the tile is
 //   R[xy][z] = sum over candidates c and terms t of A_t[xy][c] * B_t[c][z]
-// with the force term   A_0 = F * gx gy,            B_0 = gz,
-// and the torque terms  A_1 = (ax, ay, az) gdx gdy,  B_1 = gdz,
-//                       A_2 = (-G_y, G_x, 0) gdx gdy, B_2 = gdz * grad_z
-// (ax = G_z grad_y, ay = -G_z grad_x, az = G_y grad_x - G_x grad_y, G the
-// half torque: the same sum as k_spread). Each MFMA 16x16x4 step takes four
+// with the force term   A_0 = F * gx gy,                      B_0 = gz,
+// and the torque terms  A_1 = (G_z gDx hy, -G_z hx gDy,
+//                              G_y hx gDy - G_x gDx hy),       B_1 = gDz,
+//                       A_2 = (-G_y, G_x, 0) gDx gDy,          B_2 = hz
+// (h the derivative of the dipole Gaussian gD, G the half torque: the same
+// sum as k_spread). Each MFMA 16x16x4 step takes four
 // candidates of one term; lane l supplies A[xy = l % 16][c = l / 16] and
 // B[c = l / 16][z = l % 16] and holds R[xy = Mfma<T>::row(l, r)][z = l % 16].
-// Weights are zero off a candidate's stencil and for the unused rows of a
-// round. Candidates are summed in tile-list order: no atomics, no zeroing
-// pass, every grid point written once.
+// Weights are zero off a candidate's stencil, and the entries that fill a
+// wave's last step are the zero row. Candidates are summed in tile-list
+// order: no atomics, no zeroing pass, every grid point written once.
+// Bound by the matrix instructions and the latency of LDS reads and barriers
+// (a tile's grid values are 25 to 50 KB a workgroup, written once): the
+// matrix and vector units of a SIMD do not work at the same time here (12
+// MFMA 162 ns, 64 FMA 68 ns, both 239 ns), so instructions count, wherever
+// they run. 30k segments on 256^3 83 us FP32 / 151 us FP64 (with exp() for
+// the FP64 weights and the candidates walked in a bit mask 83 / 156), 128^3
+// FP64 39 -> 36 us. One wavefront to a tile, without barriers: 118 / 193 us.
 // ---------------------------------------------------------------------
 // Candidates per round (FP32 32, FP64 16: the same 13 KB of weights).
 template <typename T>
@@ -676,6 +698,7 @@ __device__ __forceinline__ void d_spread_mfma(const int *__restrict__ act, SG G,
   if (act && !*act) return;  // batched sweep: suspension converged
   __shared__ SegRec<T> s_rec[kTileCap];
   __shared__ T s_w[KC + 1][kTileW];  // row KC stays zero
+  __shared__ int s_wl[4][KC + 4];    // each wave's candidate list
 
   int bx, by, bz;
   tile_of_block(G, blockIdx.x, &bx, &by, &bz);
@@ -701,41 +724,26 @@ __device__ __forceinline__ void d_spread_mfma(const int *__restrict__ act, SG G,
     __syncthreads();
     for (int c0 = 0; c0 < nb; c0 += KC) {
       const int nc = min(KC, nb - c0);
-      tile_chunk_weights<T, KC, true>(g, s_rec, c0, nc, px0, py0, pz0, s_w);
+      tile_chunk_weights<T, true>(g, s_rec, c0, nc, px0, py0, pz0, s_w);
       __syncthreads();
-      // this wave's rows lie in x columns 2 wave and 2 wave + 1: candidates
-      // with no stencil point there (zero monopole and dipole weights in
-      // both) add exact zeros to them and are skipped
-      const T *wl = s_w[lane < nc ? lane : KC];
-      unsigned long long m = __ballot(
-          lane < nc && (wl[2 * wave] != (T)0 || wl[2 * wave + 1] != (T)0 ||
-                        wl[32 + 2 * wave] != (T)0 || wl[33 + 2 * wave] != (T)0));
-      const int nw = __popcll(m);
+      const int nw = wave_candidates<T, KC>(s_w, nc, wave, lane, 4, s_wl[wave]);
       for (int c4 = 0; c4 < nw; c4 += 4) {
         // lane group q takes the (c4 + q)-th candidate of the wave's list
         // (the zero row past its end)
-        int c = KC;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int ck = m ? (int)__builtin_ctzll(m) : KC;
-          if (k == q) c = ck;
-          m &= m - 1;
-        }
-        const T *w = s_w[c];
+        const T *w = s_w[s_wl[wave][c4 + q]];
         const T *cf = w + 96;
-        const T gxy = w[lx] * w[8 + ly], dxy = w[32 + lx] * w[40 + ly];
-        const T xx = w[64 + lx], yy = w[72 + ly];
-        const T gz = w[16 + lz], gdz = w[48 + lz], grz = w[80 + lz];
-        const T ax = cf[5] * yy, ay = -cf[5] * xx, az = cf[4] * xx - cf[3] * yy;
-        const T b2 = gdz * grz;
+        const T gx = w[lx], dx = w[32 + lx], hx = w[64 + lx];
+        const T gy = w[8 + ly], dy = w[40 + ly], hy = w[72 + ly];
+        const T gz = w[16 + lz], dz = w[48 + lz], hz = w[80 + lz];
+        const T gxy = gx * gy, dxy = dx * dy, dhy = dx * hy, hdy = hx * dy;
         acc0 = Mfma<T>::step(cf[0] * gxy, gz, acc0);
         acc1 = Mfma<T>::step(cf[1] * gxy, gz, acc1);
         acc2 = Mfma<T>::step(cf[2] * gxy, gz, acc2);
-        acc0 = Mfma<T>::step(ax * dxy, gdz, acc0);
-        acc1 = Mfma<T>::step(ay * dxy, gdz, acc1);
-        acc2 = Mfma<T>::step(az * dxy, gdz, acc2);
-        acc0 = Mfma<T>::step(-cf[4] * dxy, b2, acc0);
-        acc1 = Mfma<T>::step(cf[3] * dxy, b2, acc1);
+        acc0 = Mfma<T>::step(cf[5] * dhy, dz, acc0);
+        acc1 = Mfma<T>::step(-cf[5] * hdy, dz, acc1);
+        acc2 = Mfma<T>::step(cf[4] * hdy - cf[3] * dhy, dz, acc2);
+        acc0 = Mfma<T>::step(-cf[4] * dxy, hz, acc0);
+        acc1 = Mfma<T>::step(cf[3] * dxy, hz, acc1);
       }
       __syncthreads();  // the next round overwrites the weights
     }
@@ -1469,13 +1477,20 @@ __global__ void __launch_bounds__(256)
 // with each segment's weights:
 //   P_m[xy][c] = sum_z u_d[xy][z] b_m,c[z]   (per wave 16 xy rows x 16
 //   segments, v_mfma 16x16x4 over z; 8 products m: u_0..2 with g_z,
-//   u_0..2 with gD_z, u_0..1 with gD_z grad_z)
+//   u_0..2 with gD_z, u_0..1 with the derivative h_z)
 // then weights each (x, y) row with the segment's x and y factors, sums
 // the lane's rows, the four lane groups and the four waves in a fixed
 // order, and stores the tile's 6 partial sums per segment in
 // part[segment][component][slot] (slot = the tile's offset from the
 // segment's origin tile). k_interp_sum adds a segment's slots in slot
 // order: no atomics, results independent of scheduling.
+// Latency bound: of the FP64 270 us at 30k segments on 256^3 the products
+// take 90, the weights' reads from LDS 100, making the weights 50 and the
+// grid's loads 50, one after another. So wavefronts count: three accumulators
+// at a time fit 128 registers, four waves a SIMD instead of two (FP64 297 ->
+// 270 us, FP32 125 -> 120 us; 128^3 FP64 55 -> 46 us). One wavefront to a
+// tile 257 / 140 us, and slower on small grids; weights read 16 bytes at a
+// time 313 / 125 us (spills).
 // ---------------------------------------------------------------------
 template <int NGD>
 constexpr int kInterpSlots = stencil_tiles(NGD, 8) * stencil_tiles(NGD, 8) *
@@ -1501,8 +1516,8 @@ __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G,
   if (act && !*act) return;  // batched sweep: suspension converged
   __shared__ SegRec<T> s_rec[kTileCap];
   __shared__ T s_w[KC + 1][kTileW];  // row KC stays zero
-  __shared__ T s_red[4][KC][6];
-  __shared__ int s_wl[4][KC];  // each wave's candidate list
+  __shared__ T s_red[4][KC][8];  // 6 sums; two more keep the stores uniform
+  __shared__ int s_wl[4][KC + 16];  // each wave's candidate list
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int q = lane >> 4, i16 = lane & 15;
@@ -1551,79 +1566,83 @@ __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G,
         stage_tile_records<T>(slab, pool, tile, ovf, r0, nc, s_rec);
       }
       __syncthreads();
-      tile_chunk_weights<T, KC, false>(g, s_rec, 0, nc, px0, py0, pz0, s_w);
+      tile_chunk_weights<T, false>(g, s_rec, 0, nc, px0, py0, pz0, s_w);
       __syncthreads();
-      // this wave's rows lie in x columns 2 wave and 2 wave + 1: it handles
-      // only the candidates with a stencil point there (non-zero monopole or
-      // dipole weight), 16 per group, and leaves zeros for the others
+      // the wave handles its own candidates, 16 per group, and leaves zeros
+      // for the others
       {
-        const T *wl = s_w[lane < nc ? lane : KC];
-        const bool mine = lane < nc && (wl[2 * wave] != (T)0 ||
-                                        wl[2 * wave + 1] != (T)0 ||
-                                        wl[32 + 2 * wave] != (T)0 ||
-                                        wl[33 + 2 * wave] != (T)0);
-        const unsigned long long mm = __ballot(mine);
-        if (mine) s_wl[wave][__popcll(mm & ((1ull << lane) - 1ull))] = lane;
-        for (int e = lane; e < KC * 6; e += 64) (&s_red[wave][0][0])[e] = 0;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int nw = __popcll(mm);
+        for (int e = lane; e < KC * 8; e += 64) (&s_red[wave][0][0])[e] = 0;
+        const int nw = wave_candidates<T, KC>(s_w, nc, wave, lane, 16, s_wl[wave]);
         for (int g0 = 0; g0 < nw; g0 += 16) {
           // B operands: this lane's column is the wave's candidate g0 + i16
-          const int c = g0 + i16 < nw ? s_wl[wave][g0 + i16] : KC;
+          const int c = s_wl[wave][g0 + i16];
           const T *w = s_w[c];
+          // the monopole, dipole and derivative products one after another:
+          // three accumulators live at a time leave room for twice the
+          // wavefronts. Lane holds P[xy = wave*16 + row(lane, r)][candidate
+          // c] and weights each row with the candidate's x/y factors.
           const v4 z4 = {0, 0, 0, 0};
-          v4 pg0 = z4, pg1 = z4, pg2 = z4, pd0 = z4, pd1 = z4, pd2 = z4,
-             pr0 = z4, pr1 = z4;
-  #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int z = 4 * q + k;
-            const T gz = w[16 + z], gdz = w[48 + z];
-            const T grz = gdz * w[80 + z];
-            pg0 = Mfma<T>::step(u[0][k], gz, pg0);
-            pg1 = Mfma<T>::step(u[1][k], gz, pg1);
-            pg2 = Mfma<T>::step(u[2][k], gz, pg2);
-            pd0 = Mfma<T>::step(u[0][k], gdz, pd0);
-            pd1 = Mfma<T>::step(u[1][k], gdz, pd1);
-            pd2 = Mfma<T>::step(u[2][k], gdz, pd2);
-            pr0 = Mfma<T>::step(u[0][k], grz, pr0);
-            pr1 = Mfma<T>::step(u[1][k], grz, pr1);
-          }
-          // lane holds P[xy = wave*16 + row(lane, r)][candidate c]: weight
-          // each row with the candidate's x/y factors
           T v0 = 0, v1 = 0, v2 = 0, w0 = 0, w1 = 0, w2 = 0;
-  #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int rxy = wave * 16 + Mfma<T>::row(lane, r);
-            const int x = rxy >> 3, y = rxy & 7;
-            const T gxy = w[x] * w[8 + y], dxy = w[32 + x] * w[40 + y];
-            const T xx = w[64 + x], yy = w[72 + y];
-            v0 += gxy * pg0[r];
-            v1 += gxy * pg1[r];
-            v2 += gxy * pg2[r];
-            w0 += dxy * (yy * pd2[r] - pr1[r]);
-            w1 += dxy * (pr0[r] - xx * pd2[r]);
-            w2 += dxy * (xx * pd1[r] - yy * pd0[r]);
+          {
+            v4 p0 = z4, p1 = z4, p2 = z4;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const T gz = w[16 + 4 * q + k];
+              p0 = Mfma<T>::step(u[0][k], gz, p0);
+              p1 = Mfma<T>::step(u[1][k], gz, p1);
+              p2 = Mfma<T>::step(u[2][k], gz, p2);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int rxy = wave * 16 + Mfma<T>::row(lane, r);
+              const T gxy = w[rxy >> 3] * w[8 + (rxy & 7)];
+              v0 += gxy * p0[r];
+              v1 += gxy * p1[r];
+              v2 += gxy * p2[r];
+            }
           }
-          // the four lane groups (rows) of the wave
-  #pragma unroll
-          for (int off = 16; off < 64; off <<= 1) {
-            v0 += __shfl_xor(v0, off, 64);
-            v1 += __shfl_xor(v1, off, 64);
-            v2 += __shfl_xor(v2, off, 64);
-            w0 += __shfl_xor(w0, off, 64);
-            w1 += __shfl_xor(w1, off, 64);
-            w2 += __shfl_xor(w2, off, 64);
+          {
+            v4 p0 = z4, p1 = z4, p2 = z4;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const T dz = w[48 + 4 * q + k];
+              p0 = Mfma<T>::step(u[0][k], dz, p0);
+              p1 = Mfma<T>::step(u[1][k], dz, p1);
+              p2 = Mfma<T>::step(u[2][k], dz, p2);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int rxy = wave * 16 + Mfma<T>::row(lane, r);
+              const int x = rxy >> 3, y = rxy & 7;
+              const T dhy = w[32 + x] * w[72 + y], hdy = w[64 + x] * w[40 + y];
+              w0 += dhy * p2[r];
+              w1 -= hdy * p2[r];
+              w2 += hdy * p1[r] - dhy * p0[r];
+            }
           }
-          if (q == 0 && c < KC) {
-            T *sr = s_red[wave][c];
-            sr[0] = v0;
-            sr[1] = v1;
-            sr[2] = v2;
-            sr[3] = w0;
-            sr[4] = w1;
-            sr[5] = w2;
+          {
+            v4 p0 = z4, p1 = z4;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const T hz = w[80 + 4 * q + k];
+              p0 = Mfma<T>::step(u[0][k], hz, p0);
+              p1 = Mfma<T>::step(u[1][k], hz, p1);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int rxy = wave * 16 + Mfma<T>::row(lane, r);
+              const T dxy = w[32 + (rxy >> 3)] * w[40 + (rxy & 7)];
+              w0 -= dxy * p1[r];
+              w1 += dxy * p0[r];
+            }
+          }
+          // the four lane groups (rows) of the wave: group q gets sums q and
+          // 4 + q
+          const T a = lane_reduce4<T>(v0, v1, v2, w0);
+          const T b = lane_reduce4<T>(w1, w2, (T)0, (T)0);
+          if (c < KC) {
+            s_red[wave][c][q] = a;
+            s_red[wave][c][4 + q] = b;
           }
         }
       }
@@ -1647,7 +1666,7 @@ __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G,
   }
 }
 template <typename T, int NGD>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 4)
     k_interp_mfma(const int *__restrict__ act, SpreadGeom G, GaussConst g,
                   const SegRec<T> *__restrict__ slab,
                   const SegRec<T> *__restrict__ pool,
@@ -1671,7 +1690,7 @@ struct A_interp_mfma {
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
 template <typename T, int NGD>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 4)
     k_interp_mfma_multi(const A_interp_mfma<T, NGD> *__restrict__ a) {
   const A_interp_mfma<T, NGD> &A = a[blockIdx.z];
   d_interp_mfma<T, NGD, const SpreadGeom &, const GaussConst &>(A.act, A.G, A.g, A.slab, A.pool, A.tcnt, A.tovf, A.R, A.part);
