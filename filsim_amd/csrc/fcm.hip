@@ -135,6 +135,7 @@ int FcmImpl::init(const fs_fcm_params &pp, int maxnp, int prec) {
   FS_TRY(bin.alloc((size_t)maxnp * sizeof(int)));
   FS_TRY(slot.alloc((size_t)maxnp * sizeof(int)));
   FS_TRY(ids.alloc((size_t)maxnp * sizeof(int)));
+  FS_TRY(sids.alloc((size_t)maxnp * sizeof(int)));
   tune.fft_batch = (prec == FS_FP64) ? 8 : 16;
   tune.spread_tile = 16;
   tune.spread_zrun = 8;
@@ -226,6 +227,12 @@ int FcmImpl::set_geometry() {
     FS_TRY(tpool.alloc((size_t)max_np * nslot * rec_bytes(tsz)));
     grid_interp = tsz == 8 ? interp_blocks<double>(*this) : interp_blocks<float>(*this);
   }
+  // Lists without bins where every row of tiles can look at all segments. Both
+  // sides in us, of all launches that make the lists, binned and direct: 240
+  // segments on 64^3 (32 row steps) 31 and 16; 3,600 on 128^3 (512) 43 and 26;
+  // 2,400 on 192^3 (864) 37 and 28, growing with the row steps.
+  direct = mfma_spread && max_np <= kDirectMax &&
+           (long)ceil_div(max_np, 1024) * geom.nby * geom.nbz <= kDirectRowSteps;
   // one more counter after the bins: the tile lists' pool top
   FS_TRY(bin_count.alloc((size_t)(nbins + 1) * sizeof(int)));
   FS_HIP(hipMemset(bin_count.p, 0, (size_t)(nbins + 1) * sizeof(int)));
@@ -268,6 +275,7 @@ void FcmImpl::release() {
   bin.release();
   slot.release();
   ids.release();
+  sids.release();
   srec.release();
   sorg.release();
   tslab.release();
@@ -291,7 +299,8 @@ bool fcm_same_shapes(const FcmImpl &a, const FcmImpl &b) {
   return a.precision == b.precision && a.p.nx == b.p.nx && a.p.ny == b.p.ny &&
          a.p.nz == b.p.nz && a.p.ngd == b.p.ngd && a.mfma_spread && b.mfma_spread &&
          a.zP == b.zP && a.yB == b.yB && a.xQ == b.xQ &&
-         a.grid_interp == b.grid_interp && a.nbins == b.nbins;
+         a.grid_interp == b.grid_interp && a.nbins == b.nbins &&
+         a.direct == b.direct;
 }
 
 int FcmGroup::build() {

@@ -31,6 +31,9 @@ struct alignas(16) SegRec {
   T cf[6];
 };
 constexpr int kTileCap = 32;  // records in a tile's slab; the rest: pool
+constexpr int kDirectMax = 4096;  // segments of tile lists without bins (LDS)
+// steps of 1,024 segments over all rows of tiles, where the line to them lies
+constexpr long kDirectRowSteps = 1024;
 inline size_t rec_bytes(int tsz) {
   return tsz == 8 ? sizeof(SegRec<double>) : sizeof(SegRec<float>);
 }

@@ -36,13 +36,14 @@ struct FcmImpl {
   SpreadGeom geom{};
   int nbins = 0;
   bool mfma_spread = false;  // spread on the matrix cores (8 x 8 x 16 tiles)
+  bool direct = false;  // tile lists straight from the segments, without bins
   int grid_interp = 0;  // blocks of the persistent interpolation
   int zP = 1, yB = 1, xQ = 1;  // FFT pass workgroup shapes
   // device flag read by every kernel of a solve: 0 = skip (a converged
   // suspension of a batched sweep); nullptr = always run
   const int *act = nullptr;
   dbuf R, C, twx, twy, twz;
-  dbuf tab, origin, coef, bin, slot, ids, bin_count, bin_start, scan_tmp;
+  dbuf tab, origin, coef, bin, slot, ids, sids, bin_count, bin_start, scan_tmp;
   // matrix-core path: segment records and packed origins in bin order,
   // per-tile record lists (slab of kTileCap per tile, count, pool block of
   // the rest, the pool) and the interpolation's partial sums

@@ -30,11 +30,18 @@ constexpr int kCandChunk = 16;  // segments staged in LDS per spread chunk
 // FCMfunctions.cpp:565-567. A coordinate that is not finite or lies more
 // than 2^30 cells out (a diverged iterate) gets cell s instead: no
 // saturating conversion or signed overflow downstream, and such segments
-// spread over many bins rather than piling into one (the per-bin sort is
+// spread over many bins rather than piling into one (the order in a bin is
 // quadratic in the bin's population). Its tables are then 0 or NaN.
 __device__ __forceinline__ int stencil_cell(double y, double dx, int s) {
   const double cy = y / dx;
   return fabs(cy) < 1073741824.0 ? (int)cy : s;
+}
+
+// Wrapped index of support point 0 of the stencil around coordinate y.
+__device__ __forceinline__ int stencil_origin(double y, double dx, int s,
+                                              int ngdh, int n) {
+  const int w = (stencil_cell(y, dx, s) - ngdh + 1) % n;
+  return w < 0 ? w + n : w;
 }
 
 // Bin of tile (bx, by, bz): z fastest, so the bin-sorted segment list runs
@@ -79,20 +86,20 @@ __device__ __forceinline__ void d_prepare(const int *__restrict__ act, int np, c
   const int nn[3] = {g.nx, g.ny, g.nz};
   int o[3];
   for (int d = 0; d < 3; ++d) {
-    int c = stencil_cell(Y[3 * s + d], g.dx, s);
-    int w = (c - g.ngdh + 1) % nn[d];
-    if (w < 0) w += nn[d];
-    o[d] = w;
-    origin[3 * s + d] = w;
+    o[d] = stencil_origin(Y[3 * s + d], g.dx, s, g.ngdh, nn[d]);
+    origin[3 * s + d] = o[d];
   }
-  // spread coefficients: F and half torque (GA_setup: GA = T/2 pattern),
-  // kCoef per segment so a record is whole 16-byte words
-  for (int d = 0; d < 3; ++d) {
-    coef[kCoef * s + d] = (T)F[3 * s + d];
-    coef[kCoef * s + 3 + d] = (T)(0.5 * Tq[3 * s + d]);
+  // spread coefficients of the vector path (the matrix-core path keeps them in
+  // its records): F and half torque (GA_setup: GA = T/2 pattern), kCoef per
+  // segment so a record is whole 16-byte words
+  if (coef) {
+    for (int d = 0; d < 3; ++d) {
+      coef[kCoef * s + d] = (T)F[3 * s + d];
+      coef[kCoef * s + 3 + d] = (T)(0.5 * Tq[3 * s + d]);
+    }
+    coef[kCoef * s + 6] = (T)0;
+    coef[kCoef * s + 7] = (T)0;
   }
-  coef[kCoef * s + 6] = (T)0;
-  coef[kCoef * s + 7] = (T)0;
   int b = spread_bin(o[0] / tx, o[1] / ty, o[2] / tz, nbx, nby, nbz);
   bin[s] = b;
   slot[s] = atomicAdd(&bin_count[b], 1);
@@ -185,68 +192,78 @@ static __global__ void k_scatter_multi(const A_scatter *__restrict__ a) {
   d_scatter(A.np, A.bin, A.slot, A.start, A.ids);
 }
 
-// Ascending segment order inside each bin (atomic slots are unordered);
-// srec and sorg (the matrix-core path; may be null) receive each segment's
-// record and packed stencil origin in the same order.
+// Record of segment s, whose stencil origin is (o0, o1, o2).
 template <typename T>
-__device__ __forceinline__ void d_sort_bins(const int *__restrict__ act, int nbins,
-                            const int *__restrict__ start,
-                            int *__restrict__ ids,
-                            const int *__restrict__ origin,
-                            const double *__restrict__ Y,
-                            const double *__restrict__ F,
-                            const double *__restrict__ Tq, double dx,
-                            int ngdh, SegRec<T> *__restrict__ srec,
-                            int *__restrict__ sorg) {
-  if (act && !*act) return;  // batched sweep: suspension converged
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nbins) return;
-  int lo = start[b], hi = start[b + 1];
-  for (int i = lo + 1; i < hi; ++i) {
-    int v = ids[i];
-    int j = i - 1;
-    while (j >= lo && ids[j] > v) {
-      ids[j + 1] = ids[j];
-      --j;
-    }
-    ids[j + 1] = v;
+__device__ __forceinline__ SegRec<T> segment_record(
+    int s, int o0, int o1, int o2, const double *__restrict__ Y,
+    const double *__restrict__ F, const double *__restrict__ Tq, double dx,
+    int ngdh) {
+  SegRec<T> r;
+  for (int d = 0; d < 3; ++d) {
+    const double y = Y[3 * s + d];
+    r.xx0[d] = ((double)(stencil_cell(y, dx, s) - ngdh + 1)) * dx - y;
+    r.cf[d] = (T)F[3 * s + d];
+    r.cf[3 + d] = (T)(0.5 * Tq[3 * s + d]);
   }
-  if (srec)
-    for (int i = lo; i < hi; ++i) {
-      const int sid = ids[i];
-      SegRec<T> r;
-      for (int d = 0; d < 3; ++d) {
-        const double y = Y[3 * sid + d];
-        r.xx0[d] = ((double)(stencil_cell(y, dx, sid) - ngdh + 1)) * dx - y;
-        r.cf[d] = (T)F[3 * sid + d];
-        r.cf[3 + d] = (T)(0.5 * Tq[3 * sid + d]);
-      }
-      r.id = sid;
-      r.org = origin[3 * sid] | (origin[3 * sid + 1] << 10) |
-              (origin[3 * sid + 2] << 20);
-      srec[i] = r;
-      sorg[i] = r.org;
-    }
+  r.id = s;
+  r.org = o0 | (o1 << 10) | (o2 << 20);
+  return r;
 }
+
+// Ascending segment order inside each bin (atomic slots are unordered): a
+// thread per segment counts the smaller ids in its bin (ids, unordered) and
+// writes its id to that place of sids, or (the matrix-core path) its record
+// and packed stencil origin to that place of srec and sorg. A thread per bin
+// sorting it by insertion is a chain of dependent loads and stores: all launches
+// up to here 36 -> 22 us at 30k segments on 256^3, 63 -> 50 us at 240k on 512^3.
 template <typename T>
-__global__ void k_sort_bins(const int *__restrict__ act, int nbins,
+__device__ __forceinline__ void d_bin_order(const int *__restrict__ act, int np,
+                            const int *__restrict__ bin,
                             const int *__restrict__ start,
-                            int *__restrict__ ids,
+                            const int *__restrict__ ids,
                             const int *__restrict__ origin,
                             const double *__restrict__ Y,
                             const double *__restrict__ F,
                             const double *__restrict__ Tq, double dx,
                             int ngdh, SegRec<T> *__restrict__ srec,
-                            int *__restrict__ sorg) {
-  d_sort_bins<T>(act, nbins, start, ids, origin, Y, F, Tq, dx, ngdh, srec, sorg);
+                            int *__restrict__ sorg, int *__restrict__ sids) {
+  if (act && !*act) return;  // batched sweep: suspension converged
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= np) return;
+  const int b = bin[s];
+  const int lo = start[b], hi = start[b + 1];
+  int pos = lo;
+  for (int i = lo; i < hi; ++i) pos += ids[i] < s;
+  if (srec) {
+    const SegRec<T> r = segment_record<T>(s, origin[3 * s], origin[3 * s + 1],
+                                          origin[3 * s + 2], Y, F, Tq, dx, ngdh);
+    srec[pos] = r;
+    sorg[pos] = r.org;
+  } else {
+    sids[pos] = s;
+  }
 }
-// arguments of one suspension for k_sort_bins_multi
 template <typename T>
-struct A_sort_bins {
+__global__ void k_bin_order(const int *__restrict__ act, int np,
+                            const int *__restrict__ bin,
+                            const int *__restrict__ start,
+                            const int *__restrict__ ids,
+                            const int *__restrict__ origin,
+                            const double *__restrict__ Y,
+                            const double *__restrict__ F,
+                            const double *__restrict__ Tq, double dx,
+                            int ngdh, SegRec<T> *__restrict__ srec,
+                            int *__restrict__ sorg, int *__restrict__ sids) {
+  d_bin_order<T>(act, np, bin, start, ids, origin, Y, F, Tq, dx, ngdh, srec, sorg, sids);
+}
+// arguments of one suspension for k_bin_order_multi
+template <typename T>
+struct A_bin_order {
   const int *act;
-  int nbins;
+  int np;
+  const int *bin;
   const int *start;
-  int *ids;
+  const int *ids;
   const int *origin;
   const double *Y;
   const double *F;
@@ -259,9 +276,9 @@ struct A_sort_bins {
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
 template <typename T>
-__global__ void k_sort_bins_multi(const A_sort_bins<T> *__restrict__ a) {
-  const A_sort_bins<T> &A = a[blockIdx.z];
-  d_sort_bins<T>(A.act, A.nbins, A.start, A.ids, A.origin, A.Y, A.F, A.Tq, A.dx, A.ngdh, A.srec, A.sorg);
+__global__ void k_bin_order_multi(const A_bin_order<T> *__restrict__ a) {
+  const A_bin_order<T> &A = a[blockIdx.z];
+  d_bin_order<T>(A.act, A.np, A.bin, A.start, A.ids, A.origin, A.Y, A.F, A.Tq, A.dx, A.ngdh, A.srec, A.sorg, nullptr);
 }
 
 // ---------------------------------------------------------------------
@@ -581,6 +598,142 @@ __global__ void __launch_bounds__(256)
     k_tile_lists_multi(const A_tile_lists<T> *__restrict__ a) {
   const A_tile_lists<T> &A = a[blockIdx.z];
   d_tile_lists<T, const SpreadGeom &>(A.act, A.G, A.start, A.sorg, A.srec, A.slab, A.tcnt, A.tovf, A.pool, A.pool_top);
+}
+
+// The tile lists of few segments without bins: one workgroup per row of tiles
+// along x. Its threads form every segment's origin and keep, in ascending
+// order, those whose stencil meets the row in y and z; then each wavefront
+// fills the lists of tiles of the row (order, slab, pool and counts as above,
+// except that a tile's segments are in ascending order over all bins). It
+// replaces prepare, scan, scatter, order and list launches, whose time is
+// latency at these sizes: 240 segments on 64^3 31 -> 16 us, 1,350 on 96^3 39 ->
+// 20 us, 2,400 on 192^3 37 -> 28 us. The pool's counter is zeroed by
+// k_interp_sum, which runs after the last use of the pool.
+template <typename T, typename SG = SpreadGeom>
+__device__ __forceinline__ void d_tile_lists_direct(
+    const int *__restrict__ act, int np, SG G, double dx,
+    const double *__restrict__ Y, const double *__restrict__ F,
+    const double *__restrict__ Tq, int *__restrict__ origin,
+    SegRec<T> *__restrict__ slab, int *__restrict__ tcnt,
+    int *__restrict__ tovf, SegRec<T> *__restrict__ pool,
+    int *__restrict__ pool_top) {
+  if (act && !*act) return;  // batched sweep: suspension converged
+  __shared__ int s_id[kDirectMax], s_org[kDirectMax];
+  __shared__ int s_cnt[2][16];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const int by = blockIdx.x % G.nby, bz = blockIdx.x / G.nby;
+  const int ngdh = G.ngd / 2;
+  int nrow = 0;  // segments that meet the row
+  for (int s0 = 0, it = 0; s0 < np; s0 += 1024, ++it) {
+    const int s = s0 + threadIdx.x;
+    // one workgroup a round also stores the origins
+    const bool own = it % (int)gridDim.x == (int)blockIdx.x;
+    bool keep = false;
+    int org = 0;
+    if (s < np) {
+      const int oy = stencil_origin(Y[3 * s + 1], dx, s, ngdh, G.ny);
+      const int oz = stencil_origin(Y[3 * s + 2], dx, s, ngdh, G.nz);
+      keep = stencil_meets(oy, by * G.ty, G.ty, G.ngd, G.ny) &&
+             stencil_meets(oz, bz * G.tz, G.tz, G.ngd, G.nz);
+      if (keep || own) {
+        const int ox = stencil_origin(Y[3 * s], dx, s, ngdh, G.nx);
+        org = ox | (oy << 10) | (oz << 20);
+        if (own) {
+          origin[3 * s] = ox;
+          origin[3 * s + 1] = oy;
+          origin[3 * s + 2] = oz;
+        }
+      }
+    }
+    const unsigned long long kb = __ballot(keep);
+    if (lane == 0) s_cnt[it & 1][wave] = __popcll(kb);
+    __syncthreads();
+    int at = nrow;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const int n = s_cnt[it & 1][w];
+      if (w < wave) at += n;
+      nrow += n;
+    }
+    if (keep) {
+      at += __popcll(kb & below);
+      s_id[at] = s;
+      s_org[at] = org;
+    }
+  }
+  __syncthreads();
+  for (int bx = wave; bx < G.nbx; bx += 16) {
+    const int tile = bx + G.nbx * blockIdx.x;
+    int kept = 0, base = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+      if (pass == 1) {
+        if (kept <= kTileCap) break;
+        int b0 = 0;
+        if (lane == 0) b0 = atomicAdd(pool_top, kept - kTileCap);
+        base = __shfl(b0, 0, 64);
+        kept = 0;
+      }
+      for (int j0 = 0; j0 < nrow; j0 += 64) {
+        const int j = j0 + lane;
+        const int org = j < nrow ? s_org[j] : 0;
+        const bool keep =
+            j < nrow && stencil_meets(org & 1023, bx * G.tx, G.tx, G.ngd, G.nx);
+        const unsigned long long kb = __ballot(keep);
+        const int k = kept + __popcll(kb & below);
+        if (keep && (pass == 0) == (k < kTileCap)) {
+          const SegRec<T> r =
+              segment_record<T>(s_id[j], org & 1023, (org >> 10) & 1023,
+                                org >> 20, Y, F, Tq, dx, ngdh);
+          if (pass == 0)
+            slab[(size_t)tile * kTileCap + k] = r;
+          else
+            pool[base + k - kTileCap] = r;
+        }
+        kept += __popcll(kb);
+      }
+    }
+    if (lane == 0) {
+      tcnt[tile] = kept;
+      tovf[tile] = base;
+    }
+  }
+}
+template <typename T>
+__global__ void __launch_bounds__(1024)
+    k_tile_lists_direct(const int *__restrict__ act, int np, SpreadGeom G,
+                        double dx, const double *__restrict__ Y,
+                        const double *__restrict__ F,
+                        const double *__restrict__ Tq, int *__restrict__ origin,
+                        SegRec<T> *__restrict__ slab, int *__restrict__ tcnt,
+                        int *__restrict__ tovf, SegRec<T> *__restrict__ pool,
+                        int *__restrict__ pool_top) {
+  d_tile_lists_direct<T>(act, np, G, dx, Y, F, Tq, origin, slab, tcnt, tovf, pool, pool_top);
+}
+// arguments of one suspension for k_tile_lists_direct_multi
+template <typename T>
+struct A_tile_lists_direct {
+  const int *act;
+  int np;
+  SpreadGeom G;
+  double dx;
+  const double *Y;
+  const double *F;
+  const double *Tq;
+  int *origin;
+  SegRec<T> *slab;
+  int *tcnt;
+  int *tovf;
+  SegRec<T> *pool;
+  int *pool_top;
+};
+// one launch for a group of suspensions with equal launch shapes:
+// blockIdx.z selects the suspension
+template <typename T>
+__global__ void __launch_bounds__(1024)
+    k_tile_lists_direct_multi(const A_tile_lists_direct<T> *__restrict__ a) {
+  const A_tile_lists_direct<T> &A = a[blockIdx.z];
+  d_tile_lists_direct<T, const SpreadGeom &>(A.act, A.np, A.G, A.dx, A.Y, A.F, A.Tq, A.origin, A.slab, A.tcnt, A.tovf, A.pool, A.pool_top);
 }
 
 // Gaussian weights of one segment at a tile's axis points. Point a: x
@@ -1704,11 +1857,14 @@ template <typename T, int NGD, typename SG = SpreadGeom>
 __device__ __forceinline__ void d_interp_sum(const int *__restrict__ act, int np, SG G,
                              double dx3, const int *__restrict__ origin,
                              const T *__restrict__ part,
-                             double *__restrict__ V, double *__restrict__ W) {
+                             double *__restrict__ V, double *__restrict__ W,
+                             int *__restrict__ pool_top) {
   constexpr int SX = stencil_tiles(NGD, 8), SZ = stencil_tiles(NGD, 16);
   constexpr int NSLOT = kInterpSlots<NGD>;
   if (act && !*act) return;  // batched sweep: suspension converged
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  // lists without bins: the pool's counter for the next solve
+  if (pool_top && e == 0) *pool_top = 0;
   const int s = e / 6, m = e - 6 * s;
   if (s >= np) return;
   const int ox = origin[3 * s], oy = origin[3 * s + 1], oz = origin[3 * s + 2];
@@ -1746,8 +1902,9 @@ template <typename T, int NGD>
 __global__ void k_interp_sum(const int *__restrict__ act, int np, SpreadGeom G,
                              double dx3, const int *__restrict__ origin,
                              const T *__restrict__ part,
-                             double *__restrict__ V, double *__restrict__ W) {
-  d_interp_sum<T, NGD>(act, np, G, dx3, origin, part, V, W);
+                             double *__restrict__ V, double *__restrict__ W,
+                             int *__restrict__ pool_top) {
+  d_interp_sum<T, NGD>(act, np, G, dx3, origin, part, V, W, pool_top);
 }
 // arguments of one suspension for k_interp_sum_multi
 template <typename T, int NGD>
@@ -1760,13 +1917,14 @@ struct A_interp_sum {
   const T *part;
   double *V;
   double *W;
+  int *pool_top;
 };
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
 template <typename T, int NGD>
 __global__ void k_interp_sum_multi(const A_interp_sum<T, NGD> *__restrict__ a) {
   const A_interp_sum<T, NGD> &A = a[blockIdx.z];
-  d_interp_sum<T, NGD, const SpreadGeom &>(A.act, A.np, A.G, A.dx3, A.origin, A.part, A.V, A.W);
+  d_interp_sum<T, NGD, const SpreadGeom &>(A.act, A.np, A.G, A.dx3, A.origin, A.part, A.V, A.W, A.pool_top);
 }
 
 // ---------------------------------------------------------------------
@@ -1947,42 +2105,52 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   };
   mark(0);
   kmark(0);
-  // bin counting sort. Up to kScanOneMax bins the counts are scanned by one
-  // workgroup that also zeroes them (and the pool counter after them) for
-  // the next solve: they start zeroed (set_geometry) and every solve leaves
-  // them so, so no fill pass is needed.
-  const bool scan_one = nbins <= kScanOneMax;
-  if (!scan_one)
-    hipLaunchKernelGGL(k_fill_int, dim3(ceil_div(nbins + 1, 256)), dim3(256), 0, st,
-                       act, bin_count.as<int>(), nbins + 1, 0);
-  if (!mfma_spread)  // the matrix-core kernels form their weights per tile
-    hipLaunchKernelGGL(k_prepare_tab<T>, dim3(ceil_div((long)np * 3 * p.ngd, 256)),
-                       dim3(256), 0, st, act, np, Y, g, tab.as<T>());
-  hipLaunchKernelGGL(k_prepare<T>, dim3(ceil_div(np, 64)), dim3(64), 0, st, act, np,
-                     Y, F, Tq, g, geom.tx, geom.ty, geom.tz, geom.nbx, geom.nby,
-                     geom.nbz, origin.as<int>(), coef.as<T>(), bin.as<int>(),
-                     bin_count.as<int>(), slot.as<int>());
-  if (scan_one)
-    FS_TRY(device_scan_one(act, bin_count.as<int>(), nbins, bin_start.as<int>(), 1, st));
-  else
-    FS_TRY(device_scan(bin_count.as<int>(), nbins, bin_start.as<int>(),
-                       scan_tmp.as<int>(), st));
-  hipLaunchKernelGGL(k_scatter, dim3(ceil_div(np, 256)), dim3(256), 0, st, np,
-                     bin.as<int>(), slot.as<int>(), bin_start.as<int>(),
-                     ids.as<int>());
-  hipLaunchKernelGGL(k_sort_bins<T>, dim3(ceil_div(nbins, 64)), dim3(64), 0, st,
-                     act, nbins, bin_start.as<int>(), ids.as<int>(),
-                     (const int *)origin.as<int>(), Y, F, Tq, p.dx, p.ngd / 2,
-                     mfma_spread ? srec.as<SegRec<T>>() : (SegRec<T> *)nullptr,
-                     mfma_spread ? sorg.as<int>() : (int *)nullptr);
   const int ntiles = nbins;
-  kmark(1);
-  if (mfma_spread)
-    hipLaunchKernelGGL(k_tile_lists<T>, dim3(ceil_div(ntiles, 4)), dim3(256), 0, st,
-                       act, geom, bin_start.as<int>(), (const int *)sorg.as<int>(),
-                       srec.as<SegRec<T>>(),
-                       tslab.as<SegRec<T>>(), tcnt.as<int>(), tovf.as<int>(),
-                       tpool.as<SegRec<T>>(), bin_count.as<int>() + nbins);
+  if (direct) {
+    kmark(1);
+    hipLaunchKernelGGL(k_tile_lists_direct<T>, dim3(geom.nby * geom.nbz),
+                       dim3(1024), 0, st, act, np, geom, p.dx, Y, F, Tq,
+                       origin.as<int>(), tslab.as<SegRec<T>>(), tcnt.as<int>(),
+                       tovf.as<int>(), tpool.as<SegRec<T>>(),
+                       bin_count.as<int>() + nbins);
+  } else {
+    // bin counting sort. Up to kScanOneMax bins the counts are scanned by one
+    // workgroup that also zeroes them (and the pool counter after them) for
+    // the next solve: they start zeroed (set_geometry) and every solve leaves
+    // them so, so no fill pass is needed.
+    const bool scan_one = nbins <= kScanOneMax;
+    if (!scan_one)
+      hipLaunchKernelGGL(k_fill_int, dim3(ceil_div(nbins + 1, 256)), dim3(256), 0, st,
+                         act, bin_count.as<int>(), nbins + 1, 0);
+    if (!mfma_spread)  // the matrix-core kernels form their weights per tile
+      hipLaunchKernelGGL(k_prepare_tab<T>, dim3(ceil_div((long)np * 3 * p.ngd, 256)),
+                         dim3(256), 0, st, act, np, Y, g, tab.as<T>());
+    hipLaunchKernelGGL(k_prepare<T>, dim3(ceil_div(np, 64)), dim3(64), 0, st, act, np,
+                       Y, F, Tq, g, geom.tx, geom.ty, geom.tz, geom.nbx, geom.nby,
+                       geom.nbz, origin.as<int>(),
+                       mfma_spread ? (T *)nullptr : coef.as<T>(), bin.as<int>(),
+                       bin_count.as<int>(), slot.as<int>());
+    if (scan_one)
+      FS_TRY(device_scan_one(act, bin_count.as<int>(), nbins, bin_start.as<int>(), 1, st));
+    else
+      FS_TRY(device_scan(bin_count.as<int>(), nbins, bin_start.as<int>(),
+                         scan_tmp.as<int>(), st));
+    hipLaunchKernelGGL(k_scatter, dim3(ceil_div(np, 256)), dim3(256), 0, st, np,
+                       bin.as<int>(), slot.as<int>(), bin_start.as<int>(),
+                       ids.as<int>());
+    hipLaunchKernelGGL(k_bin_order<T>, dim3(ceil_div(np, 64)), dim3(64), 0, st,
+                       act, np, bin.as<int>(), bin_start.as<int>(), ids.as<int>(),
+                       origin.as<int>(), Y, F, Tq, p.dx, p.ngd / 2,
+                       mfma_spread ? srec.as<SegRec<T>>() : (SegRec<T> *)nullptr,
+                       sorg.as<int>(), sids.as<int>());
+    kmark(1);
+    if (mfma_spread)
+      hipLaunchKernelGGL(k_tile_lists<T>, dim3(ceil_div(ntiles, 4)), dim3(256), 0, st,
+                         act, geom, bin_start.as<int>(), (const int *)sorg.as<int>(),
+                         srec.as<SegRec<T>>(),
+                         tslab.as<SegRec<T>>(), tcnt.as<int>(), tovf.as<int>(),
+                         tpool.as<SegRec<T>>(), bin_count.as<int>() + nbins);
+  }
   mark(1);
   if (mfma_spread) kmark(2);
   bool okz = true;
@@ -1995,7 +2163,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
       constexpr int TZ = decltype(z)::value;
       hipLaunchKernelGGL((k_spread<T, TZ>), dim3(ntiles), dim3(geom.tx * geom.ty),
                          0, st, act, geom, tab.as<T>(), origin.as<int>(), coef.as<T>(),
-                         bin_start.as<int>(), ids.as<int>(), R.as<T>());
+                         bin_start.as<int>(), sids.as<int>(), R.as<T>());
     });
   FS_CHECK(okz, FS_ERR_ARG, "spread dispatch failed");
   FS_LAUNCHED();
@@ -2067,12 +2235,13 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
       kmark(9);
       hipLaunchKernelGGL((k_interp_sum<T, NG>), dim3(ceil_div(6L * np, 256)),
                          dim3(256), 0, st, act, np, geom, dx3,
-                         origin.as<int>(), ipart.as<T>(), V, W);
+                         origin.as<int>(), ipart.as<T>(), V, W,
+                         direct ? bin_count.as<int>() + nbins : (int *)nullptr);
     } else {
       hipLaunchKernelGGL((k_interp<T, NG>),
                          dim3(8 * ceil_div(ceil_div(np, 4), 8)), dim3(256), 0,
                          st, act, np, geom, dx3, tab.as<T>(), origin.as<int>(),
-                         ids.as<int>(), R.as<T>(), V, W);
+                         sids.as<int>(), R.as<T>(), V, W);
     }
   });
   FS_CHECK(okn, FS_ERR_ARG, "interp dispatch failed");
@@ -2163,65 +2332,80 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
   const GaussConst g = gauss_const(p);
   const ProjConst pc = proj_const(p);
   const double dx3 = p.dx * p.dx * p.dx;
-  {
-    auto t = table([&](const FcmGroupMember &m) {
-      return A_fill_int{m.act, m.fcm->bin_count.as<int>(), nbins + 1, 0};
-    });
-    if (!host)
-      hipLaunchKernelGGL(k_fill_int_multi, dim3(ceil_div(nbins + 1, 256), 1, S),
-                         dim3(256), 0, st, (const A_fill_int *)t);
-  }
-  {
+  if (f0.direct) {
     auto t = table([&](const FcmGroupMember &m) {
       const FcmImpl &f = *m.fcm;
-      return A_prepare<T>{m.act, m.np, m.Y, m.F, m.T, g, f.geom.tx, f.geom.ty,
-                          f.geom.tz, f.geom.nbx, f.geom.nby, f.geom.nbz,
-                          f.origin.as<int>(), f.coef.as<T>(), f.bin.as<int>(),
-                          f.bin_count.as<int>(), f.slot.as<int>()};
+      return A_tile_lists_direct<T>{
+          m.act, m.np, f.geom, p.dx, m.Y, m.F, m.T, f.origin.as<int>(),
+          f.tslab.as<SegRec<T>>(), f.tcnt.as<int>(), f.tovf.as<int>(),
+          f.tpool.as<SegRec<T>>(), f.bin_count.as<int>() + nbins};
     });
     if (!host)
-      hipLaunchKernelGGL(k_prepare_multi<T>, dim3(ceil_div(npmax, 64), 1, S),
-                         dim3(64), 0, st, (const A_prepare<T> *)t);
-  }
-  {
-    auto t = table([&](const FcmGroupMember &m) {
-      return A_scan_small{m.act, m.fcm->bin_count.as<int>(), nbins,
-                          m.fcm->bin_start.as<int>()};
-    });
-    if (!host)
-      hipLaunchKernelGGL(k_scan_small_multi, dim3(1, 1, S), dim3(1024), 0, st,
-                         (const A_scan_small *)t);
-  }
-  {
-    auto t = table([&](const FcmGroupMember &m) {
-      const FcmImpl &f = *m.fcm;
-      return A_scatter{m.np, f.bin.as<int>(), f.slot.as<int>(),
-                       f.bin_start.as<int>(), f.ids.as<int>()};
-    });
-    if (!host)
-      hipLaunchKernelGGL(k_scatter_multi, dim3(ceil_div(npmax, 256), 1, S),
-                         dim3(256), 0, st, (const A_scatter *)t);
-  }
-  {
-    auto t = table([&](const FcmGroupMember &m) {
-      const FcmImpl &f = *m.fcm;
-      return A_sort_bins<T>{m.act, nbins, f.bin_start.as<int>(), f.ids.as<int>(),
-                            f.origin.as<int>(), m.Y, m.F, m.T, p.dx, p.ngd / 2,
-                            f.srec.as<SegRec<T>>(), f.sorg.as<int>()};
-    });
-    if (!host)
-      hipLaunchKernelGGL(k_sort_bins_multi<T>, dim3(ceil_div(nbins, 64), 1, S),
-                         dim3(64), 0, st, (const A_sort_bins<T> *)t);
-    auto t2 = table([&](const FcmGroupMember &m) {
-      const FcmImpl &f = *m.fcm;
-      return A_tile_lists<T>{m.act, f.geom, f.bin_start.as<int>(), f.sorg.as<int>(),
-                             f.srec.as<SegRec<T>>(), f.tslab.as<SegRec<T>>(),
-                             f.tcnt.as<int>(), f.tovf.as<int>(),
-                             f.tpool.as<SegRec<T>>(), f.bin_count.as<int>() + nbins};
-    });
-    if (!host)
-      hipLaunchKernelGGL(k_tile_lists_multi<T>, dim3(ceil_div(ntiles, 4), 1, S),
-                         dim3(256), 0, st, (const A_tile_lists<T> *)t2);
+      hipLaunchKernelGGL(k_tile_lists_direct_multi<T>,
+                         dim3(f0.geom.nby * f0.geom.nbz, 1, S), dim3(1024), 0, st,
+                         (const A_tile_lists_direct<T> *)t);
+  } else {
+    {
+      auto t = table([&](const FcmGroupMember &m) {
+        return A_fill_int{m.act, m.fcm->bin_count.as<int>(), nbins + 1, 0};
+      });
+      if (!host)
+        hipLaunchKernelGGL(k_fill_int_multi, dim3(ceil_div(nbins + 1, 256), 1, S),
+                           dim3(256), 0, st, (const A_fill_int *)t);
+    }
+    {
+      auto t = table([&](const FcmGroupMember &m) {
+        const FcmImpl &f = *m.fcm;
+        return A_prepare<T>{m.act, m.np, m.Y, m.F, m.T, g, f.geom.tx, f.geom.ty,
+                            f.geom.tz, f.geom.nbx, f.geom.nby, f.geom.nbz,
+                            f.origin.as<int>(), nullptr, f.bin.as<int>(),
+                            f.bin_count.as<int>(), f.slot.as<int>()};
+      });
+      if (!host)
+        hipLaunchKernelGGL(k_prepare_multi<T>, dim3(ceil_div(npmax, 64), 1, S),
+                           dim3(64), 0, st, (const A_prepare<T> *)t);
+    }
+    {
+      auto t = table([&](const FcmGroupMember &m) {
+        return A_scan_small{m.act, m.fcm->bin_count.as<int>(), nbins,
+                            m.fcm->bin_start.as<int>()};
+      });
+      if (!host)
+        hipLaunchKernelGGL(k_scan_small_multi, dim3(1, 1, S), dim3(1024), 0, st,
+                           (const A_scan_small *)t);
+    }
+    {
+      auto t = table([&](const FcmGroupMember &m) {
+        const FcmImpl &f = *m.fcm;
+        return A_scatter{m.np, f.bin.as<int>(), f.slot.as<int>(),
+                         f.bin_start.as<int>(), f.ids.as<int>()};
+      });
+      if (!host)
+        hipLaunchKernelGGL(k_scatter_multi, dim3(ceil_div(npmax, 256), 1, S),
+                           dim3(256), 0, st, (const A_scatter *)t);
+    }
+    {
+      auto t = table([&](const FcmGroupMember &m) {
+        const FcmImpl &f = *m.fcm;
+        return A_bin_order<T>{m.act, m.np, f.bin.as<int>(), f.bin_start.as<int>(),
+                              f.ids.as<int>(), f.origin.as<int>(), m.Y, m.F, m.T,
+                              p.dx, p.ngd / 2, f.srec.as<SegRec<T>>(),
+                              f.sorg.as<int>()};
+      });
+      if (!host)
+        hipLaunchKernelGGL(k_bin_order_multi<T>, dim3(ceil_div(npmax, 64), 1, S),
+                           dim3(64), 0, st, (const A_bin_order<T> *)t);
+      auto t2 = table([&](const FcmGroupMember &m) {
+        const FcmImpl &f = *m.fcm;
+        return A_tile_lists<T>{m.act, f.geom, f.bin_start.as<int>(), f.sorg.as<int>(),
+                               f.srec.as<SegRec<T>>(), f.tslab.as<SegRec<T>>(),
+                               f.tcnt.as<int>(), f.tovf.as<int>(),
+                               f.tpool.as<SegRec<T>>(), f.bin_count.as<int>() + nbins};
+      });
+      if (!host)
+        hipLaunchKernelGGL(k_tile_lists_multi<T>, dim3(ceil_div(ntiles, 4), 1, S),
+                           dim3(256), 0, st, (const A_tile_lists<T> *)t2);
+    }
   }
   {
     auto t = table([&](const FcmGroupMember &m) {
@@ -2309,7 +2493,9 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
     auto t2 = table([&](const FcmGroupMember &m) {
       const FcmImpl &f = *m.fcm;
       return A_interp_sum<T, NG>{m.act, m.np, f.geom, dx3, f.origin.as<int>(),
-                                 f.ipart.as<T>(), m.V, m.W};
+                                 f.ipart.as<T>(), m.V, m.W,
+                                 f.direct ? f.bin_count.as<int>() + nbins
+                                          : (int *)nullptr};
     });
     if (!host)
       hipLaunchKernelGGL((k_interp_sum_multi<T, NG>),

@@ -1,0 +1,63 @@
+"""Tile lists formed straight from the segments and through bins."""
+import numpy as np
+import pytest
+
+from filsim_amd import abi, api, params
+from helpers import random_segments, rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("grid,n,spread", [
+    ((16, 16, 32), 1, 1.0),       # one row of tiles wide, one segment
+    ((24, 16, 32), 63, 0.05),     # more than a tile's slab in few tiles
+    ((64, 32, 48), 1023, 1.0),    # one segment short of a step
+    ((64, 32, 48), 1025, 0.02),   # all in one row of tiles: long pool blocks
+    ((144, 24, 32), 300, 1.0),    # 18 tiles a row: two wavefronts take two
+    ((32, 40, 48), 4096, 1.0),    # most segments of the way without bins
+    ((32, 40, 48), 4097, 1.0),    # fewest of the way through bins
+    ((32, 40, 48), 5000, 0.02),   # crowded bins
+    ((128, 128, 128), 2500, 0.3),  # rows times steps below the line
+    ((320, 320, 320), 2500, 1.0),  # above it
+])
+def test_lists_match_vector_path(cuda, grid, n, spread):
+    """Against the solver's vector path, which has no tile lists. FP64, other
+    summation orders: 1e-12, the solver's parity bar, of |V| and of the larger
+    of |W| and |V| / a. Three solves: the second must not see what the first
+    left in the lists' pool, and segments that moved must change lists."""
+    fp = params.fcm_params(grid)
+    Y, F, T = random_segments(fp, n, seed=n + grid[0])
+    Y *= spread
+    shift = np.array(params.box(fp)) * 0.47
+    with api.Fcm(fp, n) as fcm, api.Fcm(fp, n) as vec:
+        vec.set_tuning(spread_mfma=0)
+        for k in range(3):
+            Yk = np.mod(Y + k * shift, params.box(fp))
+            V, W = fcm.mobility_host(Yk, F, T)
+            Vo, Wo = vec.mobility_host(Yk, F, T)
+            top = max(np.linalg.norm(Wo), np.linalg.norm(Vo) / fp.a)
+            assert rel(V, Vo) <= 1e-12, k
+            assert np.linalg.norm(W - Wo) <= 1e-12 * top, k
+
+
+def test_binned_groups_equal_unbatched(cuda):
+    """Two suspensions of more segments than the way without bins takes,
+    stepped with fused stages and one after another: the same bits."""
+    solo, bat = [], []
+    for seed in (1, 2):
+        fp, sp, nws, props, st, info = params.sweep_point(
+            seed, grids=(160,), nfil_range=(260, 270), nw_range=(18, 20),
+            precision=abi.FS_FP32, tol=1e-4, dt=0.01)
+        assert info["segments"] > 4096
+        for group in (solo, bat):
+            s = api.System(sp, nws, props)
+            s.set_state(**st)
+            group.append(s)
+    batch = api.Batch(bat)
+    batch.set_fused(True)
+    assert batch.timestep(1) == [s.timestep(1) for s in solo]
+    for a, b in zip(solo, bat):
+        sa, sb = a.get_state(), b.get_state()
+        for k in ("X", "U", "q", "lam"):
+            assert np.array_equal(sa[k], sb[k]), k
+    batch.close()
