@@ -80,21 +80,18 @@ __global__ void k_cb_scatter(int np, const int *__restrict__ cell,
   ids[start[cell[s]] + slot[s]] = s;
 }
 
-// Descending order inside each cell = LIFO chain order of the reference.
-__global__ void k_cb_sort(int ncell, const int *__restrict__ start,
-                          int *__restrict__ ids) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  int lo = start[c], hi = start[c + 1];
-  for (int i = lo + 1; i < hi; ++i) {
-    int v = ids[i];
-    int j = i - 1;
-    while (j >= lo && ids[j] < v) {
-      ids[j + 1] = ids[j];
-      --j;
-    }
-    ids[j + 1] = v;
-  }
+// Descending order inside each cell = LIFO chain order of the reference: a
+// thread per segment counts the larger ids of its cell in ids (any order) and
+// writes its own to that place of list.
+__global__ void k_cb_order(int np, const int *__restrict__ cell,
+                           const int *__restrict__ start,
+                           const int *__restrict__ ids, int *__restrict__ list) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= np) return;
+  const int c = cell[s], lo = start[c], hi = start[c + 1];
+  int pos = lo;
+  for (int e = lo; e < hi; ++e) pos += ids[e] > s;
+  list[pos] = s;
 }
 
 // Pair mask of the barrier variants: apply_collision_barrier_not_swimmer
@@ -120,9 +117,11 @@ __device__ __forceinline__ bool cb_pair(const double *yi, const double *yj,
   f[0] = f[1] = f[2] = 0.0;
   if (!(!(jfil == ifil && abs(jseg - iseg) == 1) || c.nt < c.ifs)) return false;
   double xij = yi[0] - yj[0], yij = yi[1] - yj[1], zij = yi[2] - yj[2];
-  xij = xij - c.Lx * floor(xij / c.Lx + 0.5);
-  yij = yij - c.Ly * floor(yij / c.Ly + 0.5);
-  zij = zij - c.Lz * floor(zij / c.Lz + 0.5);
+  // up to 0.49 L the quotient's floor is 0 and the image is the value itself:
+  // the division is for pairs across the box's faces
+  if (fabs(xij) > 0.49 * c.Lx) xij = xij - c.Lx * floor(xij / c.Lx + 0.5);
+  if (fabs(yij) > 0.49 * c.Ly) yij = yij - c.Ly * floor(yij / c.Ly + 0.5);
+  if (fabs(zij) > 0.49 * c.Lz) zij = zij - c.Lz * floor(zij / c.Lz + 0.5);
   double rijsq = xij * xij + yij * yij + zij * zij;
   rsq = rijsq;
   if (rijsq < c.chiRnm2) {
@@ -145,19 +144,44 @@ __device__ __forceinline__ bool cb_pair(const double *yi, const double *yj,
   return true;
 }
 
+// v in [-1, m]
 __device__ __forceinline__ int cb_wrap(int v, int m) {
-  v %= m;
-  return v < 0 ? v + m : v;
+  return v < 0 ? v + m : (v >= m ? v - m : v);
+}
+
+// The list entries of three cells next to each other along x around cx (cells
+// are numbered along x first, so they are one range, or two where the box
+// wraps): lo first entry and na entries of the one, lo2 first entry of the
+// other, n entries of both.
+struct CbRow {
+  int lo, na, lo2, n;
+};
+__device__ __forceinline__ CbRow cb_row(const CbGeom &g, int cx, int cy, int cz,
+                                        int k, const int *__restrict__ start) {
+  const int *row = start + g.MX * (cb_wrap(cy + k % 3 - 1, g.MY) +
+                                   g.MY * cb_wrap(cz + k / 3 - 1, g.MZ));
+  const bool first = cx == 0, last = cx == g.MX - 1;
+  const int a0 = first ? g.MX - 1 : cx - 1, a1 = first || last ? g.MX : cx + 2;
+  CbRow r;
+  r.lo = row[a0];
+  r.na = row[a1] - r.lo;
+  r.lo2 = 0;
+  r.n = r.na;
+  if (first || last) {
+    r.lo2 = row[0];
+    r.n += row[first ? 2 : 1] - r.lo2;
+  }
+  return r;
 }
 
 // mode 0: F[i] += sum of pair forces, min distance; mode 1: count pairs
 // (i<j) inside the cutoff into *npairs and write them when room.
-// kCbLanes lanes per segment split its 27 cells (lane q: cells q,
-// q + kCbLanes, ..., in the reference's dz, dy, dx order) and combine their
-// partial forces pairwise by xor distance 1, 2 (deterministic); more
-// wavefronts in flight for the dependent cell/id/position loads than one
-// thread per segment.
-constexpr int kCbLanes = 4;
+// Bound by the latency of dependent loads (row starts, id, position): the
+// kCbLanes lanes of a segment look up its 9 rows of three cells together, lay
+// their entries end to end and take every kCbLanes-th each, so the usual
+// segment (10 entries) needs two rounds of loads. Partial forces are combined
+// pairwise by xor distance 1, 2, 4 (deterministic).
+constexpr int kCbLanes = 8;
 
 __global__ void __launch_bounds__(256)
     k_cb_apply(const int *__restrict__ act, int np,
@@ -169,56 +193,66 @@ __global__ void __launch_bounds__(256)
                int *__restrict__ npairs, int max_pairs,
                int *__restrict__ pairs) {
   if (act && !*act) return;  // batched sweep: suspension converged
-  __shared__ double s_min[256];
+  __shared__ double s_min[4];
   const int gt = blockIdx.x * blockDim.x + threadIdx.x;
   const int i = gt / kCbLanes, q = gt % kCbLanes;
   double mymin = 100000.0;
   double fx = 0, fy = 0, fz = 0;
+  double yi[3] = {0, 0, 0};
+  int ifil = 0, iseg = 0;
+  CbRow r = {0, 0, 0, 0}, r8 = {0, 0, 0, 0};  // row q, row 8 (every lane)
   if (i < np) {
-    const double yi[3] = {Y[3 * i], Y[3 * i + 1], Y[3 * i + 2]};
-    const int ifil = sfil[i], iseg = sseg[i];
+    for (int d = 0; d < 3; ++d) yi[d] = Y[3 * i + d];
+    ifil = sfil[i];
+    iseg = sseg[i];
     const int ci = cell[i];
     const int cx = ci % g.MX, cy = (ci / g.MX) % g.MY, cz = ci / (g.MX * g.MY);
-    // the lane's cell ranges first, all loads in flight together (most
-    // cells are empty), then the pairs in the same cell order
-    constexpr int kCells = (27 + kCbLanes - 1) / kCbLanes;
-    int lo[kCells], hi[kCells];
+    r = cb_row(g, cx, cy, cz, q, start);
+    r8 = cb_row(g, cx, cy, cz, 8, start);
+  }
+  int incl = r.n;  // entries of rows 0 .. q
 #pragma unroll
-    for (int t = 0; t < kCells; ++t) {
-      const int k = q + kCbLanes * t;
-      lo[t] = hi[t] = 0;
-      if (k < 27) {
-        const int dz = k / 9 - 1, dy = (k / 3) % 3 - 1, dx = k % 3 - 1;
-        const int nc = cb_wrap(cx + dx, g.MX) +
-                       g.MX * (cb_wrap(cy + dy, g.MY) + g.MY * cb_wrap(cz + dz, g.MZ));
-        lo[t] = start[nc];
-        hi[t] = start[nc + 1];
-      }
+  for (int off = 1; off < kCbLanes; off <<= 1) {
+    const int t = __shfl_up(incl, off, kCbLanes);
+    if (q >= off) incl += t;
+  }
+  const int pre = incl - r.n;
+  int before[kCbLanes];  // entries before each row
+#pragma unroll
+  for (int w = 1; w < kCbLanes; ++w) before[w] = __shfl(pre, w, kCbLanes);
+  const int n8 = __shfl(incl, kCbLanes - 1, kCbLanes), n = n8 + r8.n;
+  // whole wavefronts go round: the shuffles read every lane
+  for (int k0 = 0; __any(k0 < n); k0 += kCbLanes) {
+    const int k = k0 + q;
+    int w = 0;
+#pragma unroll
+    for (int v = 1; v < kCbLanes; ++v) w += before[v] <= k;
+    int lo = __shfl(r.lo, w, kCbLanes), na = __shfl(r.na, w, kCbLanes),
+        lo2 = __shfl(r.lo2, w, kCbLanes), o = k - __shfl(pre, w, kCbLanes);
+    if (k >= n8) {
+      lo = r8.lo;
+      na = r8.na;
+      lo2 = r8.lo2;
+      o = k - n8;
     }
-#pragma unroll
-    for (int t = 0; t < kCells; ++t) {
-      for (int e = lo[t]; e < hi[t]; ++e) {
-        int j = ids[e];
-        if (j == i) continue;
-        const int jfil = sfil[j];
-        if (!cb_mask_in(c, i, j, ifil, jfil)) continue;
-        double yj[3] = {Y[3 * j], Y[3 * j + 1], Y[3 * j + 2]};
-        double rsq, f[3];
-        if (!cb_pair(yi, yj, ifil, iseg, jfil, sseg[j], c, rsq, f))
-          continue;
-        mymin = fmin(mymin, rsq);
-        if (rsq < c.chiRnm2) {
-          if (mode == 0) {
-            fx += f[0];
-            fy += f[1];
-            fz += f[2];
-          } else if (i < j) {
-            int kk = atomicAdd(npairs, 1);
-            if (kk < max_pairs) {
-              pairs[2 * kk] = i;
-              pairs[2 * kk + 1] = j;
-            }
-          }
+    if (k >= n) continue;
+    const int j = ids[o < na ? lo + o : lo2 + o - na];
+    const int jfil = sfil[j], jseg = sseg[j];
+    const double yj[3] = {Y[3 * j], Y[3 * j + 1], Y[3 * j + 2]};
+    if (j == i || !cb_mask_in(c, i, j, ifil, jfil)) continue;
+    double rsq, f[3];
+    if (!cb_pair(yi, yj, ifil, iseg, jfil, jseg, c, rsq, f)) continue;
+    mymin = fmin(mymin, rsq);
+    if (rsq < c.chiRnm2) {
+      if (mode == 0) {
+        fx += f[0];
+        fy += f[1];
+        fz += f[2];
+      } else if (i < j) {
+        int kk = atomicAdd(npairs, 1);
+        if (kk < max_pairs) {
+          pairs[2 * kk] = i;
+          pairs[2 * kk + 1] = j;
         }
       }
     }
@@ -235,16 +269,18 @@ __global__ void __launch_bounds__(256)
     F[3 * i + 1] += fy;
     F[3 * i + 2] += fz;
   }
-  s_min[threadIdx.x] = mymin;
+  if (mode != 0) return;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) mymin = fmin(mymin, __shfl_xor(mymin, m, 64));
+  if ((threadIdx.x & 63) == 0) s_min[threadIdx.x >> 6] = mymin;
   __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off)
-      s_min[threadIdx.x] = fmin(s_min[threadIdx.x], s_min[threadIdx.x + off]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0 && mode == 0) {
-    // positive doubles order like their bit patterns
-    atomicMin(min_bits, (unsigned long long)__double_as_longlong(s_min[0]));
+  if (threadIdx.x == 0) {
+    // positive doubles order like their bit patterns. A value read before can
+    // only be too large, so what it already undercuts needs no atomic.
+    const unsigned long long b = (unsigned long long)__double_as_longlong(
+        fmin(fmin(s_min[0], s_min[1]), fmin(s_min[2], s_min[3])));
+    if (b < __hip_atomic_load(min_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMin(min_bits, b);
   }
 }
 
@@ -288,7 +324,9 @@ int ColbarImpl::init(const fs_colbar_params &pp, int n, const int *seg_fil,
   FS_TRY(cell.alloc(sizeof(int) * std::max(n, 1)));
   FS_TRY(slot.alloc(sizeof(int) * std::max(n, 1)));
   FS_TRY(ids.alloc(sizeof(int) * std::max(n, 1)));
-  FS_TRY(cnt.alloc(sizeof(int) * ncell));
+  FS_TRY(cnt.alloc(sizeof(int) * (ncell + 1)));
+  // counts start zeroed and every link leaves them so
+  FS_HIP(hipMemset(cnt.p, 0, sizeof(int) * (ncell + 1)));
   FS_TRY(start.alloc(sizeof(int) * (ncell + 1)));
   FS_TRY(scan_tmp.alloc(sizeof(int) * (ncell / kScanBlock + 4)));
   FS_TRY(sfil.alloc(sizeof(int) * std::max(n, 1)));
@@ -316,19 +354,19 @@ void ColbarImpl::release() {
 
 int ColbarImpl::link(const double *Xs, hipStream_t st) {
   FS_CHECK(np == 0 || Xs, FS_ERR_ARG, "null Xs");
-  hipLaunchKernelGGL(k_cb_fill, dim3(ceil_div(ncell, 256)), dim3(256), 0, st,
-                     cnt.as<int>(), ncell, 0);
   if (np > 0)
     hipLaunchKernelGGL(k_cb_bin, dim3(ceil_div(np, 256)), dim3(256), 0, st, np,
                        Xs, g, cell.as<int>(), cnt.as<int>(), slot.as<int>());
   FS_TRY(device_scan(cnt.as<int>(), ncell, start.as<int>(),
-                     scan_tmp.as<int>(), st));
+                     scan_tmp.as<int>(), 1, st));
   if (np > 0)
     hipLaunchKernelGGL(k_cb_scatter, dim3(ceil_div(np, 256)), dim3(256), 0, st,
                        np, cell.as<int>(), slot.as<int>(), start.as<int>(),
                        ids.as<int>());
-  hipLaunchKernelGGL(k_cb_sort, dim3(ceil_div(ncell, 256)), dim3(256), 0, st,
-                     ncell, start.as<int>(), ids.as<int>());
+  if (np > 0)
+    hipLaunchKernelGGL(k_cb_order, dim3(ceil_div(np, 256)), dim3(256), 0, st, np,
+                       cell.as<int>(), start.as<int>(), ids.as<int>(),
+                       slot.as<int>());
   FS_LAUNCHED();
   linked = true;
   return FS_OK;
@@ -364,7 +402,7 @@ int ColbarImpl::apply(const double *Y, int nt, double *F, double *min_dist2,
   if (np > 0)
     hipLaunchKernelGGL(k_cb_apply, dim3(ceil_div((long)np * kCbLanes, 256)), dim3(256), 0, st,
                        act, np, Y, g, consts(nt), cell.as<int>(), start.as<int>(),
-                       ids.as<int>(), sfil.as<int>(), sseg.as<int>(), F,
+                       slot.as<int>(), sfil.as<int>(), sseg.as<int>(), F,
                        minb.as<unsigned long long>(), 0, (int *)nullptr, 0,
                        (int *)nullptr);
   FS_LAUNCHED();
@@ -384,7 +422,7 @@ int ColbarImpl::get_lists(int *head, int *list) {
   FS_HIP(hipMemcpy(hs.data(), start.p, sizeof(int) * (ncell + 1),
                    hipMemcpyDeviceToHost));
   if (np > 0)
-    FS_HIP(hipMemcpy(hid.data(), ids.p, sizeof(int) * np, hipMemcpyDeviceToHost));
+    FS_HIP(hipMemcpy(hid.data(), slot.p, sizeof(int) * np, hipMemcpyDeviceToHost));
   for (int c = 0; c < ncell; ++c) {
     head[c] = (hs[c] < hs[c + 1]) ? hid[hs[c]] : -1;
     for (int e = hs[c]; e < hs[c + 1]; ++e)
@@ -406,7 +444,7 @@ int ColbarImpl::pairs(const double *Y, int nt, int max_pairs, int *out,
     hipLaunchKernelGGL(k_cb_apply, dim3(ceil_div((long)np * kCbLanes, 256)), dim3(256), 0, 0,
                        (const int *)nullptr, np,
                        Y, g, consts(nt), cell.as<int>(), start.as<int>(),
-                       ids.as<int>(), sfil.as<int>(), sseg.as<int>(),
+                       slot.as<int>(), sfil.as<int>(), sseg.as<int>(),
                        (double *)nullptr, (unsigned long long *)nullptr, 1, dn,
                        max_pairs, dp);
   FS_LAUNCHED();
@@ -530,12 +568,13 @@ int colbar_barrier_noalloc(const fs_colbar_params *pp, int np,
   if (np > 0)
     hipLaunchKernelGGL(k_cb_bin, dim3(ceil_div(np, 256)), dim3(256), 0, st, np,
                        Xs, cb.g, cell, cnt, slot);
-  FS_TRY(device_scan(cnt, cb.ncell, start, scan, st));
+  FS_TRY(device_scan(cnt, cb.ncell, start, scan, 0, st));
   if (np > 0)
     hipLaunchKernelGGL(k_cb_scatter, dim3(ceil_div(np, 256)), dim3(256), 0, st,
                        np, cell, slot, start, ids);
-  hipLaunchKernelGGL(k_cb_sort, dim3(ceil_div(cb.ncell, 256)), dim3(256), 0,
-                     st, cb.ncell, start, ids);
+  if (np > 0)  // the slots are free now: the lists take their place
+    hipLaunchKernelGGL(k_cb_order, dim3(ceil_div(np, 256)), dim3(256), 0, st, np,
+                       cell, start, ids, slot);
   // apply
   double init = 100000.0;
   unsigned long long ib;
@@ -545,7 +584,7 @@ int colbar_barrier_noalloc(const fs_colbar_params *pp, int np,
   if (np > 0)
     hipLaunchKernelGGL(k_cb_apply, dim3(ceil_div((long)np * kCbLanes, 256)),
                        dim3(256), 0, st, (const int *)nullptr, np, Y, cb.g,
-                       cb.consts(nt), cell, start, ids, seg_fil, seg_idx, F,
+                       cb.consts(nt), cell, start, slot, seg_fil, seg_idx, F,
                        minb, 0, (int *)nullptr, 0, (int *)nullptr);
   if (min_dist2)
     hipLaunchKernelGGL(k_cb_store_min, dim3(1), dim3(1), 0, st, minb,

@@ -26,6 +26,7 @@ struct ColbarImpl {
   CbGeom g{};
   bool linked = false;
   int mask = FS_BARRIER_ALL;
+  // slot: a segment's place in its cell during link(), then the cells' lists
   dbuf cell, slot, ids, cnt, start, scan_tmp, sfil, sseg, minb;
 
   // cell grid and sizes only (no allocation)

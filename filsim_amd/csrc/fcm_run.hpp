@@ -143,28 +143,6 @@ __global__ void k_prepare_multi(const A_prepare<T> *__restrict__ a) {
   d_prepare<T, const GaussConst &>(A.act, A.np, A.Y, A.F, A.Tq, A.g, A.tx, A.ty, A.tz, A.nbx, A.nby, A.nbz, A.origin, A.coef, A.bin, A.bin_count, A.slot);
 }
 
-__device__ __forceinline__ void d_fill_int(const int *__restrict__ act, int *p, int n, int v) {
-  if (act && !*act) return;  // batched sweep: suspension converged
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-static __global__ void k_fill_int(const int *__restrict__ act, int *p, int n, int v) {
-  d_fill_int(act, p, n, v);
-}
-// arguments of one suspension for k_fill_int_multi
-struct A_fill_int {
-  const int *act;
-  int *p;
-  int n;
-  int v;
-};
-// one launch for a group of suspensions with equal launch shapes:
-// blockIdx.z selects the suspension
-static __global__ void k_fill_int_multi(const A_fill_int *__restrict__ a) {
-  const A_fill_int &A = a[blockIdx.z];
-  d_fill_int(A.act, A.p, A.n, A.v);
-}
-
 __device__ __forceinline__ void d_scatter(int np, const int *__restrict__ bin,
                           const int *__restrict__ slot,
                           const int *__restrict__ start, int *__restrict__ ids) {
@@ -2114,14 +2092,9 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
                        tovf.as<int>(), tpool.as<SegRec<T>>(),
                        bin_count.as<int>() + nbins);
   } else {
-    // bin counting sort. Up to kScanOneMax bins the counts are scanned by one
-    // workgroup that also zeroes them (and the pool counter after them) for
-    // the next solve: they start zeroed (set_geometry) and every solve leaves
-    // them so, so no fill pass is needed.
-    const bool scan_one = nbins <= kScanOneMax;
-    if (!scan_one)
-      hipLaunchKernelGGL(k_fill_int, dim3(ceil_div(nbins + 1, 256)), dim3(256), 0, st,
-                         act, bin_count.as<int>(), nbins + 1, 0);
+    // bin counting sort. The scan also zeroes the counts (and the pool counter
+    // after them) for the next solve: they start zeroed (set_geometry) and
+    // every solve leaves them so, so no fill pass is needed.
     if (!mfma_spread)  // the matrix-core kernels form their weights per tile
       hipLaunchKernelGGL(k_prepare_tab<T>, dim3(ceil_div((long)np * 3 * p.ngd, 256)),
                          dim3(256), 0, st, act, np, Y, g, tab.as<T>());
@@ -2130,11 +2103,11 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
                        geom.nbz, origin.as<int>(),
                        mfma_spread ? (T *)nullptr : coef.as<T>(), bin.as<int>(),
                        bin_count.as<int>(), slot.as<int>());
-    if (scan_one)
+    if (nbins <= kScanOneMax)
       FS_TRY(device_scan_one(act, bin_count.as<int>(), nbins, bin_start.as<int>(), 1, st));
     else
       FS_TRY(device_scan(bin_count.as<int>(), nbins, bin_start.as<int>(),
-                         scan_tmp.as<int>(), st));
+                         scan_tmp.as<int>(), 1, st));
     hipLaunchKernelGGL(k_scatter, dim3(ceil_div(np, 256)), dim3(256), 0, st, np,
                        bin.as<int>(), slot.as<int>(), bin_start.as<int>(),
                        ids.as<int>());
@@ -2268,9 +2241,9 @@ struct A_scan_small {
   int n;
   int *start;
 };
-// start[0..n] = exclusive scan of cnt[0..n) with one workgroup per member;
-// up to kScanOneMax bins the single-solve scan, which leaves cnt[0..n]
-// zeroed as the single-solve path expects, else 1024-element chunks with a
+// start[0..n] = exclusive scan of cnt[0..n) with one workgroup per member,
+// which leaves cnt[0..n] zeroed as the single-solve path does: up to
+// kScanOneMax bins the single-solve scan, else 1024-element chunks with a
 // running carry
 static __global__ void __launch_bounds__(1024)
     k_scan_small_multi(const A_scan_small *__restrict__ a) {
@@ -2293,11 +2266,17 @@ static __global__ void __launch_bounds__(1024)
       s[t] += v;
       __syncthreads();
     }
-    if (i < A.n) A.start[i] = carry + ((t == 0) ? 0 : s[t - 1]);
+    if (i < A.n) {
+      A.start[i] = carry + ((t == 0) ? 0 : s[t - 1]);
+      A.cnt[i] = 0;
+    }
     carry += s[1023];
     __syncthreads();  // s is rewritten by the next chunk
   }
-  if (t == 0) A.start[A.n] = carry;
+  if (t == 0) {
+    A.start[A.n] = carry;
+    A.cnt[A.n] = 0;
+  }
 }
 
 // One pass over the stages: with `host` set, appends each stage's argument
@@ -2345,14 +2324,6 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
                          dim3(f0.geom.nby * f0.geom.nbz, 1, S), dim3(1024), 0, st,
                          (const A_tile_lists_direct<T> *)t);
   } else {
-    {
-      auto t = table([&](const FcmGroupMember &m) {
-        return A_fill_int{m.act, m.fcm->bin_count.as<int>(), nbins + 1, 0};
-      });
-      if (!host)
-        hipLaunchKernelGGL(k_fill_int_multi, dim3(ceil_div(nbins + 1, 256), 1, S),
-                           dim3(256), 0, st, (const A_fill_int *)t);
-    }
     {
       auto t = table([&](const FcmGroupMember &m) {
         const FcmImpl &f = *m.fcm;

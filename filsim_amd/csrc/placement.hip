@@ -356,7 +356,7 @@ extern "C" int fs_make_filaments_gpu(const double box[3], int nfil,
                          st, placed, pts.as<double>(), G, cell.as<int>(),
                          cnt.as<int>(), slot.as<int>());
       FS_TRY(device_scan(cnt.as<int>(), (int)ncell, start.as<int>(),
-                         tmp.as<int>(), st));
+                         tmp.as<int>(), 0, st));
       hipLaunchKernelGGL(k_pl_scatter, dim3(ceil_div(placed, 256)), dim3(256),
                          0, st, placed, cell.as<int>(), slot.as<int>(),
                          start.as<int>(), ids.as<int>());

@@ -1,7 +1,6 @@
 // scan.hpp -- device-wide exclusive scan of int counts (counting sorts of
-// the spread bins and the barrier cells): block sums, one-block scan of the
-// block sums, then block-local scans with the block offsets; arrays of up
-// to 16Ki counts in one workgroup instead.
+// the spread bins and the barrier cells): block sums, then block-local scans
+// with the block offsets; arrays of up to 16Ki counts in one workgroup instead.
 #pragma once
 
 #include "common.hpp"
@@ -13,20 +12,29 @@ constexpr int kScanMaxBlocks = 65536;  // up to 64Mi elements
 
 namespace {  // each including translation unit gets its own kernels
 
+// Four consecutive counts of a block (thread t of 256: lo + 4 t), zero past n.
+__device__ __forceinline__ int4 scan_load(const int *__restrict__ cnt, int i,
+                                          int n) {
+  if (i + 4 <= n) return *reinterpret_cast<const int4 *>(cnt + i);
+  return int4{i < n ? cnt[i] : 0, i + 1 < n ? cnt[i + 1] : 0,
+              i + 2 < n ? cnt[i + 2] : 0, 0};
+}
+
+// Sum of v over 256 threads, on all of them.
+__device__ __forceinline__ int scan_block_total(int v, int *wsum) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+}
+
 __global__ void __launch_bounds__(256)
     k_scan_blocksum(const int *__restrict__ cnt, int n, int *__restrict__ bsum) {
-  __shared__ int red[256];
-  const int b = blockIdx.x;
-  const int lo = b * kScanBlock;
-  int s = 0;
-  for (int i = lo + threadIdx.x; i < min(n, lo + kScanBlock); i += 256) s += cnt[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) bsum[b] = red[0];
+  __shared__ int wsum[4];
+  const int4 c = scan_load(cnt, blockIdx.x * kScanBlock + 4 * threadIdx.x, n);
+  const int s = scan_block_total(c.x + c.y + c.z + c.w, wsum);
+  if (threadIdx.x == 0) bsum[blockIdx.x] = s;
 }
 
 // Exclusive scan in place of nb block sums, 1024 at a time with a running
@@ -52,22 +60,51 @@ __global__ void __launch_bounds__(1024) k_scan_top(int *__restrict__ bsum, int n
   if (t == 0) bsum[nb] = carry;
 }
 
-__global__ void __launch_bounds__(1024)
-    k_scan_apply(const int *__restrict__ cnt, int n,
-                 const int *__restrict__ bsum, int nb, int *__restrict__ start) {
-  __shared__ int s[kScanBlock];
-  const int b = blockIdx.x, t = threadIdx.x;
-  const int i = b * kScanBlock + t;
-  s[t] = (i < n) ? cnt[i] : 0;
-  __syncthreads();
-  for (int off = 1; off < kScanBlock; off <<= 1) {
-    int v = (t >= off) ? s[t - off] : 0;
-    __syncthreads();
-    s[t] += v;
-    __syncthreads();
+// start of a block's 1,024 counts. bsum: the block sums, which the block adds
+// up to its own (exclusive == 0), or their exclusive scan. clear != 0 zeroes
+// the counts and the extra counter cnt[n] after they are read.
+__global__ void __launch_bounds__(256)
+    k_scan_apply(int *__restrict__ cnt, int n, const int *__restrict__ bsum,
+                 int exclusive, int *__restrict__ start, int clear) {
+  __shared__ int wsum[4], wpre[4];
+  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int i = b * kScanBlock + 4 * t;
+  const int4 c = scan_load(cnt, i, n);
+  int base;
+  if (exclusive) {
+    base = bsum[b];
+  } else {
+    int v = 0;
+    for (int k = t; k < b; k += 256) v += bsum[k];
+    base = scan_block_total(v, wsum);
   }
-  if (i < n) start[i] = bsum[b] + ((t == 0) ? 0 : s[t - 1]);
-  if (b == 0 && t == 0) start[n] = bsum[nb];
+  const int own = c.x + c.y + c.z + c.w;
+  int x = own;  // inclusive prefix over the wavefront
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(x, off, 64);
+    if (lane >= off) x += y;
+  }
+  if (lane == 63) wpre[w] = x;
+  __syncthreads();
+  for (int k = 0; k < w; ++k) base += wpre[k];
+  base += x - own;
+  const int4 r = {base, base + c.x, base + c.x + c.y, base + c.x + c.y + c.z};
+  if (i + 4 <= n) {
+    *reinterpret_cast<int4 *>(start + i) = r;
+    if (clear) *reinterpret_cast<int4 *>(cnt + i) = int4{0, 0, 0, 0};
+  } else {
+    const int v[4] = {r.x, r.y, r.z, r.w};
+    for (int k = 0; k < 4; ++k)
+      if (i + k < n) {
+        start[i + k] = v[k];
+        if (clear) cnt[i + k] = 0;
+      }
+  }
+  if (b == (int)gridDim.x - 1 && t == 255) {
+    start[n] = base + own;
+    if (clear) cnt[n] = 0;
+  }
 }
 
 // One-workgroup exclusive scan for short count arrays (n <= kScanOneMax):
@@ -166,17 +203,23 @@ inline int device_scan_one(const int *act, int *cnt, int n, int *start,
   return FS_OK;
 }
 
-// start[0..n] = exclusive scan of cnt[0..n); scratch: >= n/1024 + 2 ints.
-inline int device_scan(const int *cnt, int n, int *start, int *scratch,
+// start[0..n] = exclusive scan of cnt[0..n); scratch: >= n/1024 + 2 ints;
+// clear != 0 also zeroes cnt[0..n]. Up to 4Mi counts a block adds the sums
+// before its own itself (at most 16 loads a thread); above, a launch scans them
+// first, which would take 6 us of latency for any number of sums. cnt and
+// start: 16-byte aligned.
+inline int device_scan(int *cnt, int n, int *start, int *scratch, int clear,
                        hipStream_t st) {
   const int nb = (n + kScanBlock - 1) / kScanBlock;
   FS_CHECK(nb >= 1 && nb <= kScanMaxBlocks, FS_ERR_ARG,
            "scan of %d elements too large", n);
+  const int exclusive = nb > 4096;
   hipLaunchKernelGGL(k_scan_blocksum, dim3(nb), dim3(256), 0, st, cnt, n,
                      scratch);
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, st, scratch, nb);
-  hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanBlock), 0, st, cnt, n,
-                     scratch, nb, start);
+  if (exclusive)
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, st, scratch, nb);
+  hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, st, cnt, n, scratch,
+                     exclusive, start, clear);
   return FS_OK;
 }
 
