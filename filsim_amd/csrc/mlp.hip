@@ -28,6 +28,7 @@ namespace fs {
 
 typedef short s4v __attribute__((ext_vector_type(4)));
 typedef float f4v __attribute__((ext_vector_type(4)));
+typedef __bf16 b8v __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ uint16_t f2bf(float f) {  // round to nearest even
   uint32_t u = __float_as_uint(f);
@@ -54,6 +55,8 @@ enum { EPI_STORE = 0, EPI_HIDDEN = 1, EPI_OUT = 2, EPI_DRELU = 3, EPI_ADD = 4 };
 //            OUT    Cf = acc + bias
 //            DRELU  g = acc * (Zf > 0): Cf = g, Hb = BF16(g)
 //            ADD    Cf += acc
+// Bound by the latency of the loads: those of kGemmAhead steps go out together.
+constexpr int kGemmAhead = 4;
 template <bool AV, bool BV>
 __global__ void __launch_bounds__(256)
     k_gemm_bf16(int M, int N, int K, const uint16_t *__restrict__ A, long sam,
@@ -74,39 +77,49 @@ __global__ void __launch_bounds__(256)
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f4v{0.f, 0.f, 0.f, 0.f};
-  for (int s = s0; s < s1; ++s) {
-    const int k = 16 * s + kq;
-    s4v a[2], b[2];
+  for (int sb = s0; sb < s1; sb += kGemmAhead) {
+    s4v a[kGemmAhead][2], b[kGemmAhead][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int m = m0 + 16 * i + r;
-      if (AV && m < M && k + 4 <= K) {
-        a[i] = *reinterpret_cast<const s4v *>(A + (long)m * sam + k);
-      } else {
+    for (int u = 0; u < kGemmAhead; ++u) {
+      // past the wave's steps k is K: zeros
+      const int k = sb + u < s1 ? 16 * (sb + u) + kq : K;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          a[i][q] = (m < M && k + q < K) ? (short)A[(long)m * sam + (long)(k + q) * sak]
-                                         : (short)0;
+      for (int i = 0; i < 2; ++i) {
+        const int m = m0 + 16 * i + r;
+        if (AV && m < M && k + 4 <= K) {
+          a[u][i] = *reinterpret_cast<const s4v *>(A + (long)m * sam + k);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            a[u][i][q] = (m < M && k + q < K)
+                             ? (short)A[(long)m * sam + (long)(k + q) * sak]
+                             : (short)0;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int n = n0 + 16 * j + r;
+        if (BV && n < N && k + 4 <= K) {
+          b[u][j] = *reinterpret_cast<const s4v *>(B + (long)n * sbn + k);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            b[u][j][q] = (n < N && k + q < K)
+                             ? (short)B[(long)(k + q) * sbk + (long)n * sbn]
+                             : (short)0;
+        }
       }
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + 16 * j + r;
-      if (BV && n < N && k + 4 <= K) {
-        b[j] = *reinterpret_cast<const s4v *>(B + (long)n * sbn + k);
-      } else {
+    for (int u = 0; u < kGemmAhead; ++u)
+      if (sb + u < s1) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          b[j][q] = (n < N && k + q < K) ? (short)B[(long)(k + q) * sbk + (long)n * sbn]
-                                         : (short)0;
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                a[u][i], b[u][j], acc[i][j], 0, 0, 0);
       }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j],
-                                                             acc[i][j], 0, 0, 0);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -140,10 +153,173 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// ---------------------------------------------------------------------
+// The whole inference pass of 16 rows in one workgroup of 16 wavefronts:
+// normalised inputs and activations stay in LDS as BF16, the weights are read
+// from L2. Each wavefront makes 16 outputs of a layer (16 x 16 MFMA tile, all
+// of K; further tiles 16 wavefronts on). Same roundings as the layers one by
+// one (inputs, activations BF16, sums FP32, bias and skip term added in FP32).
+// Bound by the latency and the rate at which a CU reads the weights: they are
+// kept a second time in the order of the loads, 1 KB of a wavefront in one
+// piece (as stored, a load's 16 rows of 64 bytes each are looked up one by
+// one: 27 us instead of 16 us for 1,000 rows of 716-256-256-256-180 with a skip
+// map, and 46 us layer by layer). 8,000 rows 147 -> 38 us.
+// ---------------------------------------------------------------------
+constexpr int kMlpRows = 16, kMlpWaves = 16, kMlpAhead = 8;
+
+// LDS row of n BF16 values: whole steps of 32, and 16 bytes so that 16 rows
+// fall on different banks.
+__host__ __device__ constexpr int mlp_row(int n) { return (n + 31) / 32 * 32 + 8; }
+
+// Place of element (n, k) of a matrix with K columns among its tiles of 16
+// rows by 32 columns: lane l of a wavefront reads row l % 16, columns
+// 8 (l / 16) .. + 7 of a tile as 16 bytes, the tiles of 16 rows in a row.
+__host__ __device__ inline long mlp_packed(int K, int n, int k) {
+  const long tile = (long)(n >> 4) * ((K + 31) / 32) + (k >> 5);
+  return (tile * 64 + (n & 15) + 16 * ((k >> 3) & 3)) * 8 + (k & 7);
+}
+__host__ __device__ inline long mlp_packed_size(int K, int N) {
+  return (long)((N + 15) / 16) * ((K + 31) / 32) * 512;
+}
+
+// Layers of the network: offsets of W_l and b_l in the parameters, of the
+// packed W_l (l < 4) and skip map (l = 4) in packed (nullptr: not kept).
+struct MlpNet {
+  long woff[4], boff[4], poff[5];
+  int dims[5];
+  uint16_t *packed;
+};
+
+__device__ __forceinline__ void mlp_pack_param(const MlpNet &net, long i,
+                                               uint16_t v) {
+  if (!net.packed) return;
+#pragma unroll
+  for (int l = 0; l < 4; ++l)
+    if (i >= net.woff[l] && i < net.boff[l]) {
+      const uint32_t K = net.dims[l], r = (uint32_t)(i - net.woff[l]), n = r / K;
+      net.packed[net.poff[l] + mlp_packed(K, n, r - n * K)] = v;
+    }
+}
+
+__global__ void k_pack_skip(const uint16_t *__restrict__ S, MlpNet net) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int K = net.dims[0];
+  if (i >= (long)K * net.dims[4]) return;
+  const int n = (int)(i / K);
+  net.packed[net.poff[4] + mlp_packed(K, n, (int)(i - (long)n * K))] = S[i];
+}
+
+// 16 x 16 tile sum_k A[m][k] W[n][k] over the LDS rows a (stride lda) and 16
+// packed rows w of W. Lane l holds rows 4 (l / 16) + i of column l % 16.
+__device__ __forceinline__ f4v mlp_tile(const uint16_t *a, int lda,
+                                        const uint16_t *__restrict__ w, int K,
+                                        int lane) {
+  constexpr int P = kMlpAhead;
+  const int steps = (K + 31) / 32;
+  const b8v *wl = reinterpret_cast<const b8v *>(w) + lane;
+  const uint16_t *ar = a + (lane & 15) * lda + 8 * (lane >> 4);
+  f4v acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < steps; s += P) {
+    b8v v[P];  // the last step's again past the end
+#pragma unroll
+    for (int j = 0; j < P; ++j) v[j] = wl[64 * min(s + j, steps - 1)];
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+      if (s + j < steps) {
+        const b8v x = *reinterpret_cast<const b8v *>(ar + 32 * (s + j));
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, v[j], acc, 0, 0, 0);
+      }
+  }
+  return acc;
+}
+
+// P: the FP32 parameters (biases).
+__global__ void __launch_bounds__(64 * kMlpWaves)
+    k_mlp_forward(int rows, MlpNet net, int skip, const float *__restrict__ mu,
+                  const float *__restrict__ sig, const float *__restrict__ tau,
+                  const float *__restrict__ P, const float *__restrict__ X,
+                  float *__restrict__ Y) {
+  extern __shared__ __align__(16) uint16_t s_mlp[];
+  const int nin = net.dims[0], width = net.dims[1], nout = net.dims[4];
+  const int ldx = mlp_row(nin), ldh = mlp_row(width);
+  uint16_t *xn = s_mlp, *h0 = xn + kMlpRows * ldx, *h1 = h0 + kMlpRows * ldh;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r0 = blockIdx.x * kMlpRows;
+  // one wavefront a row; what pads K to whole steps is zero
+  const bool row = r0 + wave < rows;
+  for (int c = lane; c < ldx; c += 64) {
+    float v = 0.f;
+    if (row && c < nin) v = (X[(long)(r0 + wave) * nin + c] - mu[c]) / sig[c];
+    xn[wave * ldx + c] = f2bf(v);
+  }
+  for (int c = width + lane; c < ldh; c += 64)
+    h0[wave * ldh + c] = h1[wave * ldh + c] = 0;
+  __syncthreads();
+  const int n16 = lane & 15, m4 = 4 * (lane >> 4);
+  const uint16_t *a = xn;
+  int lda = ldx, K = nin;
+  for (int l = 0; l < 3; ++l) {
+    uint16_t *h = (l & 1) ? h1 : h0;
+    for (int t = wave; 16 * t < width; t += kMlpWaves) {
+      const int n = 16 * t + n16;
+      const f4v acc = mlp_tile(
+          a, lda, net.packed + net.poff[l] + mlp_packed(K, 16 * t, 0), K, lane);
+      if (n < width) {
+        const float b = P[net.boff[l] + n];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float z = acc[i] + b;
+          h[(m4 + i) * ldh + n] = f2bf(z > 0.f ? z : 0.f);
+        }
+      }
+    }
+    __syncthreads();
+    a = h;
+    lda = ldh;
+    K = width;
+  }
+  for (int t = wave; 16 * t < nout; t += kMlpWaves) {
+    const int n = 16 * t + n16;
+    const f4v acc = mlp_tile(
+        a, lda, net.packed + net.poff[3] + mlp_packed(K, 16 * t, 0), K, lane);
+    f4v sk = {0.f, 0.f, 0.f, 0.f};
+    if (skip)
+      sk = mlp_tile(xn, ldx,
+                    net.packed + net.poff[4] + mlp_packed(nin, 16 * t, 0), nin,
+                    lane);
+    if (n < nout) {
+      const float b = P[net.boff[3] + n], tn = tau[n];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float y = acc[i] + b;
+        if (skip) y += sk[i];
+        if (r0 + m4 + i < rows) Y[(long)(r0 + m4 + i) * nout + n] = y * tn;
+      }
+    }
+  }
+}
+static_assert(kMlpRows == kMlpWaves, "one wavefront normalises a row");
+
 __global__ void k_to_bf16(const float *__restrict__ x, long n,
                           uint16_t *__restrict__ y) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = f2bf(x[i]);
+}
+
+// BF16 parameters, as stored and packed
+__global__ void k_quantise(const float *__restrict__ x, long n,
+                           uint16_t *__restrict__ y, MlpNet net) {
+  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint16_t v = f2bf(x[i]);
+  y[i] = v;
+  mlp_pack_param(net, i, v);
+}
+
+// Column of element i of n elements in rows of cols: a 64-bit division only
+// where 32 bits do not hold the elements.
+__device__ __forceinline__ int column_of(long i, long n, int cols) {
+  return n <= 0xFFFFFFFFl ? (int)((uint32_t)i % (uint32_t)cols) : (int)(i % cols);
 }
 
 // x_n = BF16((x - mu) / sigma) per column
@@ -153,7 +329,7 @@ __global__ void k_normalise_in(const float *__restrict__ x, int rows, int cols,
                                uint16_t *__restrict__ y) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (long)rows * cols) return;
-  int c = (int)(i % cols);
+  const int c = column_of(i, (long)rows * cols, cols);
   y[i] = f2bf((x[i] - mu[c]) / sig[c]);
 }
 
@@ -161,7 +337,7 @@ __global__ void k_scale_out(float *__restrict__ y, int rows, int cols,
                             const float *__restrict__ tau) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (long)rows * cols) return;
-  y[i] *= tau[i % cols];
+  y[i] *= tau[column_of(i, (long)rows * cols, cols)];
 }
 
 // dL/dy_n for L = mean((y_n - t/tau)^2); partial loss sums per block.
@@ -175,7 +351,7 @@ __global__ void __launch_bounds__(256)
   const long n = (long)rows * cols;
   float l = 0.f;
   if (i < n) {
-    float d = yn[i] - t[i] / tau[i % cols];
+    float d = yn[i] - t[i] / tau[column_of(i, n, cols)];
     float gi = 2.f * d / (float)n;
     g[i] = gi;
     gb[i] = f2bf(gi);
@@ -193,7 +369,8 @@ __global__ void __launch_bounds__(256)
 // column sums (bias gradients) in a fixed order: a workgroup of 16
 // wavefronts per 64 columns, wavefront w adds the w-th contiguous sixteenth
 // of the rows (one coalesced row segment per load), then the 16 partial
-// sums are added in wavefront order
+// sums are added in wavefront order. Few workgroups, so bound by the latency
+// of the loads: 16 of them are in flight.
 __global__ void __launch_bounds__(1024)
     k_colsum(const float *__restrict__ g, int rows, int cols,
              float *__restrict__ out) {
@@ -204,8 +381,15 @@ __global__ void __launch_bounds__(1024)
             r1 = min(rows, r0 + per);
   float s = 0.f;
   if (c < cols) {
-#pragma unroll 8
-    for (int r = r0; r < r1; ++r) s += g[(long)r * cols + c];
+    int r = r0;
+    for (; r + 16 <= r1; r += 16) {
+      float v[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = g[(long)(r + j) * cols + c];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) s += v[j];
+    }
+    for (; r < r1; ++r) s += g[(long)r * cols + c];
   }
   part[w][lane] = s;
   __syncthreads();
@@ -238,7 +422,7 @@ __global__ void __launch_bounds__(256)
 __global__ void k_adam(float *__restrict__ w, const float *__restrict__ g,
                        float *__restrict__ m, float *__restrict__ v, long n,
                        float lr, float b1, float b2, float eps, float c1,
-                       float c2, uint16_t *__restrict__ wb) {
+                       float c2, uint16_t *__restrict__ wb, MlpNet net) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   float gi = g[i];
@@ -248,8 +432,16 @@ __global__ void k_adam(float *__restrict__ w, const float *__restrict__ g,
   v[i] = vi;
   float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   w[i] = wi;
-  if (wb) wb[i] = f2bf(wi);
+  const uint16_t b = f2bf(wi);
+  wb[i] = b;
+  mlp_pack_param(net, i, b);
 }
+
+// Packed values up to which inference goes in one launch. One launch and layer
+// by layer in us, 716 inputs and 180 outputs, 16 and 1,000 rows: 256 wide (0.5
+// Mi values) 15 and 16, 36 and 46; 768 wide (2.0 Mi) 44 and 47, 47 and 85;
+// 1,024 wide (3.0 Mi) 73 and 67, 52 and 115.
+constexpr long kMlpFusedWeights = 2 << 20;
 
 struct MlpImpl {
   int nin = 0, width = 0, nout = 0;
@@ -260,6 +452,8 @@ struct MlpImpl {
   dbuf norm;                                 // mu[nin], sigma[nin], tau[nout]
   dbuf skip;                                 // BF16 S[nout][nin] (optional)
   bool has_skip = false;
+  MlpNet net{};                              // one-launch inference
+  dbuf packed;
   dbuf act;                                  // activations / scratch
   long act_rows = 0;
   long step = 0;
@@ -294,6 +488,7 @@ struct MlpImpl {
     FS_TRY(adam_v.alloc(sizeof(float) * nparams));
     FS_TRY(wbf.alloc(sizeof(uint16_t) * nparams));
     FS_TRY(norm.alloc(sizeof(float) * (2 * nin + nout)));
+    FS_TRY(init_packed());
     // He-uniform initialisation from a splitmix64 stream, zero biases
     std::vector<float> h(nparams, 0.f);
     uint64_t s = seed;
@@ -330,11 +525,12 @@ struct MlpImpl {
     wbf.release();
     norm.release();
     skip.release();
+    packed.release();
     act.release();
   }
   int requantise() {
-    hipLaunchKernelGGL(k_to_bf16, dim3(ceil_div(nparams, 256)), dim3(256), 0,
-                       st, params.as<float>(), nparams, wbf.as<uint16_t>());
+    hipLaunchKernelGGL(k_quantise, dim3(ceil_div(nparams, 256)), dim3(256), 0,
+                       st, params.as<float>(), nparams, wbf.as<uint16_t>(), net);
     FS_LAUNCHED();
     return FS_OK;
   }
@@ -413,7 +609,50 @@ struct MlpImpl {
     FS_LAUNCHED();
     return FS_OK;
   }
+  // Whether inference goes in one launch. Every workgroup reads all weights,
+  // so nets beyond kMlpFusedWeights go layer by layer, where workgroups share
+  // them out. Its outputs must not lie over inputs that another workgroup has
+  // yet to read.
+  bool fused(int B, const float *X, const float *Yout) const {
+    const uintptr_t x = (uintptr_t)X, y = (uintptr_t)Yout;
+    return net.packed && (x + sizeof(float) * (size_t)B * nin <= y ||
+                          y + sizeof(float) * (size_t)B * nout <= x);
+  }
+  size_t fused_lds() const {
+    return sizeof(uint16_t) * kMlpRows *
+           ((size_t)mlp_row(nin) + 2 * (size_t)mlp_row(width));
+  }
+  int init_packed() {
+    long o = 0;
+    for (int l = 0; l < 5; ++l) {
+      net.dims[l] = dims[l];
+      if (l < 4) {
+        net.woff[l] = woff[l];
+        net.boff[l] = boff[l];
+      }
+      net.poff[l] = o;
+      o += l < 4 ? mlp_packed_size(dims[l], dims[l + 1])
+                 : mlp_packed_size(nin, nout);
+    }
+    net.packed = nullptr;
+    if (o > kMlpFusedWeights || fused_lds() > 160 * 1024) return FS_OK;
+    FS_TRY(packed.alloc(sizeof(uint16_t) * o));
+    FS_HIP(hipMemset(packed.p, 0, sizeof(uint16_t) * o));
+    FS_HIP(hipFuncSetAttribute((const void *)k_mlp_forward,
+                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                               160 * 1024));
+    net.packed = packed.as<uint16_t>();
+    return FS_OK;
+  }
   int forward(int B, const float *X, float *Yout) {
+    if (fused(B, X, Yout)) {
+      hipLaunchKernelGGL(k_mlp_forward, dim3(ceil_div(B, kMlpRows)),
+                         dim3(64 * kMlpWaves), fused_lds(), st, B, net,
+                         (int)has_skip, mu(), sig(), tau(), params.as<float>(),
+                         X, Yout);
+      FS_LAUNCHED();
+      return FS_OK;
+    }
     FS_TRY(forward_n(B, X));
     FS_HIP(hipMemcpyAsync(Yout, Y, sizeof(float) * B * nout,
                           hipMemcpyDeviceToDevice, st));
@@ -474,7 +713,7 @@ struct MlpImpl {
     hipLaunchKernelGGL(k_adam, dim3(ceil_div(nparams, 256)), dim3(256), 0, st,
                        params.as<float>(), grads.as<float>(), adam_m.as<float>(),
                        adam_v.as<float>(), nparams, lr, b1, b2, 1e-8f, c1, c2,
-                       wbf.as<uint16_t>());
+                       wbf.as<uint16_t>(), net);
     FS_LAUNCHED();
     return FS_OK;
   }
@@ -597,6 +836,9 @@ extern "C" int fs_mlp_set_skip(fs_mlp *h, const float *S) {
   if (rc == FS_OK) {
     hipLaunchKernelGGL(fs::k_to_bf16, dim3(fs::ceil_div(n, 256)), dim3(256), 0,
                        nullptr, tmp.as<float>(), n, m.skip.as<uint16_t>());
+    if (m.net.packed)
+      hipLaunchKernelGGL(fs::k_pack_skip, dim3(fs::ceil_div(n, 256)), dim3(256), 0,
+                         nullptr, m.skip.as<uint16_t>(), m.net);
     if (hipDeviceSynchronize() != hipSuccess) {
       fs::set_error("conversion of the skip map failed");
       rc = FS_ERR_HIP;
