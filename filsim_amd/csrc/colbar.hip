@@ -174,7 +174,7 @@ __device__ __forceinline__ CbRow cb_row(const CbGeom &g, int cx, int cy, int cz,
   return r;
 }
 
-// mode 0: F[i] += sum of pair forces, min distance; mode 1: count pairs
+// mode 0: F[i] += sum of pair forces, min distance (min_bits may be null); mode 1: count pairs
 // (i<j) inside the cutoff into *npairs and write them when room.
 // Bound by the latency of dependent loads (row starts, id, position): the
 // kCbLanes lanes of a segment look up its 9 rows of three cells together, lay
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(256)
     F[3 * i + 1] += fy;
     F[3 * i + 2] += fz;
   }
-  if (mode != 0) return;
+  if (!min_bits) return;
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) mymin = fmin(mymin, __shfl_xor(mymin, m, 64));
   if ((threadIdx.x & 63) == 0) s_min[threadIdx.x >> 6] = mymin;
@@ -394,17 +394,19 @@ int ColbarImpl::apply(const double *Y, int nt, double *F, double *min_dist2,
                       hipStream_t st) {
   FS_CHECK(linked, FS_ERR_STATE, "apply before link");
   FS_CHECK(np == 0 || (Y && F), FS_ERR_ARG, "null array");
-  double init = 100000.0;
-  unsigned long long ib;
-  memcpy(&ib, &init, sizeof ib);
-  hipLaunchKernelGGL(k_cb_init_min, dim3(1), dim3(1), 0, st, act,
-                     minb.as<unsigned long long>(), ib);
+  // the minimum only where it is asked for
+  unsigned long long *mb = min_dist2 ? minb.as<unsigned long long>() : nullptr;
+  if (mb) {
+    double init = 100000.0;
+    unsigned long long ib;
+    memcpy(&ib, &init, sizeof ib);
+    hipLaunchKernelGGL(k_cb_init_min, dim3(1), dim3(1), 0, st, act, mb, ib);
+  }
   if (np > 0)
     hipLaunchKernelGGL(k_cb_apply, dim3(ceil_div((long)np * kCbLanes, 256)), dim3(256), 0, st,
                        act, np, Y, g, consts(nt), cell.as<int>(), start.as<int>(),
                        slot.as<int>(), sfil.as<int>(), sseg.as<int>(), F,
-                       minb.as<unsigned long long>(), 0, (int *)nullptr, 0,
-                       (int *)nullptr);
+                       mb, 0, (int *)nullptr, 0, (int *)nullptr);
   FS_LAUNCHED();
   if (min_dist2) {
     unsigned long long hb;

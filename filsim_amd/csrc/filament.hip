@@ -350,9 +350,15 @@ __global__ void k_forces(SysDev S, int nt) {
   d_forces(S, nt);
 }
 // Filament::update then the forces of the updated state, one workgroup per
-// filament: both read and write only their own filament's beads
-__global__ void k_update_forces(SysDev S, const double *__restrict__ u, int nt) {
+// filament: both read and write only their own filament's beads. Clears the
+// words of the residual that follows (mb, see k_resid_reset).
+__global__ void k_update_forces(SysDev S, const double *__restrict__ u, int nt,
+                                unsigned long long *__restrict__ mb) {
   if (S.act && !*S.act) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    mb[0] = 0ull;
+    mb[3] = 0ull;
+  }
   d_update(S, u);
   __syncthreads();
   d_forces(S, nt);
@@ -1095,10 +1101,56 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+//
+// Workgroups past the filaments make the differences of the Broyden step (dd):
+// both only read the new residual, and a launch of their own would cost more
+// than their work.
+struct DiffDots {
+  const double *En, *Eo;
+  double *dE;
+  double *partial;  // 2 sums per workgroup
+  size_t n;
+  int blocks;  // of kDiffChunk entries; 0: none
+};
+constexpr int kDiffChunk = 512;
+// dE = En - Eo of chunk `blk`, and its sums of dE.dE and dE.En (fixed partition
+// and order: deterministic). One wavefront.
+__device__ __forceinline__ void d_diff_dots(const DiffDots &dd, int blk) {
+  const size_t lo = (size_t)blk * kDiffChunk + threadIdx.x;
+  double a = 0, b = 0;
+#pragma unroll
+  for (int k = 0; k < kDiffChunk / 64; ++k) {
+    const size_t r = lo + 64 * k;
+    const double e = r < dd.n ? dd.En[r] : 0.0;
+    const double d = r < dd.n ? e - dd.Eo[r] : 0.0;
+    if (r < dd.n) dd.dE[r] = d;
+    a += d * d;
+    b += d * e;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    a += __shfl_xor(a, off, 64);
+    b += __shfl_xor(b, off, 64);
+  }
+  if (threadIdx.x == 0) {
+    dd.partial[2 * blk] = a;
+    dd.partial[2 * blk + 1] = b;
+  }
+}
+__global__ void __launch_bounds__(64)
+    k_diff_dots(const int *__restrict__ act, DiffDots dd) {
+  if (act && !*act) return;
+  d_diff_dots(dd, blockIdx.x);
+}
 __global__ void __launch_bounds__(64)
     k_blk_solve(SysDev S, const double *__restrict__ Fall,
-                const double *__restrict__ b, double *__restrict__ x) {
+                const double *__restrict__ b, double *__restrict__ x,
+                DiffDots dd) {
   if (S.act && !*S.act) return;
+  if (blockIdx.x >= gridDim.x - dd.blocks) {
+    d_diff_dots(dd, blockIdx.x - (gridDim.x - dd.blocks));
+    return;
+  }
   __shared__ double sy[kBandMaxNwBlk * kBlk];  // permuted b, then y, x
   __shared__ double sr[kBlk];
   const int f = blockIdx.x;
@@ -1261,18 +1313,37 @@ __global__ void __launch_bounds__(64)
   if (lane == 0) out[i] = s;
 }
 
-__global__ void k_hist_axpy(const int *__restrict__ act,
-                            const double *__restrict__ C, size_t lda, int ncol,
-                            const int *__restrict__ ncolp, int noff,
-                            const double *__restrict__ coef, size_t nrow,
-                            double *__restrict__ x) {
+// x += C coef. With nblk > 0 the coefficients are still the partial sums of
+// k_dots_partial, and every workgroup adds them up itself: for a few sums that
+// costs less than a launch.
+__global__ void __launch_bounds__(256)
+    k_hist_axpy(const int *__restrict__ act, const double *__restrict__ C,
+                size_t lda, int ncol, const int *__restrict__ ncolp, int noff,
+                const double *__restrict__ coef,
+                const double *__restrict__ partial, int nblk, int ldp,
+                size_t nrow, double *__restrict__ x) {
   if (act && !*act) return;
   if (ncolp) ncol = *ncolp + noff;
-  size_t r = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nrow) return;
-  double v = x[r];
-  for (int i = 0; i < ncol; ++i) v += C[lda * i + r] * coef[i];
-  x[r] = v;
+  __shared__ double s_coef[256];
+  const size_t r = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  double v = r < nrow ? x[r] : 0.0;
+  for (int i0 = 0; i0 < ncol; i0 += 256) {
+    const int i = i0 + threadIdx.x, m = min(256, ncol - i0);
+    __syncthreads();
+    if (i < ncol) {
+      double c = 0;
+      if (nblk > 0)
+        for (int b = 0; b < nblk; ++b) c += partial[(size_t)b * ldp + i];
+      else
+        c = coef[i];
+      s_coef[threadIdx.x] = c;
+    }
+    __syncthreads();
+    if (r < nrow)
+#pragma unroll 4
+      for (int k = 0; k < m; ++k) v += C[lda * (i0 + k) + r] * s_coef[k];
+  }
+  if (r < nrow) x[r] = v;
 }
 
 __global__ void k_sub(const double *__restrict__ a, const double *__restrict__ b,
@@ -1297,49 +1368,18 @@ __global__ void k_broyden_cols(const double *__restrict__ tmp,
   Dcol[r] = dE[r] / nrm;
 }
 
-// dE = Enew - E and the per-block partial sums of dE.dE and dE.Enew
-// (fixed partition: deterministic).
-__global__ void __launch_bounds__(256)
-    k_diff_dots(const int *__restrict__ act, const double *__restrict__ En,
-                const double *__restrict__ Eo, double *__restrict__ dE,
-                size_t n, int chunk, double *__restrict__ partial) {
-  if (act && !*act) return;
-  __shared__ double r1[256], r2[256];
-  const size_t lo = (size_t)blockIdx.x * chunk;
-  const size_t hi = min(n, lo + chunk);
-  double a = 0, b = 0;
-  for (size_t r = lo + threadIdx.x; r < hi; r += 256) {
-    double e = En[r], d = e - Eo[r];
-    dE[r] = d;
-    a += d * d;
-    b += d * e;
-  }
-  r1[threadIdx.x] = a;
-  r2[threadIdx.x] = b;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off) {
-      r1[threadIdx.x] += r1[threadIdx.x + off];
-      r2[threadIdx.x] += r2[threadIdx.x + off];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    partial[2 * blockIdx.x] = r1[0];
-    partial[2 * blockIdx.x + 1] = r2[0];
-  }
-}
-
 // Fused bad-Broyden step. With g = H_k E_new (history columns < k), the
 // reference's second solve H_k dE equals g - Update, so its column
 // C_k = (-H_k dE - Update)/|dE| = -g/|dE|, D_k = dE/|dE|, and the next
 // update H_{k+1} E_new = g + C_k (D_k . E_new) = g (1 - dE.E_new/|dE|^2).
-// Columns col of C and D (column stride n); with iterp, col = *iterp - 1.
+// Columns col of C and D (column stride n); with iterp, col = *iterp - 1. Each
+// workgroup adds the nblk partial sums of |dE|^2 and dE.E_new itself (a fixed
+// order), 6 loads a lane at 30k segments.
 __global__ void k_broyden_fused(const int *__restrict__ act,
                                 const double *__restrict__ g,
                                 const double *__restrict__ dE,
-                                const double *__restrict__ dots, size_t n,
-                                double *__restrict__ Cm,
+                                const double *__restrict__ partial, int nblk,
+                                size_t n, double *__restrict__ Cm,
                                 double *__restrict__ Dm, int col,
                                 const int *__restrict__ iterp,
                                 double *__restrict__ upd) {
@@ -1347,8 +1387,17 @@ __global__ void k_broyden_fused(const int *__restrict__ act,
   if (iterp) col = *iterp - 1;
   double *Ccol = Cm + n * (size_t)col, *Dcol = Dm + n * (size_t)col;
   size_t r = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  double nrm2 = 0, dEN = 0;  // every wavefront for itself
+  for (int b = threadIdx.x & 63; b < nblk; b += 64) {
+    nrm2 += partial[2 * b];
+    dEN += partial[2 * b + 1];
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    nrm2 += __shfl_xor(nrm2, off, 64);
+    dEN += __shfl_xor(dEN, off, 64);
+  }
   if (r >= n) return;
-  const double nrm2 = dots[0], dEN = dots[1];
   const double nrm = sqrt(nrm2);
   const double gr = g[r];
   Ccol[r] = -gr / nrm;
@@ -1540,12 +1589,15 @@ int SystemImpl::init(const fs_sim_params &pp, int nfil, const int *nwv,
   }
   dot_chunk = 2048;
   dot_blocks = ceil_div((long)n6, dot_chunk);
+  diff_blocks = ceil_div((long)n6, kDiffChunk);
+  FS_TRY(diffp.alloc(sizeof(double) * 2 * (size_t)diff_blocks));
   FS_TRY(alloc_history(p.broyden_maxiter));
   FS_TRY(flags.alloc(64));
   FS_TRY(ctl.alloc(4 * sizeof(int)));
   hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(4), 0, st, ctl.as<int>(), 4, 0);
   FS_LAUNCHED();
   FS_HIP(hipHostMalloc((void **)&hflags, 64, hipHostMallocDefault));
+  FS_HIP(hipEventCreateWithFlags(&resid_ev, hipEventDisableTiming));
   d.np = np;
   d.nlam = nlam;
   d.nf = nf;
@@ -1589,10 +1641,13 @@ void SystemImpl::release() {
   Dm.release();
   partial.release();
   coefb.release();
+  diffp.release();
   flags.release();
   ctl.release();
   if (hflags) (void)hipHostFree(hflags);
   hflags = nullptr;
+  if (resid_ev) (void)hipEventDestroy(resid_ev);
+  resid_ev = nullptr;
   fcm.release();
   cb.release();
   if (st) (void)hipStreamDestroy(st);
@@ -1669,10 +1724,12 @@ int SystemImpl::initial_guess() {
   return FS_OK;
 }
 
-// update(u) then forces(nt) in one launch
+// update(u) then forces(nt) in one launch, which also clears the residual's
+// flag words
 int SystemImpl::update_forces(const double *u, int nt) {
   ProfScope ps_(*this, P_ASSIGN);
-  hipLaunchKernelGGL(k_update_forces, dim3(nf), dim3(64), 0, st, d, u, nt);
+  hipLaunchKernelGGL(k_update_forces, dim3(nf), dim3(64), 0, st, d, u, nt,
+                     flags.as<unsigned long long>());
   FS_LAUNCHED();
   return springs();
 }
@@ -1864,7 +1921,7 @@ int SystemImpl::jinv_dense(int f, double *out) {
                        dim3(256), 0, st, b, n6, 0.0);
     hipLaunchKernelGGL(k_fill_f64, dim3(1), dim3(1), 0, st, b + so + c, (size_t)1,
                        1.0);
-    rc = jsolve_impl(b, x, 0, nullptr, 0);
+    rc = jsolve_impl(b, x, 0, nullptr, 0, nullptr);
     if (rc == FS_OK &&
         hipMemcpyAsync(col.data(), x + so, sizeof(double) * n,
                        hipMemcpyDeviceToHost, st) != hipSuccess) {
@@ -1881,23 +1938,28 @@ int SystemImpl::jinv_dense(int f, double *out) {
   return rc;
 }
 
-int SystemImpl::jsolve(const double *b, double *x, int iter) {
+int SystemImpl::jsolve(const double *b, double *x, int iter, const double *Eo) {
   FS_CHECK(iter >= 0 && iter < hcols, FS_ERR_ARG, "bad iter %d", iter);
   FS_CHECK(b != x, FS_ERR_ARG, "jsolve needs distinct b and x");
-  return jsolve_impl(b, x, iter, nullptr, 0);
+  return jsolve_impl(b, x, iter, nullptr, 0, Eo);
 }
 
 // x = blockdiag(J^-1) b + sum_{i < ncol} C_i (D_i . b). With ncolp the
 // history length is *ncolp + noff, read on the device (grids sized for
-// broyden_maxiter); the launches honour d.act.
+// broyden_maxiter); the launches honour d.act. With Eo also dE = b - Eo and
+// the partial sums of dE.dE and dE.b (diffp).
 int SystemImpl::jsolve_impl(const double *b, double *x, int ncol,
-                            const int *ncolp, int noff) {
+                            const int *ncolp, int noff, const double *Eo) {
   ProfScope ps_(*this, P_SLVJ);
   const int *act = d.act;
+  const DiffDots dd{b, Eo, dE, diffp.as<double>(), 6 * (size_t)np,
+                    Eo ? diff_blocks : 0};
   if (banded()) {
-    hipLaunchKernelGGL(k_blk_solve, dim3(nf), dim3(64), 0, st, d,
-                       Fb.as<double>(), b, x);
+    hipLaunchKernelGGL(k_blk_solve, dim3(nf + dd.blocks), dim3(64), 0, st, d,
+                       Fb.as<double>(), b, x, dd);
   } else {
+    if (Eo)
+      hipLaunchKernelGGL(k_diff_dots, dim3(dd.blocks), dim3(64), 0, st, act, dd);
     hipLaunchKernelGGL(k_jsolve_block, dim3(nf), dim3(256), 0, st, d,
                        Jinv_cm(), b, x);
   }
@@ -1908,12 +1970,16 @@ int SystemImpl::jsolve_impl(const double *b, double *x, int ncol,
     hipLaunchKernelGGL(k_dots_partial, dim3(dot_blocks, gy), dim3(256), 0, st,
                        act, Dm.as<double>(), n6, ncol, ncolp, noff, gy, b, n6,
                        dot_chunk, partial.as<double>());
-    hipLaunchKernelGGL(k_dots_final, dim3(gy), dim3(64), 0, st, act,
-                       partial.as<double>(), dot_blocks, gy, ncol, ncolp, noff,
-                       coefb.as<double>());
+    // up to 8 sums a column (2,730 segments) the axpy adds them itself
+    const bool few = dot_blocks <= 8;
+    if (!few)
+      hipLaunchKernelGGL(k_dots_final, dim3(gy), dim3(64), 0, st, act,
+                         partial.as<double>(), dot_blocks, gy, ncol, ncolp, noff,
+                         coefb.as<double>());
     hipLaunchKernelGGL(k_hist_axpy, dim3(ceil_div((long)n6, 256)), dim3(256), 0,
                        st, act, Cm.as<double>(), n6, ncol, ncolp, noff,
-                       coefb.as<double>(), n6, x);
+                       coefb.as<double>(), partial.as<double>(),
+                       few ? dot_blocks : 0, gy, n6, x);
     FS_LAUNCHED();
   }
   return FS_OK;
@@ -1945,15 +2011,29 @@ int SystemImpl::broyden_update(const double *Eo, const double *En,
 
 int SystemImpl::residual(int nt, const double *V, const double *W, double *err,
                          int *check, double *maxabs) {
+  hipLaunchKernelGGL(k_resid_reset, dim3(1), dim3(1), 0, st, d.act,
+                     flags.as<unsigned long long>());
+  FS_TRY(residual_launch(nt, V, W, err));
+  return residual_wait(check, maxabs);
+}
+
+// The residual kernel and the copy of its flag words, which are clear before;
+// residual_wait() returns what they say.
+int SystemImpl::residual_launch(int nt, const double *V, const double *W,
+                                double *err) {
   ProfScope ps_(*this, P_ERRCHK);
   unsigned long long *mb = flags.as<unsigned long long>();
-  hipLaunchKernelGGL(k_resid_reset, dim3(1), dim3(1), 0, st, d.act, mb);
   hipLaunchKernelGGL(k_residual, dim3(ceil_div(np, 256)), dim3(256), 0, st, d,
                      nt, V, W, err, mb);
   FS_LAUNCHED();
   FS_HIP(hipMemcpyAsync(hflags, mb, 4 * sizeof(unsigned long long),
                         hipMemcpyDeviceToHost, st));
-  FS_HIP(hipStreamSynchronize(st));
+  FS_HIP(hipEventRecord(resid_ev, st));
+  return FS_OK;
+}
+
+int SystemImpl::residual_wait(int *check, double *maxabs) {
+  FS_HIP(hipEventSynchronize(resid_ev));
   double m;
   memcpy(&m, hflags, sizeof m);
   if (maxabs) *maxabs = m;
@@ -2078,30 +2158,25 @@ int SystemImpl::broyden_loop(int nt, int *iters) {
     FS_TRY(update_forces(Upd, nt));
     FS_TRY(barrier(nt, 0, nullptr));
     FS_TRY(mobility(nt));
-    FS_TRY(residual(nt, d.V, d.W, NewE, &check, &last_res));
+    FS_TRY(residual_launch(nt, d.V, d.W, NewE));
     ++iter;
-    if (!check || iter >= p.broyden_maxiter) break;
-    // dE = NewE - E; |dE|^2 and dE.NewE; g = H_{iter-1} NewE
-    double *dots = coefb.as<double>() + hcols;  // 2 scalars
-    {
-      ProfScope ps_(*this, P_SLVJ);
-      hipLaunchKernelGGL(k_diff_dots, dim3(dot_blocks), dim3(256), 0, st,
-                         (const int *)nullptr, NewE, E, dE, n6, dot_chunk,
-                         partial.as<double>());
-      hipLaunchKernelGGL(k_dots_final, dim3(2), dim3(64), 0, st,
-                         (const int *)nullptr, partial.as<double>(), dot_blocks,
-                         2, 2, (const int *)nullptr, 0, dots);
-      FS_LAUNCHED();
-    }
-    FS_TRY(jsolve(NewE, tmp, h0 + iter - 1));
-    {
+    // The solve that the next iteration needs goes out before the host knows
+    // whether there is one: dE = NewE - E with |dE|^2 and dE.NewE, g = H_{iter-1}
+    // NewE. It writes only scratch and the column after the last one kept, and
+    // the wait for the flags (15 us of an idle GPU in each iteration) is hidden
+    // behind it.
+    if (iter < p.broyden_maxiter) {
+      FS_TRY(jsolve(NewE, tmp, h0 + iter - 1, E));
       ProfScope ps_(*this, P_SLVJ);
       hipLaunchKernelGGL(k_broyden_fused, dim3(ceil_div((long)n6, 256)),
-                         dim3(256), 0, st, (const int *)nullptr, tmp, dE, dots,
-                         n6, Cm.as<double>(), Dm.as<double>(), h0 + iter - 1,
-                         (const int *)nullptr, Upd);
+                         dim3(256), 0, st, (const int *)nullptr, tmp, dE,
+                         diffp.as<double>(), diff_blocks, n6, Cm.as<double>(),
+                         Dm.as<double>(), h0 + iter - 1, (const int *)nullptr,
+                         Upd);
       FS_LAUNCHED();
     }
+    FS_TRY(residual_wait(&check, &last_res));
+    if (!check || iter >= p.broyden_maxiter) break;
     std::swap(E, NewE);
   }
   if (hist_cap > 0) {
@@ -2170,7 +2245,7 @@ int SystemImpl::begin_step_dev(int *status, int part) {
                      ctl.as<int>() + 2);
   FS_LAUNCHED();
   set_device_control(ctl.as<int>() + 1, ntp);
-  FS_TRY(jsolve_impl(E, Upd, 0, nullptr, 0));
+  FS_TRY(jsolve_impl(E, Upd, 0, nullptr, 0, nullptr));
   set_device_control(nullptr, ntp);
   hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, st, ctl.as<int>(), 3,
                      status);
@@ -2194,22 +2269,14 @@ int SystemImpl::iteration_dev(int *status, int part) {
     return FS_OK;
   }
   unsigned long long *mb = flags.as<unsigned long long>();
-  hipLaunchKernelGGL(k_resid_reset, dim3(1), dim3(1), 0, st, act, mb);
   hipLaunchKernelGGL(k_residual, dim3(ceil_div(np, 256)), dim3(256), 0, st, d,
                      nt, d.V, d.W, NewE, mb);
   hipLaunchKernelGGL(k_ctl_after, dim3(1), dim3(1), 0, st, ctl.as<int>(), mb,
                      p.tol, p.broyden_maxiter);
-  double *dots = coefb.as<double>() + hcols;  // 2 scalars
-  hipLaunchKernelGGL(k_diff_dots, dim3(dot_blocks), dim3(256), 0, st, act, NewE,
-                     E, dE, n6, dot_chunk, partial.as<double>());
-  hipLaunchKernelGGL(k_dots_final, dim3(2), dim3(64), 0, st, act,
-                     partial.as<double>(), dot_blocks, 2, 2,
-                     (const int *)nullptr, 0, dots);
-  FS_LAUNCHED();
-  FS_TRY(jsolve_impl(NewE, tmp, 0, ctl.as<int>(), -1));
+  FS_TRY(jsolve_impl(NewE, tmp, 0, ctl.as<int>(), -1, E));
   hipLaunchKernelGGL(k_broyden_fused, dim3(ceil_div((long)n6, 256)), dim3(256),
-                     0, st, act, tmp, dE, dots, n6, Cm.as<double>(),
-                     Dm.as<double>(), 0, ctl.as<int>(), Upd);
+                     0, st, act, tmp, dE, diffp.as<double>(), diff_blocks, n6,
+                     Cm.as<double>(), Dm.as<double>(), 0, ctl.as<int>(), Upd);
   hipLaunchKernelGGL(k_copy_f64, dim3(ceil_div((long)n6, 256)), dim3(256), 0, st,
                      act, NewE, E, n6);
   set_device_control(nullptr, ntp);

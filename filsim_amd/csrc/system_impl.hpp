@@ -36,7 +36,7 @@ struct SystemImpl {
   std::vector<int> hnw, hboff, hloff;
   std::vector<long> hjoff;
   SysDev d{};
-  dbuf arena, ints, joffb, propsb, Jb, Mb, JTb, Cm, Dm, partial, coefb, flags;
+  dbuf arena, ints, joffb, propsb, Jb, Mb, JTb, Cm, Dm, partial, coefb, diffp, flags;
   // block-tridiagonal factors of the Jacobians, used while every filament
   // has at most 64 segments (the solve keeps a filament's factors in LDS);
   // the dense inverse JTb (Gauss-Jordan) otherwise
@@ -45,7 +45,8 @@ struct SystemImpl {
   double *E = nullptr, *NewE = nullptr, *Upd = nullptr, *tmp = nullptr,
          *dE = nullptr, *scratch6 = nullptr;
   unsigned long long *hflags = nullptr;
-  int dot_chunk = 0, dot_blocks = 0;
+  hipEvent_t resid_ev = nullptr;  // after the copy of the flags
+  int dot_chunk = 0, dot_blocks = 0, diff_blocks = 0;
   int max_nw = 0;
   double last_res0 = 0, last_res = 0;
   // Broyden history carried into the next timestep (no reference
@@ -71,12 +72,15 @@ struct SystemImpl {
   // clear_history: zero the Broyden history (the API's reset); the
   // timestep reads only the columns its own iterations wrote and skips it
   int build_jacobian(int nt, bool clear_history = true);
-  int jsolve(const double *b, double *x, int iter);
+  // Eo: also the Broyden differences dE = b - Eo
+  int jsolve(const double *b, double *x, int iter, const double *Eo = nullptr);
   int jinv_dense(int f, double *out);
   int broyden_update(const double *Eo, const double *En, const double *upd,
                      int iter);
   int residual(int nt, const double *V, const double *W, double *err,
                int *check, double *maxabs);
+  int residual_launch(int nt, const double *V, const double *W, double *err);
+  int residual_wait(int *check, double *maxabs);
   int step(int nt);
   int mobility(int nt);
   int barrier(int nt, int link, double *min_dist2);
@@ -127,7 +131,7 @@ struct SystemImpl {
   // still iterating, singular Jacobian}; ntp = device step number.
   dbuf ctl;
   int jsolve_impl(const double *b, double *x, int ncol, const int *ncolp,
-                  int noff);
+                  int noff, const double *Eo);
   int build_jacobian_dev(int nt);
   void set_device_control(const int *act, const int *ntp);
   int begin_step_dev(int *status, int part = -1);  // status: where to publish ctl
