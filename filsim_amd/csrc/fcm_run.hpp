@@ -1615,14 +1615,19 @@ __global__ void __launch_bounds__(256)
 // part[segment][component][slot] (slot = the tile's offset from the
 // segment's origin tile). k_interp_sum adds a segment's slots in slot
 // order: no atomics, results independent of scheduling.
-// Latency bound: of the FP64 270 us at 30k segments on 256^3 the products
-// take 90, the weights' reads from LDS 100, making the weights 50 and the
-// grid's loads 50, one after another. So wavefronts count: three accumulators
-// at a time fit 128 registers, four waves a SIMD instead of two (FP64 297 ->
-// 270 us, FP32 125 -> 120 us; 128^3 FP64 55 -> 46 us). One wavefront to a
-// tile 257 / 140 us, and slower on small grids; weights read 16 bytes at a
-// time 313 / 125 us (spills).
+// Latency bound: of the FP64 270 us at 30k segments on 256^3 that the form with
+// four wavefronts a SIMD took, the products were 90, the weights' reads from
+// LDS 100, making the weights 50 and the grid's loads 50, one after another. So
+// three accumulators at a time, which leaves registers for wavefronts: FP32
+// four a SIMD (125 -> 117 us; five the same, six spill: 170 us), FP64 three
+// (297 -> 224 us, two the same, four spill: 269 us; 128^3 55 -> 43 us). One
+// wavefront to a tile 257 / 140 us, and slower on small grids; weights read 16
+// bytes at a time 313 / 125 us (spills).
 // ---------------------------------------------------------------------
+// Wavefronts a SIMD that the interpolation's registers leave room for.
+template <typename T>
+constexpr int kInterpWaves = sizeof(T) == 8 ? 3 : 4;
+
 template <int NGD>
 constexpr int kInterpSlots = stencil_tiles(NGD, 8) * stencil_tiles(NGD, 8) *
                              stencil_tiles(NGD, 16);
@@ -1797,7 +1802,7 @@ __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G,
   }
 }
 template <typename T, int NGD>
-__global__ void __launch_bounds__(256, 4)
+__global__ void __launch_bounds__(256, kInterpWaves<T>)
     k_interp_mfma(const int *__restrict__ act, SpreadGeom G, GaussConst g,
                   const SegRec<T> *__restrict__ slab,
                   const SegRec<T> *__restrict__ pool,
@@ -1821,7 +1826,7 @@ struct A_interp_mfma {
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
 template <typename T, int NGD>
-__global__ void __launch_bounds__(256, 4)
+__global__ void __launch_bounds__(256, kInterpWaves<T>)
     k_interp_mfma_multi(const A_interp_mfma<T, NGD> *__restrict__ a) {
   const A_interp_mfma<T, NGD> &A = a[blockIdx.z];
   d_interp_mfma<T, NGD, const SpreadGeom &, const GaussConst &>(A.act, A.G, A.g, A.slab, A.pool, A.tcnt, A.tovf, A.R, A.part);
