@@ -180,10 +180,19 @@ int FcmImpl::set_geometry() {
     }
   FS_CHECK(tz > 0, FS_ERR_ARG, "no spread z run divides nz=%d", p.nz);
   int tx = largest_divisor_le(p.nx, t), ty = largest_divisor_le(p.ny, t);
-  // matrix-core spread: fixed 8 x 8 x 16 tiles (four 16-point MFMA rows)
-  mfma_spread = tune.spread_mfma == 1 &&
-                p.nx % 8 == 0 && p.ny % 8 == 0 && p.nz % 16 == 0 &&
-                p.nz >= 16 + p.ngd;
+  // matrix-core spread: fixed 8 x 8 x 16 tiles (four 16-point MFMA rows), the
+  // last ones of an axis cut off where it is no multiple. A stencil that wraps
+  // over a cut tile can meet one more, and one more bin can reach a tile; the
+  // list kernel looks at 64 bins, which leaves such grids with the widest
+  // supports to the vector kernels.
+  const int rx = p.nx % 8 != 0, ry = p.ny % 8 != 0, rz = p.nz % 16 != 0;
+  {
+    const int h = (p.ngd - 1 + 7) / 8, h16 = (p.ngd - 1 + 15) / 16;
+    mfma_spread = tune.spread_mfma == 1 && p.nz >= 16 + p.ngd &&
+                  std::min(h + rx + 1, ceil_div(p.nx, 8)) *
+                          std::min(h + ry + 1, ceil_div(p.ny, 8)) *
+                          std::min(h16 + rz + 1, ceil_div(p.nz, 16)) <= 64;
+  }
   if (mfma_spread) {
     tx = ty = 8;
     tz = 16;
@@ -210,16 +219,21 @@ int FcmImpl::set_geometry() {
   geom.tx = tx;
   geom.ty = ty;
   geom.tz = tz;
-  geom.nbx = p.nx / tx;
-  geom.nby = p.ny / ty;
-  geom.nbz = p.nz / tz;
+  geom.nbx = ceil_div(p.nx, tx);
+  geom.nby = ceil_div(p.ny, ty);
+  geom.nbz = ceil_div(p.nz, tz);
   geom.hx = (p.ngd - 1 + tx - 1) / tx;
   geom.hy = (p.ngd - 1 + ty - 1) / ty;
   geom.hz = (p.ngd - 1 + tz - 1) / tz;
   nbins = geom.nbx * geom.nby * geom.nbz;
+  geom.sx = stencil_tiles(p.ngd, 8) + rx;
+  geom.sy = stencil_tiles(p.ngd, 8) + ry;
+  geom.sz = stencil_tiles(p.ngd, 16) + rz;
   if (mfma_spread) {
-    const size_t nslot = (size_t)stencil_tiles(p.ngd, 8) *
-                         stencil_tiles(p.ngd, 8) * stencil_tiles(p.ngd, 16);
+    geom.hx += rx;
+    geom.hy += ry;
+    geom.hz += rz;
+    const size_t nslot = (size_t)geom.sx * geom.sy * geom.sz;
     FS_TRY(ipart.alloc((size_t)max_np * 6 * tsz * nslot));
     FS_TRY(tslab.alloc((size_t)nbins * kTileCap * rec_bytes(tsz)));
     FS_TRY(tcnt.alloc((size_t)nbins * sizeof(int)));

@@ -15,6 +15,7 @@ struct SpreadGeom {
   int tx, ty, tz;     // tile edge
   int nbx, nby, nbz;  // tiles per dimension
   int hx, hy, hz;     // neighbouring bins per dimension (besides own)
+  int sx, sy, sz;     // tiles a stencil can meet per dimension (matrix-core path)
 };
 
 struct FcmImpl {

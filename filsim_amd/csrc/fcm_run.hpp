@@ -526,9 +526,10 @@ __device__ __forceinline__ void d_tile_lists(const int *__restrict__ act, SG G,
         }
         pos = first[lo] + j - pre[lo];
         const int org = sorg[pos];
-        keep = stencil_meets(org & 1023, px0, G.tx, G.ngd, G.nx) &&
-               stencil_meets((org >> 10) & 1023, py0, G.ty, G.ngd, G.ny) &&
-               stencil_meets(org >> 20, pz0, G.tz, G.ngd, G.nz);
+        keep = stencil_meets(org & 1023, px0, min(G.tx, G.nx - px0), G.ngd, G.nx) &&
+               stencil_meets((org >> 10) & 1023, py0, min(G.ty, G.ny - py0), G.ngd,
+                             G.ny) &&
+               stencil_meets(org >> 20, pz0, min(G.tz, G.nz - pz0), G.ngd, G.nz);
       }
       const unsigned long long kb = __ballot(keep);
       const int k = kept + __popcll(kb & ((1ull << lane) - 1ull));
@@ -579,7 +580,7 @@ __global__ void __launch_bounds__(256)
 }
 
 // The tile lists of few segments without bins: one workgroup per row of tiles
-// along x. Its threads form every segment's origin and keep, in ascending
+// along x (where the rows are few, several, each with a part of the tiles). Its threads form every segment's origin and keep, in ascending
 // order, those whose stencil meets the row in y and z; then each wavefront
 // fills the lists of tiles of the row (order, slab, pool and counts as above,
 // except that a tile's segments are in ascending order over all bins). It
@@ -606,14 +607,14 @@ __device__ __forceinline__ void d_tile_lists_direct(
   for (int s0 = 0, it = 0; s0 < np; s0 += 1024, ++it) {
     const int s = s0 + threadIdx.x;
     // one workgroup a round also stores the origins
-    const bool own = it % (int)gridDim.x == (int)blockIdx.x;
+    const bool own = it % (int)gridDim.x == (int)blockIdx.x && blockIdx.y == 0;
     bool keep = false;
     int org = 0;
     if (s < np) {
       const int oy = stencil_origin(Y[3 * s + 1], dx, s, ngdh, G.ny);
       const int oz = stencil_origin(Y[3 * s + 2], dx, s, ngdh, G.nz);
-      keep = stencil_meets(oy, by * G.ty, G.ty, G.ngd, G.ny) &&
-             stencil_meets(oz, bz * G.tz, G.tz, G.ngd, G.nz);
+      keep = stencil_meets(oy, by * G.ty, min(G.ty, G.ny - by * G.ty), G.ngd, G.ny) &&
+             stencil_meets(oz, bz * G.tz, min(G.tz, G.nz - bz * G.tz), G.ngd, G.nz);
       if (keep || own) {
         const int ox = stencil_origin(Y[3 * s], dx, s, ngdh, G.nx);
         org = ox | (oy << 10) | (oz << 20);
@@ -641,7 +642,7 @@ __device__ __forceinline__ void d_tile_lists_direct(
     }
   }
   __syncthreads();
-  for (int bx = wave; bx < G.nbx; bx += 16) {
+  for (int bx = wave + 16 * blockIdx.y; bx < G.nbx; bx += 16 * gridDim.y) {
     const int tile = bx + G.nbx * blockIdx.x;
     int kept = 0, base = 0;
     for (int pass = 0; pass < 2; ++pass) {
@@ -656,7 +657,8 @@ __device__ __forceinline__ void d_tile_lists_direct(
         const int j = j0 + lane;
         const int org = j < nrow ? s_org[j] : 0;
         const bool keep =
-            j < nrow && stencil_meets(org & 1023, bx * G.tx, G.tx, G.ngd, G.nx);
+            j < nrow && stencil_meets(org & 1023, bx * G.tx,
+                                      min(G.tx, G.nx - bx * G.tx), G.ngd, G.nx);
         const unsigned long long kb = __ballot(keep);
         const int k = kept + __popcll(kb & below);
         if (keep && (pass == 0) == (k < kTileCap)) {
@@ -717,7 +719,8 @@ __global__ void __launch_bounds__(1024)
 // Gaussian weights of one segment at a tile's axis points. Point a: x
 // (a < 8), y (8 <= a < 16), z (16 <= a < 32) of the tile starting at
 // (px0, py0, pz0). w[a] = g (monopole), w[32 + a] = gD (dipole), w[64 + a]
-// = its derivative h = gD (-xx / sigma_dip^2), zero off the stencil; xx is
+// = its derivative h = gD (-xx / sigma_dip^2), zero off the stencil and past
+// the axis' end (a cut tile); xx is
 // formed in FP64, and so is the exponent (base 2); FP32 rounds it before the
 // hardware exp2.
 // weights (96) + coefficients (6) per record; odd, so that 16 rows read at one
@@ -733,7 +736,7 @@ __device__ __forceinline__ void tile_weights(const GaussConst &g,
   int i = p - ((r.org >> (10 * d)) & 1023);
   if (i < 0) i += n;
   T ga = 0, gd = 0, h = 0;
-  if (i < g.ngd) {
+  if (i < g.ngd && p < n) {
     const double x0 = d == 0 ? r.xx0[0] : (d == 1 ? r.xx0[1] : r.xx0[2]);
     const double xx = x0 + (double)i * g.dx;
     const double x2 = xx * xx;
@@ -882,9 +885,13 @@ __device__ __forceinline__ void d_spread_mfma(const int *__restrict__ act, SG G,
   // lane holds R[xy = wave*16 + Mfma<T>::row(lane, r)][z = i16]: 16 lanes
   // write 16 consecutive z of one (x, y) column
   const size_t N = (size_t)G.nx * G.ny * G.nz;
+  const bool whole = px0 + 8 <= G.nx && py0 + 8 <= G.ny && pz0 + 16 <= G.nz;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int oxy = wave * 16 + Mfma<T>::row(lane, r);
+    if (!whole && (px0 + (oxy >> 3) >= G.nx || py0 + (oxy & 7) >= G.ny ||
+                   pz0 + i16 >= G.nz))
+      continue;
     const size_t o = ((size_t)(px0 + (oxy >> 3)) * G.ny + py0 + (oxy & 7)) *
                          G.nz + pz0 + i16;
     R[o] = acc0[r];
@@ -1647,8 +1654,7 @@ __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G,
                   const T *__restrict__ R, T *__restrict__ part) {
   typedef typename Mfma<T>::v4 v4;
   constexpr int KC = kTileCap;  // candidates per round
-  constexpr int SX = stencil_tiles(NGD, 8), SZ = stencil_tiles(NGD, 16);
-  constexpr int NSLOT = kInterpSlots<NGD>;
+  const int nslot = G.sx * G.sy * G.sz;
   if (act && !*act) return;  // batched sweep: suspension converged
   __shared__ SegRec<T> s_rec[kTileCap];
   __shared__ T s_w[KC + 1][kTileW];  // row KC stays zero
@@ -1681,9 +1687,19 @@ __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G,
       const int xy = wave * 16 + i16;
       const size_t o = ((size_t)(px0 + (xy >> 3)) * G.ny + py0 + (xy & 7)) * G.nz +
                        pz0 + 4 * q;
-      ld4(R + o, u[0]);
-      ld4(R + N + o, u[1]);
-      ld4(R + 2 * N + o, u[2]);
+      if (px0 + 8 <= G.nx && py0 + 8 <= G.ny && pz0 + 16 <= G.nz &&
+          (sizeof(T) == 8 || (G.nz & 3) == 0)) {
+        ld4(R + o, u[0]);
+        ld4(R + N + o, u[1]);
+        ld4(R + 2 * N + o, u[2]);
+      } else {  // a cut tile, or lines that are not 16-byte aligned
+        const bool in = px0 + (xy >> 3) < G.nx && py0 + (xy & 7) < G.ny;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            u[d][k] = in && pz0 + 4 * q + k < G.nz ? R[d * N + o + k] : (T)0;
+      }
     }
     const int cnt = pf.cnt;
     __syncthreads();  // the last tile is done with s_rec, s_w and s_red
@@ -1795,7 +1811,7 @@ __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G,
           if (sx < 0) sx += G.nbx;
           if (sy < 0) sy += G.nby;
           if (sz < 0) sz += G.nbz;
-          part[((size_t)rc.id * 6 + m) * NSLOT + (sx * SX + sy) * SZ + sz] = sum;
+          part[((size_t)rc.id * 6 + m) * nslot + (sx * G.sy + sy) * G.sz + sz] = sum;
         }
       }
     }
@@ -1851,28 +1867,48 @@ __device__ __forceinline__ void d_interp_sum(const int *__restrict__ act, int np
   const int s = e / 6, m = e - 6 * s;
   if (s >= np) return;
   const int ox = origin[3 * s], oy = origin[3 * s + 1], oz = origin[3 * s + 2];
-  // every slot is read (in range); the ones no tile wrote are not added
-  T v[NSLOT];
-  const T *pp = part + ((size_t)s * 6 + m) * NSLOT;
-#pragma unroll
-  for (int k = 0; k < NSLOT; ++k) v[k] = pp[k];
   double acc = 0;
+  if (G.sx == SX && G.sy == SX && G.sz == SZ) {
+    // every slot is read (in range); the ones no tile wrote are not added
+    T v[NSLOT];
+    const T *pp = part + ((size_t)s * 6 + m) * NSLOT;
 #pragma unroll
-  for (int sx = 0; sx < SX; ++sx) {
-    int tx = ox / 8 + sx;
-    if (tx >= G.nbx) tx -= G.nbx;
-    const bool mx = sx < G.nbx && stencil_meets(ox, tx * 8, 8, NGD, G.nx);
+    for (int k = 0; k < NSLOT; ++k) v[k] = pp[k];
 #pragma unroll
-    for (int sy = 0; sy < SX; ++sy) {
-      int ty = oy / 8 + sy;
-      if (ty >= G.nby) ty -= G.nby;
-      const bool my = sy < G.nby && stencil_meets(oy, ty * 8, 8, NGD, G.ny);
+    for (int sx = 0; sx < SX; ++sx) {
+      int tx = ox / 8 + sx;
+      if (tx >= G.nbx) tx -= G.nbx;
+      const bool mx = sx < G.nbx && stencil_meets(ox, tx * 8, 8, NGD, G.nx);
 #pragma unroll
-      for (int sz = 0; sz < SZ; ++sz) {
-        int tz = oz / 16 + sz;
-        if (tz >= G.nbz) tz -= G.nbz;
-        const bool mz = sz < G.nbz && stencil_meets(oz, tz * 16, 16, NGD, G.nz);
-        if (mx && my && mz) acc += (double)v[(sx * SX + sy) * SZ + sz];
+      for (int sy = 0; sy < SX; ++sy) {
+        int ty = oy / 8 + sy;
+        if (ty >= G.nby) ty -= G.nby;
+        const bool my = sy < G.nby && stencil_meets(oy, ty * 8, 8, NGD, G.ny);
+#pragma unroll
+        for (int sz = 0; sz < SZ; ++sz) {
+          int tz = oz / 16 + sz;
+          if (tz >= G.nbz) tz -= G.nbz;
+          const bool mz = sz < G.nbz && stencil_meets(oz, tz * 16, 16, NGD, G.nz);
+          if (mx && my && mz) acc += (double)v[(sx * SX + sy) * SZ + sz];
+        }
+      }
+    }
+  } else {  // cut tiles, one slot more on their axes
+    const T *pp = part + ((size_t)s * 6 + m) * (G.sx * G.sy * G.sz);
+    for (int sx = 0; sx < min(G.sx, G.nbx); ++sx) {
+      int tx = ox / 8 + sx;
+      if (tx >= G.nbx) tx -= G.nbx;
+      if (!stencil_meets(ox, tx * 8, min(8, G.nx - tx * 8), NGD, G.nx)) continue;
+      for (int sy = 0; sy < min(G.sy, G.nby); ++sy) {
+        int ty = oy / 8 + sy;
+        if (ty >= G.nby) ty -= G.nby;
+        if (!stencil_meets(oy, ty * 8, min(8, G.ny - ty * 8), NGD, G.ny)) continue;
+        for (int sz = 0; sz < min(G.sz, G.nbz); ++sz) {
+          int tz = oz / 16 + sz;
+          if (tz >= G.nbz) tz -= G.nbz;
+          if (stencil_meets(oz, tz * 16, min(16, G.nz - tz * 16), NGD, G.nz))
+            acc += (double)pp[(sx * G.sy + sy) * G.sz + sz];
+        }
       }
     }
   }
@@ -2022,6 +2058,12 @@ int interp_blocks(const FcmImpl &f) {
   return b;
 }
 
+// Workgroups per row of tiles of the lists without bins: up to 16 tiles (one a
+// wavefront) each, where that fills the chip.
+static int direct_parts(const SpreadGeom &g) {
+  return std::max(1, std::min(ceil_div(g.nbx, 16), 256 / (g.nby * g.nbz)));
+}
+
 // Gaussian constants of the spread, tables and interpolation.
 static GaussConst gauss_const(const fs_fcm_params &p) {
   GaussConst g;
@@ -2091,8 +2133,8 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   const int ntiles = nbins;
   if (direct) {
     kmark(1);
-    hipLaunchKernelGGL(k_tile_lists_direct<T>, dim3(geom.nby * geom.nbz),
-                       dim3(1024), 0, st, act, np, geom, p.dx, Y, F, Tq,
+    hipLaunchKernelGGL(k_tile_lists_direct<T>,
+                       dim3(geom.nby * geom.nbz, direct_parts(geom)), dim3(1024), 0, st, act, np, geom, p.dx, Y, F, Tq,
                        origin.as<int>(), tslab.as<SegRec<T>>(), tcnt.as<int>(),
                        tovf.as<int>(), tpool.as<SegRec<T>>(),
                        bin_count.as<int>() + nbins);
@@ -2326,7 +2368,8 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
     });
     if (!host)
       hipLaunchKernelGGL(k_tile_lists_direct_multi<T>,
-                         dim3(f0.geom.nby * f0.geom.nbz, 1, S), dim3(1024), 0, st,
+                         dim3(f0.geom.nby * f0.geom.nbz, direct_parts(f0.geom), S),
+                         dim3(1024), 0, st,
                          (const A_tile_lists_direct<T> *)t);
   } else {
     {

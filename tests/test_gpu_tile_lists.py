@@ -61,3 +61,27 @@ def test_binned_groups_equal_unbatched(cuda):
         for k in ("X", "U", "q", "lam"):
             assert np.array_equal(sa[k], sb[k]), k
     batch.close()
+
+
+@pytest.mark.parametrize("ngd", [6, 8, 10, 12, 16, 20, 24])
+def test_cut_tiles_match_vector_path(cuda, ngd):
+    """Grids whose axes are no multiples of the tiles: cut by one to three
+    axes, by 2 to 14 points, lines that are not 16-byte aligned, boxes narrower
+    than a stencil and a tile. Bounds as above in FP64; FP32 1e-5, the bar of
+    the solver's FP32 tests."""
+    for grid in ((30, 36, 50), (40, 40, 40), (54, 30, 90), (36, 50, 48),
+                 (32, 40, 54), (100, 32, 48), (30, 30, 60), (50, 90, 80)):
+        if min(grid) < ngd + 4:
+            continue
+        fp = params.fcm_params(grid, ngd=ngd)
+        n = 400
+        Y, F, T = random_segments(fp, n, seed=sum(grid) + ngd)
+        for prec, bar in ((abi.FS_FP64, 1e-12), (abi.FS_FP32, 1e-5)):
+            with api.Fcm(fp, n, precision=prec) as fcm, \
+                    api.Fcm(fp, n, precision=prec) as vec:
+                vec.set_tuning(spread_mfma=0)
+                V, W = fcm.mobility_host(Y, F, T)
+                Vo, Wo = vec.mobility_host(Y, F, T)
+            top = max(np.linalg.norm(Wo), np.linalg.norm(Vo) / fp.a)
+            assert rel(V, Vo) <= bar, (grid, prec)
+            assert np.linalg.norm(W - Wo) <= bar * top, (grid, prec)
