@@ -182,16 +182,17 @@ int FcmImpl::set_geometry() {
   int tx = largest_divisor_le(p.nx, t), ty = largest_divisor_le(p.ny, t);
   // matrix-core spread: fixed 8 x 8 x 16 tiles (four 16-point MFMA rows), the
   // last ones of an axis cut off where it is no multiple. A stencil that wraps
-  // over a cut tile can meet one more, and one more bin can reach a tile; the
-  // list kernel looks at 64 bins, which leaves such grids with the widest
-  // supports to the vector kernels.
+  // over a cut tile can meet one more, and one more bin can reach a tile (5 x 5
+  // x 4 at most). Both ways, spread and interpolation in us: 90^3 FP32 with
+  // 1,080 segments 35 and (vector gather) 84, 150^3 FP64 with 3,000 75 and 108,
+  // 250^3 FP32 with 27,000 243 and 570.
   const int rx = p.nx % 8 != 0, ry = p.ny % 8 != 0, rz = p.nz % 16 != 0;
   {
     const int h = (p.ngd - 1 + 7) / 8, h16 = (p.ngd - 1 + 15) / 16;
     mfma_spread = tune.spread_mfma == 1 && p.nz >= 16 + p.ngd &&
                   std::min(h + rx + 1, ceil_div(p.nx, 8)) *
                           std::min(h + ry + 1, ceil_div(p.ny, 8)) *
-                          std::min(h16 + rz + 1, ceil_div(p.nz, 16)) <= 64;
+                          std::min(h16 + rz + 1, ceil_div(p.nz, 16)) <= kListBins;
   }
   if (mfma_spread) {
     tx = ty = 8;
@@ -247,6 +248,9 @@ int FcmImpl::set_geometry() {
   // 2,400 on 192^3 (864) 37 and 28, growing with the row steps.
   direct = mfma_spread && max_np <= kDirectMax &&
            (long)ceil_div(max_np, 1024) * geom.nby * geom.nbz <= kDirectRowSteps;
+  // FP64 weights cost nothing where launches and latency bound the tile kernels;
+  // on cut grids the vector gather, which takes them too, was the other way
+  fine = direct || rx || ry || rz;
   // one more counter after the bins: the tile lists' pool top
   FS_TRY(bin_count.alloc((size_t)(nbins + 1) * sizeof(int)));
   FS_HIP(hipMemset(bin_count.p, 0, (size_t)(nbins + 1) * sizeof(int)));

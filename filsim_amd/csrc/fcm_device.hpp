@@ -14,7 +14,8 @@ constexpr int kMaxBinsPerTile = 64;
 struct GaussConst {
   double dx, anorm, anorm2, anormdip, anormdip2, sigmadipsq;
   int ngd, ngdh, nx, ny, nz;
-  // FP32 weights: g = anorm 2^(-xx^2 e2), gD = anormdip 2^(-xx^2 ed2),
+  int fine;  // FP32 tile weights: FP64, rounded
+  // base-2 weights: g = anorm 2^(-xx^2 e2), gD = anormdip 2^(-xx^2 ed2),
   // e2 = log2(e) / anorm2, ed2 = log2(e) / anormdip2
   double e2, ed2;
   double nrsd;  // -1 / sigmadipsq
@@ -31,6 +32,7 @@ struct alignas(16) SegRec {
   T cf[6];
 };
 constexpr int kTileCap = 32;  // records in a tile's slab; the rest: pool
+constexpr int kListBins = 128;  // bins a tile's list is gathered from
 constexpr int kDirectMax = 4096;  // segments of tile lists without bins (LDS)
 // steps of 1,024 segments over all rows of tiles, where the line to them lies
 constexpr long kDirectRowSteps = 1024;

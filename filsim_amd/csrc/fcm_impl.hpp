@@ -38,6 +38,7 @@ struct FcmImpl {
   int nbins = 0;
   bool mfma_spread = false;  // spread on the matrix cores (8 x 8 x 16 tiles)
   bool direct = false;  // tile lists straight from the segments, without bins
+  bool fine = false;    // FP32 tile weights formed in FP64
   int grid_interp = 0;  // blocks of the persistent interpolation
   int zP = 1, yB = 1, xQ = 1;  // FFT pass workgroup shapes
   // device flag read by every kernel of a solve: 0 = skip (a converged

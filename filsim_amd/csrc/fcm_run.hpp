@@ -465,7 +465,7 @@ __device__ __forceinline__ void d_tile_lists(const int *__restrict__ act, SG G,
                  int *__restrict__ tcnt, int *__restrict__ tovf,
                  SegRec<T> *__restrict__ pool, int *__restrict__ pool_top) {
   if (act && !*act) return;  // batched sweep: suspension converged
-  __shared__ int s_pre[4][64], s_first[4][64];
+  __shared__ int s_pre[4][kListBins], s_first[4][kListBins];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int ntiles = G.nbx * G.nby * G.nbz;
   const int tile = blockIdx.x * 4 + wave;
@@ -475,26 +475,30 @@ __device__ __forceinline__ void d_tile_lists(const int *__restrict__ act, SG G,
             bz = tile / (G.nbx * G.nby);
   const int cx = min(G.hx + 1, G.nbx), cy = min(G.hy + 1, G.nby),
             cz = min(G.hz + 1, G.nbz);
-  const int nbins = cx * cy * cz;  // <= 64
-  int n = 0, f = 0;
-  if (lane < nbins) {
-    const int dz = lane / (cx * cy), dy = (lane / cx) % cy, dx = lane % cx;
-    const int ix = ((bx - G.hx + dx) % G.nbx + G.nbx) % G.nbx;
-    const int iy = ((by - G.hy + dy) % G.nby + G.nby) % G.nby;
-    const int iz = ((bz - G.hz + dz) % G.nbz + G.nbz) % G.nbz;
-    const int b = spread_bin(ix, iy, iz, G.nbx, G.nby, G.nbz);
-    f = start[b];
-    n = start[b + 1] - f;
-  }
-  int incl = n;
+  const int nbins = cx * cy * cz;  // <= kListBins
+  int total = 0;
+  for (int k0 = 0; k0 < nbins; k0 += 64) {
+    const int k = k0 + lane;
+    int n = 0, f = 0;
+    if (k < nbins) {
+      const int dz = k / (cx * cy), dy = (k / cx) % cy, dx = k % cx;
+      const int ix = ((bx - G.hx + dx) % G.nbx + G.nbx) % G.nbx;
+      const int iy = ((by - G.hy + dy) % G.nby + G.nby) % G.nby;
+      const int iz = ((bz - G.hz + dz) % G.nbz + G.nbz) % G.nbz;
+      const int b = spread_bin(ix, iy, iz, G.nbx, G.nby, G.nbz);
+      f = start[b];
+      n = start[b + 1] - f;
+    }
+    int incl = n;
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int t = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += t;
+    for (int off = 1; off < 64; off <<= 1) {
+      const int t = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += t;
+    }
+    pre[k] = total + incl - n;
+    first[k] = f;
+    total += __shfl(incl, 63, 64);
   }
-  const int total = __shfl(incl, 63, 64);
-  pre[lane] = incl - n;
-  first[lane] = f;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -721,8 +725,8 @@ __global__ void __launch_bounds__(1024)
 // (px0, py0, pz0). w[a] = g (monopole), w[32 + a] = gD (dipole), w[64 + a]
 // = its derivative h = gD (-xx / sigma_dip^2), zero off the stencil and past
 // the axis' end (a cut tile); xx is
-// formed in FP64, and so is the exponent (base 2); FP32 rounds it before the
-// hardware exp2.
+// formed in FP64, and so is the exponent (base 2). FP32 rounds it before the
+// hardware exp2, or (fine) rounds the FP64 weight, as the vector path does.
 // weights (96) + coefficients (6) per record; odd, so that 16 rows read at one
 // point fall on different banks
 constexpr int kTileW = 105;
@@ -744,8 +748,13 @@ __device__ __forceinline__ void tile_weights(const GaussConst &g,
       ga = g.anorm * exp2_neg(-x2 * g.e2);
       gd = g.anormdip * exp2_neg(-x2 * g.ed2);
     } else {
-      ga = (float)g.anorm * __builtin_amdgcn_exp2f((float)(-x2 * g.e2));
-      gd = (float)g.anormdip * __builtin_amdgcn_exp2f((float)(-x2 * g.ed2));
+      if (g.fine) {
+        ga = (float)(g.anorm * exp2_neg(-x2 * g.e2));
+        gd = (float)(g.anormdip * exp2_neg(-x2 * g.ed2));
+      } else {
+        ga = (float)g.anorm * __builtin_amdgcn_exp2f((float)(-x2 * g.e2));
+        gd = (float)g.anormdip * __builtin_amdgcn_exp2f((float)(-x2 * g.ed2));
+      }
     }
     h = gd * (T)(xx * g.nrsd);
   }
@@ -2065,8 +2074,10 @@ static int direct_parts(const SpreadGeom &g) {
 }
 
 // Gaussian constants of the spread, tables and interpolation.
-static GaussConst gauss_const(const fs_fcm_params &p) {
+static GaussConst gauss_const(const FcmImpl &f) {
+  const fs_fcm_params &p = f.p;
   GaussConst g;
+  g.fine = f.fine;
   g.dx = p.dx;
   double sigmadipsq = p.sigma_dip * p.sigma_dip;
   g.sigmadipsq = sigmadipsq;
@@ -2103,7 +2114,7 @@ static ProjConst proj_const(const fs_fcm_params &p) {
 template <typename T>
 int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
                  double *V, double *W, hipStream_t st) {
-  const GaussConst g = gauss_const(p);
+  const GaussConst g = gauss_const(*this);
 
   hipEvent_t *pset = nullptr;  // this solve's profiling events
   if (prof) {
@@ -2355,7 +2366,7 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
     }
     return static_cast<const char *>(G.tab.p) + G.off[k++];
   };
-  const GaussConst g = gauss_const(p);
+  const GaussConst g = gauss_const(f0);
   const ProjConst pc = proj_const(p);
   const double dx3 = p.dx * p.dx * p.dx;
   if (f0.direct) {
