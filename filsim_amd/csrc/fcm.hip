@@ -6,7 +6,8 @@
 //   bin       counting sort of segments by the grid tile holding their
 //             stencil origin (deterministic order inside a bin); on the
 //             matrix-core path each tile then gets the records of the
-//             segments whose stencil meets it (k_tile_lists)
+//             segments whose stencil meets it (k_tile_lists); few segments
+//             take one launch for both, without bins (k_tile_lists_direct)
 //   spread    gather form of mono_and_dipole_force_distribution
 //             (:596-646): one workgroup per grid tile sums, in a fixed
 //             order, every segment whose stencil covers the tile, then
@@ -17,7 +18,7 @@
 //   fft_y     strided complex FFT along y (forward)
 //   fft_x_prj forward FFT along x, the Stokes projection of flow_solve
 //             (:648-736), inverse FFT along x -- three components resident
-//             in LDS, so the spectrum makes one round trip through HBM
+//             on chip, so the spectrum makes one round trip through HBM
 //   fft_y     inverse along y
 //   fft_z_c2r half-complex->real along z
 //   interp    particle_velocities + particle_rotations (:740-808) fused:

@@ -15,6 +15,8 @@
 //             normalised output
 //   backward  g = BF16(dL/dz) feeds both MFMA products (dW = g^T h,
 //             dh = g W); bias gradients from the FP32 dL/dz
+//   inference in one launch up to 2 Mi weights (k_mlp_forward), the same
+//             rounding points
 //   optimiser Adam on FP32 master weights (beta 0.9/0.999, eps 1e-8)
 #include <hip/hip_runtime.h>
 
