@@ -243,15 +243,7 @@ int FcmImpl::set_geometry() {
     FS_TRY(tpool.alloc((size_t)max_np * nslot * rec_bytes(tsz)));
     grid_interp = tsz == 8 ? interp_blocks<double>(*this) : interp_blocks<float>(*this);
   }
-  // Lists without bins where every row of tiles can look at all segments. Both
-  // sides in us, of all launches that make the lists, binned and direct: 240
-  // segments on 64^3 (32 row steps) 31 and 16; 3,600 on 128^3 (512) 43 and 26;
-  // 2,400 on 192^3 (864) 37 and 28, growing with the row steps.
-  direct = mfma_spread && max_np <= kDirectMax &&
-           (long)ceil_div(max_np, 1024) * geom.nby * geom.nbz <= kDirectRowSteps;
-  // FP64 weights cost nothing where launches and latency bound the tile kernels;
-  // on cut grids the vector gather, which takes them too, was the other way
-  fine = direct || rx || ry || rz;
+  cut = mfma_spread && (rx || ry || rz);
   // one more counter after the bins: the tile lists' pool top
   FS_TRY(bin_count.alloc((size_t)(nbins + 1) * sizeof(int)));
   FS_HIP(hipMemset(bin_count.p, 0, (size_t)(nbins + 1) * sizeof(int)));
@@ -280,6 +272,19 @@ int FcmImpl::set_geometry() {
                x_threads(plx, xQ) <= x_max,
            FS_ERR_ARG, "no FFT workgroup shape fits %dx%dx%d", p.nx, p.ny, p.nz);
   return FS_OK;
+}
+
+// Lists without bins where every row of tiles can look at all segments. Both
+// sides in us, of all launches that make the lists, binned and direct: 240
+// segments on 64^3 (32 row steps) 31 and 16; 3,600 on 128^3 (512) 43 and 26;
+// 2,400 on 192^3 (864) 37 and 28, growing with the row steps. The way depends on
+// the solve's own segments, so that its results do not change with the
+// capacity of the handle. FP64 weights (fine_weights) cost nothing where
+// launches and latency bound the tile kernels; on cut grids the vector gather,
+// which takes them too, was the other way.
+bool FcmImpl::lists_direct(int np) const {
+  return mfma_spread && np <= kDirectMax &&
+         (long)ceil_div(np, 1024) * geom.nby * geom.nbz <= kDirectRowSteps;
 }
 
 void FcmImpl::release() {
@@ -314,18 +319,19 @@ void FcmImpl::release() {
   prof_used = 0;
 }
 
-bool fcm_same_shapes(const FcmImpl &a, const FcmImpl &b) {
+bool fcm_same_shapes(const FcmGroupMember &ma, const FcmGroupMember &mb) {
+  const FcmImpl &a = *ma.fcm, &b = *mb.fcm;
   return a.precision == b.precision && a.p.nx == b.p.nx && a.p.ny == b.p.ny &&
          a.p.nz == b.p.nz && a.p.ngd == b.p.ngd && a.mfma_spread && b.mfma_spread &&
          a.zP == b.zP && a.yB == b.yB && a.xQ == b.xQ &&
          a.grid_interp == b.grid_interp && a.nbins == b.nbins &&
-         a.direct == b.direct;
+         a.lists_direct(ma.np) == b.lists_direct(mb.np);
 }
 
 int FcmGroup::build() {
   FS_CHECK(!m.empty(), FS_ERR_ARG, "empty FCM group");
   for (auto &x : m)
-    FS_CHECK(fcm_same_shapes(*m[0].fcm, *x.fcm) && x.np >= 1 &&
+    FS_CHECK(fcm_same_shapes(m[0], x) && x.np >= 1 &&
                  x.np <= x.fcm->max_np,
              FS_ERR_ARG, "FCM group members differ in launch shapes or sizes");
   std::vector<char> host;

@@ -37,8 +37,7 @@ struct FcmImpl {
   SpreadGeom geom{};
   int nbins = 0;
   bool mfma_spread = false;  // spread on the matrix cores (8 x 8 x 16 tiles)
-  bool direct = false;  // tile lists straight from the segments, without bins
-  bool fine = false;    // FP32 tile weights formed in FP64
+  bool cut = false;  // the last tiles of an axis are cut off
   int grid_interp = 0;  // blocks of the persistent interpolation
   int zP = 1, yB = 1, xQ = 1;  // FFT pass workgroup shapes
   // device flag read by every kernel of a solve: 0 = skip (a converged
@@ -57,6 +56,10 @@ struct FcmImpl {
 
   int init(const fs_fcm_params &pp, int maxnp, int prec);
   int set_geometry();
+  // whether a solve of np segments makes its tile lists straight from the
+  // segments, without bins, and whether it forms FP32 tile weights in FP64
+  bool lists_direct(int np) const;
+  bool fine_weights(int np) const { return cut || lists_direct(np); }
   void release();
   int mobility(int np, const double *Y, const double *F, const double *Tq,
                double *V, double *W, hipStream_t st);
@@ -91,6 +94,6 @@ struct FcmGroup {
   int solve(hipStream_t st);
   void release() { tab.release(); }
 };
-bool fcm_same_shapes(const FcmImpl &a, const FcmImpl &b);
+bool fcm_same_shapes(const FcmGroupMember &a, const FcmGroupMember &b);
 
 }  // namespace fs

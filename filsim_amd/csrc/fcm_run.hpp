@@ -1871,8 +1871,8 @@ __device__ __forceinline__ void d_interp_sum(const int *__restrict__ act, int np
   constexpr int NSLOT = kInterpSlots<NGD>;
   if (act && !*act) return;  // batched sweep: suspension converged
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  // lists without bins: the pool's counter for the next solve
-  if (pool_top && e == 0) *pool_top = 0;
+  // the pool's counter for the next solve
+  if (e == 0) *pool_top = 0;
   const int s = e / 6, m = e - 6 * s;
   if (s >= np) return;
   const int ox = origin[3 * s], oy = origin[3 * s + 1], oz = origin[3 * s + 2];
@@ -2074,10 +2074,10 @@ static int direct_parts(const SpreadGeom &g) {
 }
 
 // Gaussian constants of the spread, tables and interpolation.
-static GaussConst gauss_const(const FcmImpl &f) {
+static GaussConst gauss_const(const FcmImpl &f, int np) {
   const fs_fcm_params &p = f.p;
   GaussConst g;
-  g.fine = f.fine;
+  g.fine = f.fine_weights(np);
   g.dx = p.dx;
   double sigmadipsq = p.sigma_dip * p.sigma_dip;
   g.sigmadipsq = sigmadipsq;
@@ -2114,7 +2114,7 @@ static ProjConst proj_const(const fs_fcm_params &p) {
 template <typename T>
 int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
                  double *V, double *W, hipStream_t st) {
-  const GaussConst g = gauss_const(*this);
+  const GaussConst g = gauss_const(*this, np);
 
   hipEvent_t *pset = nullptr;  // this solve's profiling events
   if (prof) {
@@ -2142,7 +2142,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   mark(0);
   kmark(0);
   const int ntiles = nbins;
-  if (direct) {
+  if (lists_direct(np)) {
     kmark(1);
     hipLaunchKernelGGL(k_tile_lists_direct<T>,
                        dim3(geom.nby * geom.nbz, direct_parts(geom)), dim3(1024), 0, st, act, np, geom, p.dx, Y, F, Tq,
@@ -2267,7 +2267,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
       hipLaunchKernelGGL((k_interp_sum<T, NG>), dim3(ceil_div(6L * np, 256)),
                          dim3(256), 0, st, act, np, geom, dx3,
                          origin.as<int>(), ipart.as<T>(), V, W,
-                         direct ? bin_count.as<int>() + nbins : (int *)nullptr);
+                         bin_count.as<int>() + nbins);
     } else {
       hipLaunchKernelGGL((k_interp<T, NG>),
                          dim3(8 * ceil_div(ceil_div(np, 4), 8)), dim3(256), 0,
@@ -2366,10 +2366,10 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
     }
     return static_cast<const char *>(G.tab.p) + G.off[k++];
   };
-  const GaussConst g = gauss_const(f0);
+  const GaussConst g = gauss_const(f0, G.m[0].np);
   const ProjConst pc = proj_const(p);
   const double dx3 = p.dx * p.dx * p.dx;
-  if (f0.direct) {
+  if (f0.lists_direct(G.m[0].np)) {
     auto t = table([&](const FcmGroupMember &m) {
       const FcmImpl &f = *m.fcm;
       return A_tile_lists_direct<T>{
@@ -2524,8 +2524,7 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
       const FcmImpl &f = *m.fcm;
       return A_interp_sum<T, NG>{m.act, m.np, f.geom, dx3, f.origin.as<int>(),
                                  f.ipart.as<T>(), m.V, m.W,
-                                 f.direct ? f.bin_count.as<int>() + nbins
-                                          : (int *)nullptr};
+                                 f.bin_count.as<int>() + nbins};
     });
     if (!host)
       hipLaunchKernelGGL((k_interp_sum_multi<T, NG>),

@@ -701,7 +701,7 @@ int batch_build_fcm(fs_batch *b, int kind) {
     m.W = S.d.W;
     fs::FcmGroup *g = nullptr;
     for (fs::FcmGroup &x : groups)
-      if (fs::fcm_same_shapes(*x.m[0].fcm, S.fcm)) g = &x;
+      if (fs::fcm_same_shapes(x.m[0], m)) g = &x;
     if (!g) {
       groups.emplace_back();
       g = &groups.back();

@@ -40,6 +40,23 @@ def test_lists_match_vector_path(cuda, grid, n, spread):
             assert np.linalg.norm(W - Wo) <= 1e-12 * top, k
 
 
+@pytest.mark.parametrize("prec", [abi.FS_FP64, abi.FS_FP32])
+def test_results_do_not_depend_on_capacity(cuda, prec):
+    """A handle for 5,000 segments, which solves few segments without bins and
+    many through them, against handles made for each count: the same bits, in
+    turn, so that neither way sees what the other left (crowded tiles: both
+    fill the lists' pool)."""
+    fp = params.fcm_params((64, 32, 48))
+    Y, F, T = random_segments(fp, 5000, seed=11)
+    Y *= 0.5
+    with api.Fcm(fp, 5000, precision=prec) as big:
+        for n in (300, 5000, 4096, 4097, 300):
+            V, W = big.mobility_host(Y[:n], F[:n], T[:n])
+            with api.Fcm(fp, n, precision=prec) as own:
+                Vo, Wo = own.mobility_host(Y[:n], F[:n], T[:n])
+            assert np.array_equal(V, Vo) and np.array_equal(W, Wo), n
+
+
 def test_binned_groups_equal_unbatched(cuda):
     """Two suspensions of more segments than the way without bins takes,
     stepped with fused stages and one after another: the same bits."""
