@@ -1372,8 +1372,8 @@ __global__ void k_broyden_cols(const double *__restrict__ tmp,
 // reference's second solve H_k dE equals g - Update, so its column
 // C_k = (-H_k dE - Update)/|dE| = -g/|dE|, D_k = dE/|dE|, and the next
 // update H_{k+1} E_new = g + C_k (D_k . E_new) = g (1 - dE.E_new/|dE|^2).
-// Columns col of C and D (column stride n); with iterp, col = *iterp - 1. Each
-// workgroup adds the nblk partial sums of |dE|^2 and dE.E_new itself (a fixed
+// Columns col of C and D (column stride n); with iterp, col = *iterp - 1. Every
+// wavefront adds the nblk partial sums of |dE|^2 and dE.E_new itself (a fixed
 // order), 6 loads a lane at 30k segments.
 __global__ void k_broyden_fused(const int *__restrict__ act,
                                 const double *__restrict__ g,
@@ -2009,6 +2009,34 @@ int SystemImpl::broyden_update(const double *Eo, const double *En,
   return FS_OK;
 }
 
+// Partial sums up to which every wavefront of k_broyden_fused adds them itself;
+// above, where that costs the square of the system's size, a launch does. An
+// iteration without its mobility solve in us, themselves and by a launch: 30,000
+// segments (352 sums) 74.8 and 77.7, 120,000 (1,407) 193.8 and 194.0, 180,000
+// (2,110) 284 and 278, 960,000 (11,250) 1,670 and 1,303.
+constexpr int kStepSums = 1536;
+
+// Broyden column and next update from g (tmp), the differences dE and their
+// partial sums (diffp); column col, or *iterp - 1 of the device.
+int SystemImpl::broyden_fused(int col, const int *iterp) {
+  ProfScope ps_(*this, P_SLVJ);
+  const size_t n6 = 6 * (size_t)np;
+  const double *sums = diffp.as<double>();
+  int nsum = diff_blocks;
+  if (nsum > kStepSums) {
+    double *dots = coefb.as<double>() + hcols;
+    hipLaunchKernelGGL(k_dots_final, dim3(2), dim3(64), 0, st, d.act, sums, nsum,
+                       2, 2, (const int *)nullptr, 0, dots);
+    sums = dots;
+    nsum = 1;
+  }
+  hipLaunchKernelGGL(k_broyden_fused, dim3(ceil_div((long)n6, 256)), dim3(256),
+                     0, st, d.act, tmp, dE, sums, nsum, n6, Cm.as<double>(),
+                     Dm.as<double>(), col, iterp, Upd);
+  FS_LAUNCHED();
+  return FS_OK;
+}
+
 int SystemImpl::residual(int nt, const double *V, const double *W, double *err,
                          int *check, double *maxabs) {
   hipLaunchKernelGGL(k_resid_reset, dim3(1), dim3(1), 0, st, d.act,
@@ -2167,13 +2195,7 @@ int SystemImpl::broyden_loop(int nt, int *iters) {
     // behind it.
     if (iter < p.broyden_maxiter) {
       FS_TRY(jsolve(NewE, tmp, h0 + iter - 1, E));
-      ProfScope ps_(*this, P_SLVJ);
-      hipLaunchKernelGGL(k_broyden_fused, dim3(ceil_div((long)n6, 256)),
-                         dim3(256), 0, st, (const int *)nullptr, tmp, dE,
-                         diffp.as<double>(), diff_blocks, n6, Cm.as<double>(),
-                         Dm.as<double>(), h0 + iter - 1, (const int *)nullptr,
-                         Upd);
-      FS_LAUNCHED();
+      FS_TRY(broyden_fused(h0 + iter - 1, nullptr));
     }
     FS_TRY(residual_wait(&check, &last_res));
     if (!check || iter >= p.broyden_maxiter) break;
@@ -2274,9 +2296,7 @@ int SystemImpl::iteration_dev(int *status, int part) {
   hipLaunchKernelGGL(k_ctl_after, dim3(1), dim3(1), 0, st, ctl.as<int>(), mb,
                      p.tol, p.broyden_maxiter);
   FS_TRY(jsolve_impl(NewE, tmp, 0, ctl.as<int>(), -1, E));
-  hipLaunchKernelGGL(k_broyden_fused, dim3(ceil_div((long)n6, 256)), dim3(256),
-                     0, st, act, tmp, dE, diffp.as<double>(), diff_blocks, n6,
-                     Cm.as<double>(), Dm.as<double>(), 0, ctl.as<int>(), Upd);
+  FS_TRY(broyden_fused(0, ctl.as<int>()));
   hipLaunchKernelGGL(k_copy_f64, dim3(ceil_div((long)n6, 256)), dim3(256), 0, st,
                      act, NewE, E, n6);
   set_device_control(nullptr, ntp);

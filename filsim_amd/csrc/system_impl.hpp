@@ -74,6 +74,7 @@ struct SystemImpl {
   int build_jacobian(int nt, bool clear_history = true);
   // Eo: also the Broyden differences dE = b - Eo
   int jsolve(const double *b, double *x, int iter, const double *Eo = nullptr);
+  int broyden_fused(int col, const int *iterp);
   int jinv_dense(int f, double *out);
   int broyden_update(const double *Eo, const double *En, const double *upd,
                      int iter);

@@ -1,11 +1,11 @@
-"""The Broyden history's coefficients on both sides of the line at which they
-are added up where they are used."""
+"""The Broyden step's sums on both sides of the lines at which they are added up
+where they are used."""
 import numpy as np
 import pytest
 
 from helpers import rel, to_dev
 from sysfix import config
-from filsim_amd import api
+from filsim_amd import api, params
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +44,30 @@ def test_solve_with_history(cuda, nfil):
                          to_dev(torch, upd), it)
         cols.append((C, D))
         assert rel(solve(bs[3], it + 1), expect(bs[3])) <= 1e-12
+
+
+@pytest.mark.parametrize("nfil", [4369, 4370])  # 1,536 and 1,537 partial sums
+def test_step_sums(cuda, nfil):
+    """Four Broyden iterations of equal filaments that do not meet: the sums
+    over all of them are nfil times one filament's, so every filament moves as
+    it does alone. 1e-10 of the displacement covers the sums' rounding (1e-13
+    for a million terms) over four iterations; one sum left out is 6e-4."""
+    nw = 30
+    fp = params.fcm_params(64)
+    sp = params.sim_params(fp, dt=0.005, tol=1e-300, maxiter=4, barrier_on=0,
+                           initial_friction_steps=10)
+    line = np.array([5., 5, 5]) + 2.2 * np.arange(nw)[:, None] * np.array(
+        [1., 0, 0])
+
+    def moved(n):
+        with api.System(sp, [nw] * n,
+                        params.swimming_props(n, nw, phases=[0.3] * n)) as s:
+            X = np.tile(line, (n, 1))
+            q = np.tile([1., 0, 0, 0], (n * nw, 1))
+            s.set_state(X=X, Xs=X, Xt=X, q=q, qs=q, qt=q)
+            assert s.timestep(1) == 4
+            return (s.get_state()["X"] - X).reshape(n, nw, 3)
+
+    one, many = moved(1)[0], moved(nfil)
+    top = np.abs(one).max()
+    assert top > 0 and np.abs(many - one).max() <= 1e-10 * top
