@@ -22,6 +22,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -57,8 +58,9 @@ enum { EPI_STORE = 0, EPI_HIDDEN = 1, EPI_OUT = 2, EPI_DRELU = 3, EPI_ADD = 4 };
 //            OUT    Cf = acc + bias
 //            DRELU  g = acc * (Zf > 0): Cf = g, Hb = BF16(g)
 //            ADD    Cf += acc
-// Bound by the latency of the loads: those of kGemmAhead steps go out together.
-constexpr int kGemmAhead = 4;
+// Bound by the latency of the loads: those of 4 steps go out together, what is
+// left of a wavefront's steps by 2 and 1 (K = 64, one step a wavefront: 4.3 us;
+// always 4 steps, with zeros past the end, 5.9 us).
 template <bool AV, bool BV>
 __global__ void __launch_bounds__(256)
     k_gemm_bf16(int M, int N, int K, const uint16_t *__restrict__ A, long sam,
@@ -79,12 +81,13 @@ __global__ void __launch_bounds__(256)
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f4v{0.f, 0.f, 0.f, 0.f};
-  for (int sb = s0; sb < s1; sb += kGemmAhead) {
-    s4v a[kGemmAhead][2], b[kGemmAhead][2];
+  // steps sb .. sb + AH - 1
+  const auto steps = [&](auto ahead, int sb) {
+    constexpr int AH = decltype(ahead)::value;
+    s4v a[AH][2], b[AH][2];
 #pragma unroll
-    for (int u = 0; u < kGemmAhead; ++u) {
-      // past the wave's steps k is K: zeros
-      const int k = sb + u < s1 ? 16 * (sb + u) + kq : K;
+    for (int u = 0; u < AH; ++u) {
+      const int k = 16 * (sb + u) + kq;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int m = m0 + 16 * i + r;
@@ -113,16 +116,21 @@ __global__ void __launch_bounds__(256)
       }
     }
 #pragma unroll
-    for (int u = 0; u < kGemmAhead; ++u)
-      if (sb + u < s1) {
+    for (int u = 0; u < AH; ++u)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                a[u][i], b[u][j], acc[i][j], 0, 0, 0);
-      }
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+              a[u][i], b[u][j], acc[i][j], 0, 0, 0);
+  };
+  int s = s0;
+  for (; s + 4 <= s1; s += 4) steps(std::integral_constant<int, 4>{}, s);
+  if (s + 2 <= s1) {
+    steps(std::integral_constant<int, 2>{}, s);
+    s += 2;
   }
+  if (s < s1) steps(std::integral_constant<int, 1>{}, s);
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -372,7 +380,8 @@ __global__ void __launch_bounds__(256)
 // wavefronts per 64 columns, wavefront w adds the w-th contiguous sixteenth
 // of the rows (one coalesced row segment per load), then the 16 partial
 // sums are added in wavefront order. Few workgroups, so bound by the latency
-// of the loads: 16 of them are in flight.
+// of the loads: 16 of them are in flight, of the last rows 8 (1,000 rows by 256
+// 4.7 us; the last rows one by one 7.9 us).
 __global__ void __launch_bounds__(1024)
     k_colsum(const float *__restrict__ g, int rows, int cols,
              float *__restrict__ out) {
@@ -391,7 +400,14 @@ __global__ void __launch_bounds__(1024)
 #pragma unroll
       for (int j = 0; j < 16; ++j) s += v[j];
     }
-    for (; r < r1; ++r) s += g[(long)r * cols + c];
+    for (; r < r1; r += 8) {
+      float v[8];  // the last row's again past the end
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = g[(long)min(r + j, r1 - 1) * cols + c];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (r + j < r1) s += v[j];
+    }
   }
   part[w][lane] = s;
   __syncthreads();

@@ -77,6 +77,27 @@ def test_gradients_match_oracle(cuda):
         o += n
 
 
+@pytest.mark.parametrize("rows", [1, 15, 17, 64, 65, 128, 129, 257, 400])
+@pytest.mark.parametrize("n_in,width,n_out", [(30, 16, 5), (84, 112, 52)])
+def test_gradients_at_step_edges(cuda, rows, n_in, width, n_out):
+    """Sums over rows, inputs and widths of none to seven steps of 16 a
+    wavefront, whole and in part, and column sums of 0 to 25 rows a wavefront.
+    Every weight block and bias on its own: 1e-2 of its norm, for hidden values
+    that FP32 sums round to the other BF16 neighbour (2^-8); one row left out
+    of 400 is 5e-2."""
+    mlp, X, T, dX, dT, mu, sig, tau = _net(cuda, n_in, n_out, width, rows,
+                                           seed=rows)
+    loss, g = mlp.gradients(dX, dT)
+    lo, go = M.loss_and_grad(mlp.get_params(), mlp.dims, X, T, mu, sig, tau)
+    assert abs(loss - lo) < 1e-2 * lo
+    o = 0
+    for a, b in zip(mlp.dims, mlp.dims[1:]):
+        for n in (a * b, b):
+            e = np.linalg.norm(g[o:o + n] - go[o:o + n])
+            assert e <= 1e-2 * np.linalg.norm(go[o:o + n]), (a, b, n)
+            o += n
+
+
 def test_training_reduces_loss(cuda):
     torch = cuda
     rng = np.random.default_rng(4)
