@@ -20,6 +20,7 @@
 //   optimiser Adam on FP32 master weights (beta 0.9/0.999, eps 1e-8)
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <type_traits>
@@ -460,6 +461,18 @@ __global__ void k_adam(float *__restrict__ w, const float *__restrict__ g,
 // Mi values) 15 and 16, 36 and 46; 768 wide (2.0 Mi) 44 and 47, 47 and 85;
 // 1,024 wide (3.0 Mi) 73 and 67, 52 and 115.
 constexpr long kMlpFusedWeights = 2 << 20;
+// Packed values in use below which many rows go layer by layer: a workgroup of
+// 16 wavefronts has work for one to four of them in so narrow a net, so its time
+// is the rows'. The line in rows follows the measured crossings, one launch and
+// layer by layer in us: 28-16-16-16-12 (2 Ki values) 30,000 rows 24 and 25,
+// 40,000 29 and 27, 200,000 130 and 81; with a skip map 60,000 42 and 48, 100,000
+// 68 and 63; 28-64-64-64-12 (11 Ki) 60,000 54 and 62, 200,000 171 and 151;
+// 92-64-64-64-24 (16 Ki) 200,000 193 and 199.
+constexpr long kMlpNarrow = 14 << 10;
+inline long mlp_fused_rows(long values, bool skip) {
+  return values >= kMlpNarrow ? LONG_MAX
+                              : 20480 + 8 * values + (skip ? 40960 : 0);
+}
 
 struct MlpImpl {
   int nin = 0, width = 0, nout = 0;
@@ -629,12 +642,15 @@ struct MlpImpl {
   }
   // Whether inference goes in one launch. Every workgroup reads all weights,
   // so nets beyond kMlpFusedWeights go layer by layer, where workgroups share
-  // them out. Its outputs must not lie over inputs that another workgroup has
-  // yet to read.
+  // them out, and so do many rows of narrow nets. Its outputs must not lie over
+  // inputs that another workgroup has yet to read.
   bool fused(int B, const float *X, const float *Yout) const {
     const uintptr_t x = (uintptr_t)X, y = (uintptr_t)Yout;
-    return net.packed && (x + sizeof(float) * (size_t)B * nin <= y ||
-                          y + sizeof(float) * (size_t)B * nout <= x);
+    const long values =
+        net.poff[4] + (has_skip ? mlp_packed_size(nin, nout) : 0);
+    return net.packed && B <= mlp_fused_rows(values, has_skip) &&
+           (x + sizeof(float) * (size_t)B * nin <= y ||
+            y + sizeof(float) * (size_t)B * nout <= x);
   }
   size_t fused_lds() const {
     return sizeof(uint16_t) * kMlpRows *

@@ -59,3 +59,27 @@ def test_forward_at_tile_edges(cuda, rows, n_in, width, n_out):
         mlp.forward(dX, Z)
         keep = [r for r in range(rows) if r not in (rows // 2, rows - 1)]
         assert torch.equal(Z[keep], Y[keep])
+
+
+@pytest.mark.parametrize("skip,rows", [(False, 36864), (False, 36865),
+                                       (True, 81920), (True, 81921)])
+def test_many_rows_of_a_narrow_net(cuda, skip, rows):
+    """The most rows in one launch and the fewest by layers, of the narrowest
+    net. Bound as above."""
+    torch = cuda
+    rng = np.random.default_rng(rows)
+    n_in, n_out = 28, 12
+    mlp = api.Mlp(n_in, n_out, width=16, seed=3)
+    S = rng.standard_normal((n_out, n_in)) * 0.05 if skip else None
+    if skip:
+        mlp.set_skip(S)
+    one, zero = np.ones(n_in, np.float32), np.zeros(n_in, np.float32)
+    X = rng.standard_normal((rows, n_in)).astype(np.float32)
+    Yo, _, _, _ = M.forward(mlp.get_params(), mlp.dims, X, zero, one,
+                            np.ones(n_out, np.float32), skip=S)
+    Y = torch.full((rows, n_out), 7.0, dtype=torch.float32, device="cuda")
+    mlp.forward(torch.tensor(X, device="cuda"), Y)
+    Y = Y.cpu().numpy()
+    assert np.linalg.norm(Y - Yo) < 2e-3 * np.linalg.norm(Yo)
+    for r in (0, 15, 16, rows - 1):
+        assert np.linalg.norm(Y[r] - Yo[r]) < 2e-2 * np.linalg.norm(Yo[r]), r
