@@ -80,6 +80,35 @@ def test_more_than_a_million_cells(cuda):
     gb.close()
 
 
+@pytest.mark.parametrize("stride", [1, 16, 17, 40])
+def test_neighbours_numbered_apart(cuda, stride):
+    """Filaments of 15 segments whose neighbours along the filament are
+    numbered `stride` apart, near and far: the pairs that neighbours of one
+    filament are left out of, and the forces, as the oracle's."""
+    torch = cuda
+    fp = params.fcm_params(64)
+    cp = params.colbar_params(fp)
+    X, sf, si = _system(fp, 40, 15, seed=6)
+    order = np.argsort(sf // stride * 10**6 + si * 10**3 + sf % stride)
+    X, sf, si = X[order], sf[order], si[order]
+    at = np.flatnonzero((sf == 0) & (si < 2))
+    assert at[1] - at[0] == stride
+    rng = np.random.default_rng(stride)
+    Xs = X + rng.normal(0, 0.6, X.shape)
+    Y = np.fmod(Xs, np.array(params.box(fp)))
+    ob, gb = O.Colbar(cp, sf, si), api.Colbar(cp, sf, si)
+    ob.link(Xs)
+    gb.link(to_dev(torch, Xs))
+    p_o = ob.pairs(Y, 1)
+    assert np.array_equal(gb.pairs(to_dev(torch, Y), 1), p_o)
+    assert np.array_equal(p_o, O.pairs_brute(cp, Y, sf, si, 1))
+    Fo, md_o = ob.apply(Y, 1, np.zeros_like(Y))
+    dF = torch.zeros(Y.shape, dtype=torch.float64, device="cuda")
+    assert gb.apply(to_dev(torch, Y), 1, dF) == md_o
+    assert rel(dF.cpu().numpy(), Fo) <= 1e-12
+    gb.close()
+
+
 def test_stale_list(cuda):
     """Between links the list is reused even after segments move
     (main.cpp:394 vs :565)."""
