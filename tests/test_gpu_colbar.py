@@ -80,6 +80,26 @@ def test_more_than_a_million_cells(cuda):
     gb.close()
 
 
+def test_more_than_four_million_cells(cuda):
+    """172^3 cells: the cell-count scan runs over more than 4,096 blocks, whose
+    sums a launch scans first. Two links, the second of moved segments, which
+    sees the counts that the first left."""
+    torch = cuda
+    fp = params.fcm_params(800)
+    cp = params.colbar_params(fp)
+    X, sf, si = _system(params.fcm_params(64), 40, 15, seed=3)
+    ob, gb = O.Colbar(cp, sf, si), api.Colbar(cp, sf, si)
+    for shift in (0.0, 391.0):  # the second across the box's faces
+        Xs = X + shift
+        ob.link(Xs)
+        gb.link(to_dev(torch, Xs))
+        h_o, l_o = ob.lists()
+        h_g, l_g = gb.lists()
+        assert len(h_o) > 4096 * 1024
+        assert np.array_equal(h_g, h_o) and np.array_equal(l_g, l_o)
+    gb.close()
+
+
 @pytest.mark.parametrize("stride", [1, 16, 17, 40])
 def test_neighbours_numbered_apart(cuda, stride):
     """Filaments of 15 segments whose neighbours along the filament are

@@ -2,6 +2,7 @@
 import numpy as np
 import pytest
 
+import _oracle as O
 from filsim_amd import abi, api, params
 from helpers import random_segments, rel
 
@@ -60,12 +61,25 @@ def test_results_do_not_depend_on_capacity(cuda, prec):
 def test_binned_groups_equal_unbatched(cuda):
     """Two suspensions of more segments than the way without bins takes,
     stepped with fused stages and one after another: the same bits."""
+    _groups_equal_unbatched((160,), (260, 270), (18, 20), (4097, 10**6))
+
+
+@pytest.mark.parametrize("grid,nfil,nw,segments", [
+    (50, (20, 24), (10, 12), (1, 4096)),       # without bins
+    (150, (240, 250), (18, 20), (4097, 10**6)),  # through bins
+])
+def test_groups_on_cut_grids_equal_unbatched(cuda, grid, nfil, nw, segments):
+    """The same on grids whose last tiles are cut off."""
+    _groups_equal_unbatched((grid,), nfil, nw, segments)
+
+
+def _groups_equal_unbatched(grids, nfil, nw, segments):
     solo, bat = [], []
     for seed in (1, 2):
         fp, sp, nws, props, st, info = params.sweep_point(
-            seed, grids=(160,), nfil_range=(260, 270), nw_range=(18, 20),
+            seed, grids=grids, nfil_range=nfil, nw_range=nw,
             precision=abi.FS_FP32, tol=1e-4, dt=0.01)
-        assert info["segments"] > 4096
+        assert segments[0] <= info["segments"] <= segments[1]
         for group in (solo, bat):
             s = api.System(sp, nws, props)
             s.set_state(**st)
@@ -102,3 +116,32 @@ def test_cut_tiles_match_vector_path(cuda, ngd):
             top = max(np.linalg.norm(Wo), np.linalg.norm(Vo) / fp.a)
             assert rel(V, Vo) <= bar, (grid, prec)
             assert np.linalg.norm(W - Wo) <= bar * top, (grid, prec)
+
+
+@pytest.mark.parametrize("ngd", [12, 20, 24])
+@pytest.mark.parametrize("grid", [(50, 90, 80), (54, 36, 90), (90, 100, 54)])
+def test_cut_tiles_through_bins(cuda, grid, ngd):
+    """More segments than the way without bins takes: one bin more on a cut
+    axis (up to 100 bins a tile, two steps of 64), pool blocks of crowded
+    tiles, and a second solve after the segments moved. Against the vector path
+    or, where that has no tile for the grid, the FP64 oracle; bounds as
+    above."""
+    fp = params.fcm_params(grid, ngd=ngd)
+    n = 4500
+    Y, F, T = random_segments(fp, n, seed=sum(grid) + ngd)
+    box = np.array(params.box(fp))
+    Y[n // 2:] *= 0.3  # half of them crowded
+    moved = [Y, np.mod(Y + 0.47 * box, box)]
+    with api.Fcm(fp, n) as vec:
+        try:
+            vec.set_tuning(spread_mfma=0)
+            ref = [vec.mobility_host(Yk, F, T) for Yk in moved]
+        except abi.FsError:
+            ref = [O.mobility(fp, Yk, F, T) for Yk in moved]
+    for prec, bar in ((abi.FS_FP64, 1e-12), (abi.FS_FP32, 1e-5)):
+        with api.Fcm(fp, n, precision=prec) as fcm:
+            for k, (Vo, Wo) in enumerate(ref):
+                V, W = fcm.mobility_host(moved[k], F, T)
+                top = max(np.linalg.norm(Wo), np.linalg.norm(Vo) / fp.a)
+                assert rel(V, Vo) <= bar, (prec, k)
+                assert np.linalg.norm(W - Wo) <= bar * top, (prec, k)
