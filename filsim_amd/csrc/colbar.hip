@@ -174,8 +174,8 @@ __device__ __forceinline__ CbRow cb_row(const CbGeom &g, int cx, int cy, int cz,
   return r;
 }
 
-// mode 0: F[i] += sum of pair forces, min distance (min_bits may be null); mode 1: count pairs
-// (i<j) inside the cutoff into *npairs and write them when room.
+// mode 0: F[i] += sum of pair forces, min distance (min_bits may be null); mode
+// 1: count pairs (i<j) inside the cutoff into *npairs and write them when room.
 // Bound by the latency of dependent loads (row starts, id, position): the
 // kCbLanes lanes of a segment look up its 9 rows of three cells together, lay
 // their entries end to end and take every kCbLanes-th each, so the usual

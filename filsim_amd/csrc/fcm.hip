@@ -62,9 +62,6 @@ static __global__ void k_friction(const int *__restrict__ act, int n3, const dou
   }
 }
 
-
-static int largest_divisor_le(int n, int t);
-
 static bool good_size(int n) {
   if (n < 2 || n > 1024 || (n & 1)) return false;
   FftPlan p;

@@ -584,10 +584,11 @@ __global__ void __launch_bounds__(256)
 }
 
 // The tile lists of few segments without bins: one workgroup per row of tiles
-// along x (where the rows are few, several, each with a part of the tiles). Its threads form every segment's origin and keep, in ascending
-// order, those whose stencil meets the row in y and z; then each wavefront
-// fills the lists of tiles of the row (order, slab, pool and counts as above,
-// except that a tile's segments are in ascending order over all bins). It
+// along x (where the rows are few, several, each with a part of the tiles). Its
+// threads form every segment's origin and keep, in ascending order, those whose
+// stencil meets the row in y and z; then each wavefront fills the lists of tiles
+// of the row (order, slab, pool and counts as above, except that a tile's
+// segments are in ascending order over all bins). It
 // replaces prepare, scan, scatter, order and list launches, whose time is
 // latency at these sizes: 240 segments on 64^3 31 -> 16 us, 1,350 on 96^3 39 ->
 // 20 us, 2,400 on 192^3 37 -> 28 us. The pool's counter is zeroed by
@@ -724,9 +725,9 @@ __global__ void __launch_bounds__(1024)
 // (a < 8), y (8 <= a < 16), z (16 <= a < 32) of the tile starting at
 // (px0, py0, pz0). w[a] = g (monopole), w[32 + a] = gD (dipole), w[64 + a]
 // = its derivative h = gD (-xx / sigma_dip^2), zero off the stencil and past
-// the axis' end (a cut tile); xx is
-// formed in FP64, and so is the exponent (base 2). FP32 rounds it before the
-// hardware exp2, or (fine) rounds the FP64 weight, as the vector path does.
+// the axis' end (a cut tile); xx is formed in FP64, and so is the exponent (base
+// 2). FP32 rounds it before the hardware exp2, or (fine) rounds the FP64 weight,
+// as the vector path does.
 // weights (96) + coefficients (6) per record; odd, so that 16 rows read at one
 // point fall on different banks
 constexpr int kTileW = 105;
@@ -1006,21 +1007,9 @@ __device__ __forceinline__ void st16(T *p, const T *in) {
   *reinterpret_cast<V *>(p) = v;
 }
 
-// Complex values per 16-byte access: 2 (FP32) or 1 (FP64).
-template <typename T>
-constexpr int kCx16 = 16 / (int)sizeof(cx<T>);
-template <typename T>
-__device__ __forceinline__ void ld16c(const cx<T> *p, cx<T> *out) {
-  ld16(reinterpret_cast<const T *>(p), reinterpret_cast<T *>(out));
-}
-template <typename T>
-__device__ __forceinline__ void st16c(cx<T> *p, const cx<T> *in) {
-  st16(reinterpret_cast<T *>(p), reinterpret_cast<const T *>(in));
-}
-
 // z forward: XB = 2P consecutive x rows at one y, as P complex sequences
 // (row 2p in the real part, row 2p+1 in the imaginary part).
-template <typename T, int E, int LOGN, typename PL = FftPlan>
+template <typename T, int LOGN, typename PL = FftPlan>
 __device__ __forceinline__ void d_fft_z_r2c(const int *__restrict__ act, const T *__restrict__ R, cx<T> *__restrict__ C, PL pl,
                 const cx<T> *__restrict__ twg, int nx, int ny, int P,
                 FastDiv dXB, FastDiv dP) {
@@ -1043,7 +1032,7 @@ __device__ __forceinline__ void d_fft_z_r2c(const int *__restrict__ act, const T
   const size_t rs = (size_t)ny * n;
   const LdsIO<T, true> io{a, 1, pn};
   __syncthreads();
-  lds_fft<T, E, true, false, LOGN>(
+  lds_fft<T, true, false, LOGN>(
       io, pl, P, tw,
       [&](int z, int p) {
         const T *r0 = row + 2 * p * rs + z;
@@ -1076,15 +1065,15 @@ __device__ __forceinline__ void d_fft_z_r2c(const int *__restrict__ act, const T
     }
   }
 }
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 __global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_z_r2c(const int *__restrict__ act, const T *__restrict__ R, cx<T> *__restrict__ C, FftPlan pl,
                 const cx<T> *__restrict__ twg, int nx, int ny, int P,
                 FastDiv dXB, FastDiv dP) {
-  d_fft_z_r2c<T, E, LOGN>(act, R, C, pl, twg, nx, ny, P, dXB, dP);
+  d_fft_z_r2c<T, LOGN>(act, R, C, pl, twg, nx, ny, P, dXB, dP);
 }
 // arguments of one suspension for k_fft_z_r2c_multi
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 struct A_fft_z_r2c {
   const int *act;
   const T *R;
@@ -1099,15 +1088,15 @@ struct A_fft_z_r2c {
 };
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 __global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
-    k_fft_z_r2c_multi(const A_fft_z_r2c<T, E, LOGN> *__restrict__ a) {
-  const A_fft_z_r2c<T, E, LOGN> &A = a[blockIdx.z];
-  d_fft_z_r2c<T, E, LOGN, const FftPlan &>(A.act, A.R, A.C, A.pl, A.twg, A.nx, A.ny, A.P, A.dXB, A.dP);
+    k_fft_z_r2c_multi(const A_fft_z_r2c<T, LOGN> *__restrict__ a) {
+  const A_fft_z_r2c<T, LOGN> &A = a[blockIdx.z];
+  d_fft_z_r2c<T, LOGN, const FftPlan &>(A.act, A.R, A.C, A.pl, A.twg, A.nx, A.ny, A.P, A.dXB, A.dP);
 }
 
 // z inverse: the mirror of k_fft_z_r2c.
-template <typename T, int E, int LOGN, typename PL = FftPlan>
+template <typename T, int LOGN, typename PL = FftPlan>
 __device__ __forceinline__ void d_fft_z_c2r(const int *__restrict__ act, const cx<T> *__restrict__ C, T *__restrict__ R, PL pl,
                 const cx<T> *__restrict__ twg, int nx, int ny, int P,
                 FastDiv dP) {
@@ -1149,22 +1138,22 @@ __device__ __forceinline__ void d_fft_z_c2r(const int *__restrict__ act, const c
   T *row = Rc + ((size_t)x0 * ny + y) * n;
   const size_t rs = (size_t)ny * n;
   const LdsIO<T, true> io{a, 1, pn};
-  lds_fft<T, E, true, true, LOGN>(io, pl, P, tw, io,
+  lds_fft<T, true, true, LOGN>(io, pl, P, tw, io,
                                   [&](int z, int p, cx<T> v) {
                                     T *r0 = row + 2 * p * rs + z;
                                     r0[0] = v.x;
                                     r0[rs] = v.y;
                                   });
 }
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 __global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_z_c2r(const int *__restrict__ act, const cx<T> *__restrict__ C, T *__restrict__ R, FftPlan pl,
                 const cx<T> *__restrict__ twg, int nx, int ny, int P,
                 FastDiv dP) {
-  d_fft_z_c2r<T, E, LOGN>(act, C, R, pl, twg, nx, ny, P, dP);
+  d_fft_z_c2r<T, LOGN>(act, C, R, pl, twg, nx, ny, P, dP);
 }
 // arguments of one suspension for k_fft_z_c2r_multi
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 struct A_fft_z_c2r {
   const int *act;
   const cx<T> *C;
@@ -1178,15 +1167,15 @@ struct A_fft_z_c2r {
 };
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 __global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
-    k_fft_z_c2r_multi(const A_fft_z_c2r<T, E, LOGN> *__restrict__ a) {
-  const A_fft_z_c2r<T, E, LOGN> &A = a[blockIdx.z];
-  d_fft_z_c2r<T, E, LOGN, const FftPlan &>(A.act, A.C, A.R, A.pl, A.twg, A.nx, A.ny, A.P, A.dP);
+    k_fft_z_c2r_multi(const A_fft_z_c2r<T, LOGN> *__restrict__ a) {
+  const A_fft_z_c2r<T, LOGN> &A = a[blockIdx.z];
+  d_fft_z_c2r<T, LOGN, const FftPlan &>(A.act, A.C, A.R, A.pl, A.twg, A.nx, A.ny, A.P, A.dP);
 }
 
 // y pass: one workgroup per (comp, kz, run of B consecutive x).
-template <typename T, int E, int LOGN, typename PL = FftPlan>
+template <typename T, int LOGN, typename PL = FftPlan>
 __device__ __forceinline__ void d_fft_y(const int *__restrict__ act, cx<T> *__restrict__ C, PL pl, const cx<T> *__restrict__ twg,
             int nx, int nh, int B, int inverse, FastDiv dB) {
   if (act && !*act) return;  // batched sweep: suspension converged
@@ -1206,18 +1195,18 @@ __device__ __forceinline__ void d_fft_y(const int *__restrict__ act, cx<T> *__re
   const auto st = [&](int m, int col, cx<T> v) { base[(size_t)m * nx + col] = v; };
   __syncthreads();
   if (inverse)
-    lds_fft<T, E, false, true, LOGN>(io, pl, B, tw, ld, st, dB);
+    lds_fft<T, false, true, LOGN>(io, pl, B, tw, ld, st, dB);
   else
-    lds_fft<T, E, false, false, LOGN>(io, pl, B, tw, ld, st, dB);
+    lds_fft<T, false, false, LOGN>(io, pl, B, tw, ld, st, dB);
 }
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 __global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
     k_fft_y(const int *__restrict__ act, cx<T> *__restrict__ C, FftPlan pl, const cx<T> *__restrict__ twg,
             int nx, int nh, int B, int inverse, FastDiv dB) {
-  d_fft_y<T, E, LOGN>(act, C, pl, twg, nx, nh, B, inverse, dB);
+  d_fft_y<T, LOGN>(act, C, pl, twg, nx, nh, B, inverse, dB);
 }
 // arguments of one suspension for k_fft_y_multi
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 struct A_fft_y {
   const int *act;
   cx<T> *C;
@@ -1231,11 +1220,11 @@ struct A_fft_y {
 };
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 __global__ void __launch_bounds__((kFftMaxThreads<T, LOGN>))
-    k_fft_y_multi(const A_fft_y<T, E, LOGN> *__restrict__ a) {
-  const A_fft_y<T, E, LOGN> &A = a[blockIdx.z];
-  d_fft_y<T, E, LOGN, const FftPlan &>(A.act, A.C, A.pl, A.twg, A.nx, A.nh, A.B, A.inverse, A.dB);
+    k_fft_y_multi(const A_fft_y<T, LOGN> *__restrict__ a) {
+  const A_fft_y<T, LOGN> &A = a[blockIdx.z];
+  d_fft_y<T, LOGN, const FftPlan &>(A.act, A.C, A.pl, A.twg, A.nx, A.nh, A.B, A.inverse, A.dB);
 }
 
 struct ProjConst {
@@ -1277,9 +1266,9 @@ __device__ __forceinline__ void project(const PC &pc, int x, int y, int kz,
 // One stage of a compile-time plan on a thread's registers: radix 2^LR, span
 // 2^LS of n = 2^LOGN; butterfly m of thread t is t + m * blockDim.x, lines
 // contiguous in LDS.
-template <typename T, int E, int LOGN, int LR, int LS>
+template <typename T, int LOGN, int LR, int LS>
 struct RegStage {
-  static constexpr int R = 1 << LR, NB = E / R, LNB = LOGN - LR, nb = 1 << LNB,
+  static constexpr int R = 1 << LR, NB = kP2E / R, LNB = LOGN - LR, nb = 1 << LNB,
                        ns = 1 << LS, PN = fft_padded_len(1 << LOGN);
   static __device__ __forceinline__ int line(int m) {
     return (threadIdx.x + m * blockDim.x) >> LNB;
@@ -1331,13 +1320,13 @@ struct RegStage {
 };
 // The stage that starts at span 2^LS, in the plan's order (FWD) or in the
 // reversed one: log2 of its radix.
-template <int LOGN, int E>
+template <int LOGN>
 constexpr int p2_log_radix(int ls, bool fwd) {
   int at = 0;
   int lr[16] = {}, n = 0;
   while (at < LOGN) {
     const int rem = LOGN - at;
-    lr[n] = rem >= 4 && E >= 16 ? 4 : rem >= 3 && E >= 8 ? 3 : rem >= 2 ? 2 : 1;
+    lr[n] = rem >= 3 ? 3 : rem >= 2 ? 2 : 1;
     at += lr[n++];
   }
   at = 0;
@@ -1350,16 +1339,16 @@ constexpr int p2_log_radix(int ls, bool fwd) {
 }
 // Stages from span 2^LS on of three components' lines; the values come in the
 // registers of the stage before it (or of this one for LS = 0).
-template <typename T, int E, int LOGN, bool INV, int LS>
+template <typename T, int LOGN, bool INV, int LS>
 __device__ __forceinline__ void x_stages(cx<T> *buf, const cx<T> *tw,
-                                         cx<T> (*v)[E]) {
+                                         cx<T> (*v)[kP2E]) {
   if constexpr (LS < LOGN) {
-    constexpr int LR = p2_log_radix<LOGN, E>(LS, !INV);
-    using S = RegStage<T, E, LOGN, LR, LS>;
+    constexpr int LR = p2_log_radix<LOGN>(LS, !INV);
+    using S = RegStage<T, LOGN, LR, LS>;
 #pragma unroll
     for (int c = 0; c < 3; ++c) S::template butterflies<INV>(tw, v[c]);
     if constexpr (LS + LR < LOGN) {
-      using N = RegStage<T, E, LOGN, p2_log_radix<LOGN, E>(LS + LR, !INV), LS + LR>;
+      using N = RegStage<T, LOGN, p2_log_radix<LOGN>(LS + LR, !INV), LS + LR>;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         __syncthreads();
@@ -1367,7 +1356,7 @@ __device__ __forceinline__ void x_stages(cx<T> *buf, const cx<T> *tw,
         __syncthreads();
         N::get(buf, v[c]);
       }
-      x_stages<T, E, LOGN, INV, LS + LR>(buf, tw, v);
+      x_stages<T, LOGN, INV, LS + LR>(buf, tw, v);
     }
   }
 }
@@ -1383,7 +1372,7 @@ __device__ __forceinline__ void x_stages(cx<T> *buf, const cx<T> *tw,
 // 225 -> 145 us; 512^3 FP32 1,111 -> 697 us. The run-time plans' radices would
 // need up to 200 registers for that (192^3: 73 -> 128 us): there the three
 // components stay in LDS.
-template <typename T, int E, int LOGN, typename PL = FftPlan, typename PC = ProjConst>
+template <typename T, int LOGN, typename PL = FftPlan, typename PC = ProjConst>
 __device__ __forceinline__ void d_fft_x_project(const int *__restrict__ act, cx<T> *__restrict__ C, PL pl,
                     const cx<T> *__restrict__ twg, PC pc, int Q,
                     FastDiv dQ) {
@@ -1399,12 +1388,12 @@ __device__ __forceinline__ void d_fft_x_project(const int *__restrict__ act, cx<
   cx<T> *base = C + ((size_t)kz * pc.ny + y0) * n;
   for (int i = threadIdx.x; i < n; i += blockDim.x) tw[i] = twg[i];
   if constexpr (LOGN > 0) {
-    using F = RegStage<T, E, LOGN, p2_log_radix<LOGN, E>(0, true), 0>;
-    constexpr int LL = p2_log_radix<LOGN, E>(0, false);  // the last stage's
-    using L = RegStage<T, E, LOGN, LL, LOGN - LL>;
-    using O = RegStage<T, E, LOGN, p2_log_radix<LOGN, E>(0, true),
-                       LOGN - p2_log_radix<LOGN, E>(0, true)>;
-    cx<T> v[3][E];
+    using F = RegStage<T, LOGN, p2_log_radix<LOGN>(0, true), 0>;
+    constexpr int LL = p2_log_radix<LOGN>(0, false);  // the last stage's
+    using L = RegStage<T, LOGN, LL, LOGN - LL>;
+    using O = RegStage<T, LOGN, p2_log_radix<LOGN>(0, true),
+                       LOGN - p2_log_radix<LOGN>(0, true)>;
+    cx<T> v[3][kP2E];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
@@ -1413,14 +1402,14 @@ __device__ __forceinline__ void d_fft_x_project(const int *__restrict__ act, cx<
 #pragma unroll
         for (int r = 0; r < F::R; ++r) v[c][m * F::R + r] = src[r * F::nb];
       }
-    x_stages<T, E, LOGN, false, 0>(a, tw, v);
+    x_stages<T, LOGN, false, 0>(a, tw, v);
 #pragma unroll
     for (int m = 0; m < L::NB; ++m)
 #pragma unroll
       for (int r = 0; r < L::R; ++r)
         project<T>(pc, L::j(m) + r * L::nb, y0 + L::line(m), kz,
                    v[0][m * L::R + r], v[1][m * L::R + r], v[2][m * L::R + r]);
-    x_stages<T, E, LOGN, true, 0>(a, tw, v);
+    x_stages<T, LOGN, true, 0>(a, tw, v);
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
@@ -1451,15 +1440,15 @@ __device__ __forceinline__ void d_fft_x_project(const int *__restrict__ act, cx<
     lds_fft_plan<T, true, true>(io, pl, 3 * Q, tw, FastDiv{0, 0}, io, st);
   }
 }
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 __global__ void __launch_bounds__((kXMaxThreads<T, LOGN>))
     k_fft_x_project(const int *__restrict__ act, cx<T> *__restrict__ C, FftPlan pl,
                     const cx<T> *__restrict__ twg, ProjConst pc, int Q,
                     FastDiv dQ) {
-  d_fft_x_project<T, E, LOGN>(act, C, pl, twg, pc, Q, dQ);
+  d_fft_x_project<T, LOGN>(act, C, pl, twg, pc, Q, dQ);
 }
 // arguments of one suspension for k_fft_x_project_multi
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 struct A_fft_x_project {
   const int *act;
   cx<T> *C;
@@ -1471,11 +1460,11 @@ struct A_fft_x_project {
 };
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
-template <typename T, int E, int LOGN>
+template <typename T, int LOGN>
 __global__ void __launch_bounds__((kXMaxThreads<T, LOGN>))
-    k_fft_x_project_multi(const A_fft_x_project<T, E, LOGN> *__restrict__ a) {
-  const A_fft_x_project<T, E, LOGN> &A = a[blockIdx.z];
-  d_fft_x_project<T, E, LOGN, const FftPlan &, const ProjConst &>(A.act, A.C, A.pl, A.twg, A.pc, A.Q, A.dQ);
+    k_fft_x_project_multi(const A_fft_x_project<T, LOGN> *__restrict__ a) {
+  const A_fft_x_project<T, LOGN> &A = a[blockIdx.z];
+  d_fft_x_project<T, LOGN, const FftPlan &, const ProjConst &>(A.act, A.C, A.pl, A.twg, A.pc, A.Q, A.dQ);
 }
 
 // ---------------------------------------------------------------------
@@ -1655,7 +1644,7 @@ __device__ __forceinline__ void ld4(const T *p, T *out) {
   if constexpr (sizeof(T) == 8) ld16(p + 2, out + 2);
 }
 
-template <typename T, int NGD, typename SG = SpreadGeom, typename GC = GaussConst>
+template <typename T, typename SG = SpreadGeom, typename GC = GaussConst>
 __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G, GC g,
                   const SegRec<T> *__restrict__ slab,
                   const SegRec<T> *__restrict__ pool,
@@ -1826,17 +1815,17 @@ __device__ __forceinline__ void d_interp_mfma(const int *__restrict__ act, SG G,
     }
   }
 }
-template <typename T, int NGD>
+template <typename T>
 __global__ void __launch_bounds__(256, kInterpWaves<T>)
     k_interp_mfma(const int *__restrict__ act, SpreadGeom G, GaussConst g,
                   const SegRec<T> *__restrict__ slab,
                   const SegRec<T> *__restrict__ pool,
                   const int *__restrict__ tcnt, const int *__restrict__ tovf,
                   const T *__restrict__ R, T *__restrict__ part) {
-  d_interp_mfma<T, NGD>(act, G, g, slab, pool, tcnt, tovf, R, part);
+  d_interp_mfma<T>(act, G, g, slab, pool, tcnt, tovf, R, part);
 }
 // arguments of one suspension for k_interp_mfma_multi
-template <typename T, int NGD>
+template <typename T>
 struct A_interp_mfma {
   const int *act;
   SpreadGeom G;
@@ -1850,11 +1839,11 @@ struct A_interp_mfma {
 };
 // one launch for a group of suspensions with equal launch shapes:
 // blockIdx.z selects the suspension
-template <typename T, int NGD>
+template <typename T>
 __global__ void __launch_bounds__(256, kInterpWaves<T>)
-    k_interp_mfma_multi(const A_interp_mfma<T, NGD> *__restrict__ a) {
-  const A_interp_mfma<T, NGD> &A = a[blockIdx.z];
-  d_interp_mfma<T, NGD, const SpreadGeom &, const GaussConst &>(A.act, A.G, A.g, A.slab, A.pool, A.tcnt, A.tovf, A.R, A.part);
+    k_interp_mfma_multi(const A_interp_mfma<T> *__restrict__ a) {
+  const A_interp_mfma<T> &A = a[blockIdx.z];
+  d_interp_mfma<T, const SpreadGeom &, const GaussConst &>(A.act, A.G, A.g, A.slab, A.pool, A.tcnt, A.tovf, A.R, A.part);
 }
 
 // One thread per (segment, component): adds the segment's tile partials in
@@ -1958,22 +1947,19 @@ __global__ void k_interp_sum_multi(const A_interp_sum<T, NGD> *__restrict__ a) {
 // ---------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------
-// Register tile E and compile-time length of an FFT plan's kernels: n =
-// 2^LOGN with E = 8 for the compile-time plans, E = LOGN = 0 for the run-time
-// plan.
+// Compile-time length of an FFT plan's kernels: n = 2^LOGN for the compile-time
+// plans, LOGN = 0 for the run-time plan.
 template <typename F>
-static bool with_EL(const FftPlan &pl, F f) {
-  using E8 = std::integral_constant<int, 8>;
-  using L0 = std::integral_constant<int, 0>;
+static bool with_LOGN(const FftPlan &pl, F f) {
   if (pl.E == 0) {
-    f(L0{}, L0{});
+    f(std::integral_constant<int, 0>{});
     return true;
   }
   switch (p2_log(pl.n)) {
-    case 6: f(E8{}, std::integral_constant<int, 6>{}); return true;
-    case 7: f(E8{}, std::integral_constant<int, 7>{}); return true;
-    case 8: f(E8{}, std::integral_constant<int, 8>{}); return true;
-    case 9: f(E8{}, std::integral_constant<int, 9>{}); return true;
+    case 6: f(std::integral_constant<int, 6>{}); return true;
+    case 7: f(std::integral_constant<int, 7>{}); return true;
+    case 8: f(std::integral_constant<int, 8>{}); return true;
+    case 9: f(std::integral_constant<int, 9>{}); return true;
   }
   return false;
 }
@@ -2008,37 +1994,38 @@ static bool with_NGD(int ngd, F f) {
 
 template <typename T>
 int set_fft_lds_attr(const FftPlan &plx, const FftPlan &ply,
-                            const FftPlan &plz) {
+                     const FftPlan &plz) {
   const int lds_max = 160 * 1024;
   bool ok = true;
-  ok &= with_EL(plz, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
-    (void)hipFuncSetAttribute((const void *)k_fft_z_r2c<T, EE, LL>,
+  ok &= with_LOGN(plz, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
+    (void)hipFuncSetAttribute((const void *)k_fft_z_r2c<T, LL>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void *)k_fft_z_c2r<T, EE, LL>,
+    (void)hipFuncSetAttribute((const void *)k_fft_z_c2r<T, LL>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void *)k_fft_z_r2c_multi<T, EE, LL>,
+    (void)hipFuncSetAttribute((const void *)k_fft_z_r2c_multi<T, LL>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void *)k_fft_z_c2r_multi<T, EE, LL>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-  });
-  ok &= with_EL(ply, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
-    (void)hipFuncSetAttribute((const void *)k_fft_y<T, EE, LL>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void *)k_fft_y_multi<T, EE, LL>,
+    (void)hipFuncSetAttribute((const void *)k_fft_z_c2r_multi<T, LL>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
   });
-  ok &= with_EL(plx, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
-    (void)hipFuncSetAttribute((const void *)k_fft_x_project<T, EE, LL>,
+  ok &= with_LOGN(ply, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
+    (void)hipFuncSetAttribute((const void *)k_fft_y<T, LL>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void *)k_fft_x_project_multi<T, EE, LL>,
+    (void)hipFuncSetAttribute((const void *)k_fft_y_multi<T, LL>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+  });
+  ok &= with_LOGN(plx, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
+    (void)hipFuncSetAttribute((const void *)k_fft_x_project<T, LL>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+    (void)hipFuncSetAttribute((const void *)k_fft_x_project_multi<T, LL>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
   });
   FS_CHECK(ok, FS_ERR_ARG, "no FFT register tile for these sizes");
   return FS_OK;
 }
+
 // Blocks of a persistent tile kernel (256 threads): as many as are resident
 // on the device at once, a multiple of 8, at most one per tile.
 template <typename K>
@@ -2056,15 +2043,10 @@ static int persistent_blocks(K kernel, int ntiles) {
   return (int)std::min<long>(b, ntiles);
 }
 
-
 // Resident blocks of the persistent interpolation.
 template <typename T>
 int interp_blocks(const FcmImpl &f) {
-  int b = 1;
-  with_NGD(f.p.ngd, [&](auto ng) {
-    b = persistent_blocks(k_interp_mfma<T, decltype(ng)::value>, f.nbins);
-  });
-  return b;
+  return persistent_blocks(k_interp_mfma<T>, f.nbins);
 }
 
 // Workgroups per row of tiles of the lists without bins: up to 16 tiles (one a
@@ -2202,18 +2184,18 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   kmark(3);
   const int nh = p.nz / 2 + 1;
   const size_t csz = sizeof(cx<T>);
-  bool ok = with_EL(plz, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
-    hipLaunchKernelGGL((k_fft_z_r2c<T, EE, LL>), dim3(p.ny * (p.nx / (2 * zP)), 3),
+  bool ok = with_LOGN(plz, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
+    hipLaunchKernelGGL((k_fft_z_r2c<T, LL>), dim3(p.ny * (p.nx / (2 * zP)), 3),
                        dim3(fft_threads(plz, zP)),
                        csz * (p.nz + (size_t)zP * fft_padded_len(p.nz)), st, act,
                        R.as<T>(), C.as<cx<T>>(), plz, twz.as<cx<T>>(), p.nx,
                        p.ny, zP, make_div(2 * zP), make_div(zP));
   });
   kmark(4);
-  ok &= with_EL(ply, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
-    hipLaunchKernelGGL((k_fft_y<T, EE, LL>), dim3(nh * (p.nx / yB), 3),
+  ok &= with_LOGN(ply, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
+    hipLaunchKernelGGL((k_fft_y<T, LL>), dim3(nh * (p.nx / yB), 3),
                        dim3(fft_threads(ply, yB)), csz * (p.ny + (size_t)yB * fft_rowpad_len(p.ny)), st, act,
                        C.as<cx<T>>(), ply, twy.as<cx<T>>(), p.nx, nh, yB, 0,
                        make_div(yB));
@@ -2223,9 +2205,9 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   mark(3);
   kmark(5);
   const ProjConst pc = proj_const(p);
-  ok = with_EL(plx, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
-    hipLaunchKernelGGL((k_fft_x_project<T, EE, LL>), dim3(nh * (p.ny / xQ)),
+  ok = with_LOGN(plx, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
+    hipLaunchKernelGGL((k_fft_x_project<T, LL>), dim3(nh * (p.ny / xQ)),
                        dim3(x_threads(plx, xQ)),
                        csz * x_lds_values(plx, xQ), st, act,
                        C.as<cx<T>>(),
@@ -2235,17 +2217,17 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   FS_LAUNCHED();
   mark(4);
   kmark(6);
-  ok = with_EL(ply, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
-    hipLaunchKernelGGL((k_fft_y<T, EE, LL>), dim3(nh * (p.nx / yB), 3),
+  ok = with_LOGN(ply, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
+    hipLaunchKernelGGL((k_fft_y<T, LL>), dim3(nh * (p.nx / yB), 3),
                        dim3(fft_threads(ply, yB)), csz * (p.ny + (size_t)yB * fft_rowpad_len(p.ny)), st, act,
                        C.as<cx<T>>(), ply, twy.as<cx<T>>(), p.nx, nh, yB, 1,
                        make_div(yB));
   });
   kmark(7);
-  ok &= with_EL(plz, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
-    hipLaunchKernelGGL((k_fft_z_c2r<T, EE, LL>), dim3(p.ny * (p.nx / (2 * zP)), 3),
+  ok &= with_LOGN(plz, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
+    hipLaunchKernelGGL((k_fft_z_c2r<T, LL>), dim3(p.ny * (p.nx / (2 * zP)), 3),
                        dim3(fft_threads(plz, zP)),
                        csz * (p.nz + (size_t)zP * fft_padded_len(p.nz)), st, act,
                        C.as<cx<T>>(), R.as<T>(), plz, twz.as<cx<T>>(), p.nx,
@@ -2259,7 +2241,7 @@ int FcmImpl::run(int np, const double *Y, const double *F, const double *Tq,
   bool okn = with_NGD(p.ngd, [&](auto ng) {
     constexpr int NG = decltype(ng)::value;
     if (mfma_spread) {
-      hipLaunchKernelGGL((k_interp_mfma<T, NG>), dim3(grid_interp), dim3(256), 0,
+      hipLaunchKernelGGL(k_interp_mfma<T>, dim3(grid_interp), dim3(256), 0,
                          st, act, geom, g, tslab.as<SegRec<T>>(),
                          tpool.as<SegRec<T>>(), tcnt.as<int>(), tovf.as<int>(),
                          R.as<T>(), ipart.as<T>());
@@ -2448,78 +2430,78 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
       hipLaunchKernelGGL(k_spread_mfma_multi<T>, dim3(ntiles, 1, S), dim3(256), 0,
                          st, (const A_spread_mfma<T> *)t);
   }
-  bool ok = with_EL(f0.plz, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
+  bool ok = with_LOGN(f0.plz, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
     auto t = table([&](const FcmGroupMember &m) {
       const FcmImpl &f = *m.fcm;
-      return A_fft_z_r2c<T, EE, LL>{m.act, f.R.as<T>(), f.C.as<cx<T>>(), f.plz,
+      return A_fft_z_r2c<T, LL>{m.act, f.R.as<T>(), f.C.as<cx<T>>(), f.plz,
                                     f.twz.as<cx<T>>(), p.nx, p.ny, f.zP,
                                     make_div(2 * f.zP), make_div(f.zP)};
     });
     if (!host)
-      hipLaunchKernelGGL((k_fft_z_r2c_multi<T, EE, LL>),
+      hipLaunchKernelGGL((k_fft_z_r2c_multi<T, LL>),
                          dim3(p.ny * (p.nx / (2 * f0.zP)), 3, S),
                          dim3(fft_threads(f0.plz, f0.zP)),
                          csz * (p.nz + (size_t)f0.zP * fft_padded_len(p.nz)), st,
-                         (const A_fft_z_r2c<T, EE, LL> *)t);
+                         (const A_fft_z_r2c<T, LL> *)t);
   });
   for (int inv = 0; inv < 2 && ok; ++inv) {
-    ok &= with_EL(f0.ply, [&](auto e, auto l) {
-      constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
+    ok &= with_LOGN(f0.ply, [&](auto l) {
+      constexpr int LL = decltype(l)::value;
       auto t = table([&](const FcmGroupMember &m) {
         const FcmImpl &f = *m.fcm;
-        return A_fft_y<T, EE, LL>{m.act, f.C.as<cx<T>>(), f.ply, f.twy.as<cx<T>>(),
+        return A_fft_y<T, LL>{m.act, f.C.as<cx<T>>(), f.ply, f.twy.as<cx<T>>(),
                                   p.nx, nh, f.yB, inv, make_div(f.yB)};
       });
       if (!host)
-        hipLaunchKernelGGL((k_fft_y_multi<T, EE, LL>),
+        hipLaunchKernelGGL((k_fft_y_multi<T, LL>),
                            dim3(nh * (p.nx / f0.yB), 3, S), dim3(fft_threads(f0.ply, f0.yB)),
                            csz * (p.ny + (size_t)f0.yB * fft_rowpad_len(p.ny)), st,
-                           (const A_fft_y<T, EE, LL> *)t);
+                           (const A_fft_y<T, LL> *)t);
     });
     if (inv == 0)
-      ok &= with_EL(f0.plx, [&](auto e, auto l) {
-        constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
+      ok &= with_LOGN(f0.plx, [&](auto l) {
+        constexpr int LL = decltype(l)::value;
         auto t = table([&](const FcmGroupMember &m) {
           const FcmImpl &f = *m.fcm;
-          return A_fft_x_project<T, EE, LL>{m.act, f.C.as<cx<T>>(), f.plx,
+          return A_fft_x_project<T, LL>{m.act, f.C.as<cx<T>>(), f.plx,
                                             f.twx.as<cx<T>>(), pc, f.xQ,
                                             make_div(f.xQ)};
         });
         if (!host)
-          hipLaunchKernelGGL((k_fft_x_project_multi<T, EE, LL>),
+          hipLaunchKernelGGL((k_fft_x_project_multi<T, LL>),
                              dim3(nh * (p.ny / f0.xQ), 1, S),
                              dim3(x_threads(f0.plx, f0.xQ)),
                              csz * x_lds_values(f0.plx, f0.xQ),
-                             st, (const A_fft_x_project<T, EE, LL> *)t);
+                             st, (const A_fft_x_project<T, LL> *)t);
       });
   }
-  ok &= with_EL(f0.plz, [&](auto e, auto l) {
-    constexpr int EE = decltype(e)::value, LL = decltype(l)::value;
+  ok &= with_LOGN(f0.plz, [&](auto l) {
+    constexpr int LL = decltype(l)::value;
     auto t = table([&](const FcmGroupMember &m) {
       const FcmImpl &f = *m.fcm;
-      return A_fft_z_c2r<T, EE, LL>{m.act, f.C.as<cx<T>>(), f.R.as<T>(), f.plz,
+      return A_fft_z_c2r<T, LL>{m.act, f.C.as<cx<T>>(), f.R.as<T>(), f.plz,
                                     f.twz.as<cx<T>>(), p.nx, p.ny, f.zP,
                                     make_div(f.zP)};
     });
     if (!host)
-      hipLaunchKernelGGL((k_fft_z_c2r_multi<T, EE, LL>),
+      hipLaunchKernelGGL((k_fft_z_c2r_multi<T, LL>),
                          dim3(p.ny * (p.nx / (2 * f0.zP)), 3, S),
                          dim3(fft_threads(f0.plz, f0.zP)),
                          csz * (p.nz + (size_t)f0.zP * fft_padded_len(p.nz)), st,
-                         (const A_fft_z_c2r<T, EE, LL> *)t);
+                         (const A_fft_z_c2r<T, LL> *)t);
   });
   ok &= with_NGD(p.ngd, [&](auto ng) {
     constexpr int NG = decltype(ng)::value;
     auto t = table([&](const FcmGroupMember &m) {
       const FcmImpl &f = *m.fcm;
-      return A_interp_mfma<T, NG>{m.act, f.geom, g, f.tslab.as<SegRec<T>>(),
-                                  f.tpool.as<SegRec<T>>(), f.tcnt.as<int>(),
-                                  f.tovf.as<int>(), f.R.as<T>(), f.ipart.as<T>()};
+      return A_interp_mfma<T>{m.act, f.geom, g, f.tslab.as<SegRec<T>>(),
+                              f.tpool.as<SegRec<T>>(), f.tcnt.as<int>(),
+                              f.tovf.as<int>(), f.R.as<T>(), f.ipart.as<T>()};
     });
     if (!host)
-      hipLaunchKernelGGL((k_interp_mfma_multi<T, NG>), dim3(f0.grid_interp, 1, S),
-                         dim3(256), 0, st, (const A_interp_mfma<T, NG> *)t);
+      hipLaunchKernelGGL(k_interp_mfma_multi<T>, dim3(f0.grid_interp, 1, S),
+                         dim3(256), 0, st, (const A_interp_mfma<T> *)t);
     auto t2 = table([&](const FcmGroupMember &m) {
       const FcmImpl &f = *m.fcm;
       return A_interp_sum<T, NG>{m.act, m.np, f.geom, dx3, f.origin.as<int>(),
@@ -2535,7 +2517,5 @@ int group_stages(FcmGroup &G, std::vector<char> *host, hipStream_t st) {
   if (!host) FS_LAUNCHED();
   return FS_OK;
 }
-
-
 
 }  // namespace fs

@@ -35,12 +35,13 @@ inline FastDiv make_div(int d) {
   return FastDiv{(1ull << 32) / (unsigned long long)d + 1ull, d};
 }
 
+// Elements per thread of the compile-time plans.
+constexpr int kP2E = 8;
+
 struct FftPlan {
   int n;
   int nst;
-  // elements per thread of the compile-time plans (lengths 2^LOGN below);
-  // 0: run-time plan
-  int E;
+  int E;  // kP2E: compile-time plan (lengths 2^LOGN below), 0: run-time plan
   int rad[kMaxStages];
   FastDiv dn;               // by n
   FastDiv dnb[kMaxStages];  // by n / rad[s]
@@ -93,10 +94,11 @@ inline bool gen_radices(int n, int maxr, int left, int *rad, int *nst,
   return false;
 }
 
-// Plan of n = 2^a 3^b 5^c. Lengths 64 to 512 that are powers of two
-// take the compile-time plan: radix 8, then what is left. (Radix 16, two stages instead of three at
-// 256 points, is within 3% of it in FP32 and 20% slower in FP64: a thread's 16
-// values leave half the wavefronts.)
+// Plan of n = 2^a 3^b 5^c. Lengths 64 to 512 that are powers of two take the
+// compile-time plan: radix 8, then what is left. (Radix 16 there, two stages
+// instead of three at 256 points, is within 3% of it in FP32 and 20% slower in
+// FP64: a thread's 16 values leave half the wavefronts. A run-time plan's stage
+// count decides, so 160 takes 16 x 10 and 192 takes 16 x 12.)
 inline bool make_plan(int n, FftPlan *p) {
   int a = 0, m = n;
   while (m % 2 == 0) m /= 2, ++a;
@@ -107,7 +109,7 @@ inline bool make_plan(int n, FftPlan *p) {
   p->nst = 0;
   p->E = 0;
   if (p2_log(n)) {
-    p->E = 8;
+    p->E = kP2E;
     while (a > 0) {
       const int l = a >= 3 ? 3 : a >= 2 ? 2 : 1;
       p->rad[p->nst++] = 1 << l;
@@ -510,29 +512,25 @@ __device__ void lds_fft_plan(LdsIO<T, PAD> io, const FftPlan &pl, int ncols,
 }
 
 // --- n = 2^LOGN with the plan fixed at compile time ------------------------
-// Same stages as make_plan (largest radix first, at most E points per
-// butterfly), so the same arithmetic; spans, butterfly counts, twiddle steps
+// Same stages as make_plan (radix 8, then what is left), so the same arithmetic; spans, butterfly counts, twiddle steps
 // and padded offsets are constants: divisions become shifts and masks, and
 // the R addresses of a butterfly are one base plus immediate offsets.
 
 constexpr int ilog2_c(int v) { return v <= 1 ? 0 : 1 + ilog2_c(v / 2); }
 
-template <int LOGN, int LOGNS, int E>
+template <int LOGN, int LOGNS>
 constexpr int p2_radix() {
-  return (LOGN - LOGNS >= 4 && E >= 16)  ? 16
-         : (LOGN - LOGNS >= 3 && E >= 8) ? 8
-         : (LOGN - LOGNS >= 2)           ? 4
-                                         : 2;
+  return LOGN - LOGNS >= 3 ? 8 : LOGN - LOGNS >= 2 ? 4 : 2;
 }
 
-template <typename T, int E, bool PAD, bool INV, int LOGN, int LOGNS,
+template <typename T, bool PAD, bool INV, int LOGN, int LOGNS,
           typename LD, typename ST>
 __device__ __forceinline__ void p2_stage(LdsIO<T, PAD> io, int ncols,
                                          const cx<T> *tw, FastDiv dcols, LD ld,
                                          ST st) {
-  constexpr int R = p2_radix<LOGN, LOGNS, E>();
+  constexpr int R = p2_radix<LOGN, LOGNS>();
   constexpr int LOGR = ilog2_c(R);
-  constexpr int NB = E / R;
+  constexpr int NB = kP2E / R;
   constexpr int LOGNB = LOGN - LOGR;
   constexpr int nb = 1 << LOGNB;
   constexpr int ns = 1 << LOGNS;
@@ -542,10 +540,9 @@ __device__ __forceinline__ void p2_stage(LdsIO<T, PAD> io, int ncols,
       LOGNS > 0 || std::is_same<LD, LdsIO<T, PAD>>::value;
   constexpr bool to_lds =
       LOGNS + LOGR < LOGN || std::is_same<ST, LdsIO<T, PAD>>::value;
-  static_assert(E % R == 0, "register tile must hold whole butterflies");
   cx<T> *buf = io.buf;
   const int sm = io.sm;
-  cx<T> v[E];
+  cx<T> v[kP2E];
   int jj[NB], cc[NB];
 #pragma unroll
   for (int m = 0; m < NB; ++m) {
@@ -622,7 +619,7 @@ __device__ __forceinline__ void p2_stage(LdsIO<T, PAD> io, int ncols,
   }
   if constexpr (LOGNS + LOGR < LOGN) {
     __syncthreads();
-    p2_stage<T, E, PAD, INV, LOGN, LOGNS + LOGR>(io, ncols, tw, dcols, ld, st);
+    p2_stage<T, PAD, INV, LOGN, LOGNS + LOGR>(io, ncols, tw, dcols, ld, st);
   }
 }
 
@@ -630,13 +627,13 @@ __device__ __forceinline__ void p2_stage(LdsIO<T, PAD> io, int ncols,
 // compile-time plan (n = 2^LOGN, PAD: sc = fft_padded_len(n)), LOGN = 0 the
 // run-time plan pl. The first stage reads from ld, the last writes to st:
 // global memory, or io for LDS. No barrier after the last writes.
-template <typename T, int E, bool PAD, bool INV, int LOGN, typename LD,
+template <typename T, bool PAD, bool INV, int LOGN, typename LD,
           typename ST>
 __device__ __forceinline__ void lds_fft(LdsIO<T, PAD> io, const FftPlan &pl,
                                         int ncols, const cx<T> *tw, LD ld, ST st,
                                         FastDiv dcols = FastDiv{0, 0}) {
   if constexpr (LOGN > 0)
-    p2_stage<T, E, PAD, INV, LOGN, 0>(io, ncols, tw, dcols, ld, st);
+    p2_stage<T, PAD, INV, LOGN, 0>(io, ncols, tw, dcols, ld, st);
   else
     lds_fft_plan<T, PAD, INV>(io, pl, ncols, tw, dcols, ld, st);
 }
