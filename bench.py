@@ -33,7 +33,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per dispatch of the FP32 y pass (k_fft_y<float, 8, 8>, the
+# HBM bytes per dispatch of the FP32 y pass (k_fft_y<float, 8>, the
 # timestep's largest kernel by total time) at 256^3, measured with rocprofv3
 # --pmc FETCH_SIZE and WRITE_SIZE in separate runs, each scaled by the same
 # counter's reading for a 1 GiB copy
@@ -723,7 +723,7 @@ def main():
                                "KB=1000, dt=0.005, TOL=1e-6, barrier on",
                    "global_batch": 30000, "seq_len": 256,
                    "parallelism": "single GPU"},
-        "roofline": {"bound": "hbm", "kernel": "k_fft_y<float, 8, 8>",
+        "roofline": {"bound": "hbm", "kernel": "k_fft_y<float, 8>",
                      "achieved": xk_bytes / (xk_ms * 1e-3) / 1e9,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": xk_bytes / (xk_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,

@@ -442,7 +442,10 @@ int FcmImpl::set_tuning(const fs_fcm_tuning &t) {
   FS_CHECK(nt.fft_batch >= 1 && nt.fft_batch <= 64 && nt.fft_xlines >= 1 &&
                nt.fft_xlines <= 16,
            FS_ERR_ARG, "fft_batch must be in [1,64], fft_xlines in [1,16]");
-  // LDS: y pass holds ny + B*(row-padded ny) complex, x pass nx + 3Q*(padded nx)
+  // LDS: y pass holds ny + B*(row-padded ny) complex, x pass nx + 3Q*(padded nx).
+  // Compile-time plans keep one component there and set_geometry reduces Q to
+  // their 256 threads, but take the same values: a larger Q would be no other
+  // shape.
   size_t cs = (size_t)tsz * 2;
   size_t lds = std::max(cs * (p.ny + (size_t)nt.fft_batch * fft_rowpad_len(p.ny)),
                         cs * (p.nx + 3 * (size_t)nt.fft_xlines *

@@ -56,7 +56,9 @@ typedef struct fs_fcm_params {
 typedef struct fs_fcm fs_fcm;
 
 /* Fcm::initialise (FCMfunctions.cpp:10-168): grids, wavenumbers, tables.
- * Sizes must factor as 2^a 3^b 5^c with nx,ny,nz <= 1024 (even). */
+ * Sizes must factor as 2^a 3^b 5^c with nx,ny,nz <= 1024 (even). A solve
+ * takes up to max_np segments; its results depend on its own segments, not
+ * on max_np. */
 int fs_fcm_create(const fs_fcm_params *p, int max_np, int precision,
                   fs_fcm **out);
 /* Fcm::free_memory (FCMfunctions.cpp:468-519). */
@@ -92,9 +94,10 @@ typedef struct fs_fcm_tuning {
   int spread_zrun;  /* largest spread tile extent in z (4..16)         */
   int fft_xlines;   /* x lines (per component) per workgroup, x pass  */
   int spread_mfma;  /* 1 spreads and interpolates with matrix-core
-                       products on 8 x 8 x 16 tiles (grids with nx, ny
-                       multiples of 8, nz of 16, nz >= 16 + ngd), 0 with
-                       the vector gather and one wavefront per segment. In
+                       products on 8 x 8 x 16 tiles, the last ones of an
+                       axis cut off where it is no multiple (nz >= 16 +
+                       ngd, else as 0), 0 with the vector gather and one
+                       wavefront per segment. In
                        fs_fcm_set_tuning a negative value keeps the current
                        setting, as do values <= 0 of the other fields. */
 } fs_fcm_tuning;
