@@ -276,9 +276,12 @@ int FcmImpl::set_geometry() {
 // segments on 64^3 (32 row steps) 31 and 16; 3,600 on 128^3 (512) 43 and 26;
 // 2,400 on 192^3 (864) 37 and 28, growing with the row steps. The way depends on
 // the solve's own segments, so that its results do not change with the
-// capacity of the handle. FP64 weights (fine_weights) cost nothing where
-// launches and latency bound the tile kernels; on cut grids the vector gather,
-// which takes them too, was the other way.
+// capacity of the handle. FP32 solves round FP64 weights there and on cut grids
+// (fine_weights): cut grids came from the vector gather, which does, and small
+// solves with hardware exp2 were up to 1.4 times further off the 64-bit result.
+// It costs 0 to 3% of a solve (96^3 with 1,350 segments 89.5 and 90.8 us), 4 to
+// 6% on densely filled cut grids (50^3 with 4,000 157 and 164, 100 x 80 x 90
+// with 10,000 184 and 195); at 250^3 with 27,000 853 and 862.
 bool FcmImpl::lists_direct(int np) const {
   return mfma_spread && np <= kDirectMax &&
          (long)ceil_div(np, 1024) * geom.nby * geom.nbz <= kDirectRowSteps;
